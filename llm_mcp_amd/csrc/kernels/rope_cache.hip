@@ -128,50 +128,122 @@ __global__ void __launch_bounds__(256) rope_cache_kernel(
   }
 }
 
-// Prefill rows: 32 consecutive tokens per workgroup.  Rotation and the K
-// write as above; V goes through an LDS tile so that the key-quad cache page
+// Prefill rows: a workgroup of grid.x takes 32 consecutive tokens, one of grid.y
+// a group of their heads: rotation of q / k heads (with the K write) or a group
+// of V heads.  V goes through an LDS tile so that the key-quad cache page
 // ([BS/4][D][4]) is written in 16-B pieces -- a thread stores 4 consecutive
 // tokens of 2 d whenever their slots are consecutive and 4-aligned (always
 // true inside a prefill chunk), and a wave covers 8 whole 128-B lines.
 // The per-token kernel's 2-B stores remain for decode rows (one token per
 // page per step, nothing to coalesce).
+//
+// The work is copying: memory bound when it fills the chip, otherwise bound by
+// one chain of dependent latencies (slot, row, store) per workgroup.  A workgroup
+// that walked all heads of its tokens ran 6 (Llama-3) to 9 (nomic) such chains one after
+// the other on T / 32 workgroups; a head group is ONE chain.
+// Measured, all heads in a workgroup -> groups of heads: 16 nomic tokens 17.0 -> 4.5 us, 160 Llama-3
+// tokens (k and v only) 19.0 -> 5.0, 6,464 of them 30 -> 17, 11,760 nomic tokens 37.7 -> 24.4 (108 MB).
 constexpr int RT = 32;
-constexpr int RT_VCOLS = 1024;   // V staging columns per LDS pass
+constexpr int RT_VCOLS = 256;    // V columns of a workgroup (at least a head)
 
-// bytes of the tiled kernel's dynamic LDS (the V staging tile)
-static size_t rope_tile_smem(int Hkv, int D) {
-  const int hg = RT_VCOLS / D < Hkv ? RT_VCOLS / D : Hkv;
-  return (size_t)RT * (hg * D + 8) * sizeof(bf16_t);
+// q / k heads that one workgroup rotates: up to 4 per thread, whose threads
+// cover (token, 8-pair chunk) pairs of one head, or of several where D is small
+__host__ __device__ constexpr int rope_head_step(int D) {
+  return RT * (D / 16) >= 256 ? 1 : 256 / (RT * (D / 16));
+}
+__host__ __device__ constexpr int rope_v_heads(int D) { return D >= RT_VCOLS ? 1 : RT_VCOLS / D; }
+
+// V heads h0 .. h0 + hg of tokens t0 .. t0 + nt (v: the first token's V row) to
+// their pages; vt: RT rows of LD elements
+__device__ __forceinline__ void v_to_pages(const bf16_t* __restrict__ v, long stride, int nt, int h0,
+                                           int hg, int Hkv, int D, const int* sslot, bf16_t* vt,
+                                           int LD, bf16_t* __restrict__ v_cache, int BS) {
+  const int chunks = hg * D / 8;
+#pragma unroll 4
+  for (int it = threadIdx.x; it < nt * chunks; it += 256) {
+    const int tt = it / chunks, c = it - tt * chunks;
+    *reinterpret_cast<u16x8*>(&vt[tt * LD + 8 * c]) =
+        *reinterpret_cast<const u16x8*>(v + (long)tt * stride + (long)h0 * D + 8 * c);
+  }
+  __syncthreads();
+  // one 16-B store per (head, key quad, d pair): 4 tokens x 2 d of the
+  // key-quad page, whenever the quad's 4 slots are consecutive and
+  // 4-aligned (always, inside a prefill chunk's whole pages)
+  const int per_h = (D / 2) * (RT / 4);
+  for (int it = threadIdx.x; it < hg * per_h; it += 256) {
+    const int hl = it / per_h, r = it - hl * per_h;
+    const int d = 2 * (r % (D / 2)), tt0 = (r / (D / 2)) * 4, h = h0 + hl;
+    if (tt0 >= nt) continue;
+    const int col = hl * D + d;
+    const int s0 = sslot[tt0];
+    bool vec = tt0 + 4 <= nt && s0 >= 0 && (s0 % 4) == 0;
+#pragma unroll
+    for (int j = 1; j < 4; ++j) vec = vec && sslot[tt0 + j] == s0 + j;
+    if (vec) {
+      u16x8 w;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        w.v[j] = vt[(tt0 + j) * LD + col];
+        w.v[4 + j] = vt[(tt0 + j) * LD + col + 1];
+      }
+      *reinterpret_cast<u16x8*>(v_cache + ((long)(s0 / BS) * Hkv + h) * BS * D +
+                                vq_off(d, s0 % BS, D)) = w;
+    } else {
+      for (int j = 0; j < 4 && tt0 + j < nt; ++j) {
+        const int sl = sslot[tt0 + j];
+        if (sl < 0) continue;
+        bf16_t* vp = v_cache + ((long)(sl / BS) * Hkv + h) * BS * D + vq_off(d, sl % BS, D);
+        vp[0] = vt[(tt0 + j) * LD + col];
+        vp[4] = vt[(tt0 + j) * LD + col + 1];
+      }
+    }
+  }
 }
 
+// grid (32-token tiles, rotation groups + V groups)
 __global__ void __launch_bounds__(256) rope_cache_tiled_kernel(
     bf16_t* __restrict__ qkv, long qkv_stride, const int* __restrict__ positions,
     const float* __restrict__ cos_sin, int row0, int T, int Hq, int Hkv, int D,
     const int* __restrict__ slot_mapping, bf16_t* __restrict__ k_cache,
     bf16_t* __restrict__ v_cache, int BS, int rotate_k_inplace,
-    const bf16_t* __restrict__ q_norm, const bf16_t* __restrict__ k_norm, float eps, int skip_q) {
-  // V staging tile (dynamic LDS, sized by the launcher): HG = min(RT_VCOLS / D,
-  // Hkv) whole heads of 32 tokens, rows of HG * D + 8 elements -- a TP rank's
-  // single kv head takes 8.7 KB instead of a fixed 66 KB (more workgroups per
-  // CU; and the 64 KB static limit of older parts is not crossed)
-  extern __shared__ __attribute__((aligned(16))) bf16_t vt[];
+    const bf16_t* __restrict__ q_norm, const bf16_t* __restrict__ k_norm, float eps, int skip_q,
+    int rot_groups) {
+  extern __shared__ __attribute__((aligned(16))) bf16_t vt[];   // [RT][rope_v_heads * D + 8]
   __shared__ int sslot[RT];
   const int t0 = row0 + blockIdx.x * RT;
   const int nt = min(RT, T - t0);
-  const int half = D >> 1, tph = half >> 3;   // 8-pair chunks per head
   if (threadIdx.x < RT)
     sslot[threadIdx.x] = (threadIdx.x < nt && slot_mapping) ? slot_mapping[t0 + threadIdx.x] : -1;
   __syncthreads();
-  // a thread owns one (token, 4-pair chunk) and walks every q / k head of the
-  // token: the cos/sin chunk is loaded once per item instead of once per
-  // head, and HU heads' loads are issued before their arithmetic
   const int H = Hq + Hkv;
+  if ((int)blockIdx.y >= rot_groups) {
+    const int hv = rope_v_heads(D), h0 = ((int)blockIdx.y - rot_groups) * hv;
+    v_to_pages(qkv + (long)t0 * qkv_stride + (long)H * D, qkv_stride, nt, h0, min(hv, Hkv - h0), Hkv,
+               D, sslot, vt, hv * D + 8, v_cache, BS);
+    return;
+  }
+  // a thread owns one (token, 8-pair chunk) of up to HU heads, whose loads are
+  // issued before their arithmetic; the cos/sin chunk is loaded once for them
+  // (heads of more than 128 channels take two turns)
   constexpr int HU = 4;
-  for (int it = threadIdx.x; it < nt * tph; it += blockDim.x) {
+  const int half = D >> 1, tph = half >> 3;   // 8-pair chunks per head
+  const int hs = rope_head_step(D), lanes = RT * tph;
+  const int h0 = (skip_q ? Hq : 0) + blockIdx.y * HU * hs + (lanes < 256 ? threadIdx.x / lanes : 0);
+  if (lanes < 256 && (int)threadIdx.x >= lanes * hs) return;
+  for (int it = lanes < 256 ? threadIdx.x % lanes : threadIdx.x; it < nt * tph; it += 256) {
     const int tt = it / tph, i = (it % tph) * 8;
     bf16_t* row = qkv + (long)(t0 + tt) * qkv_stride;
     const float* cs = cos_sin + (long)positions[t0 + tt] * D;
     const int slot = sslot[tt];
+    u16x8 x1[HU], x2[HU];
+#pragma unroll
+    for (int u = 0; u < HU; ++u) {
+      if (h0 + u * hs < H) {
+        const bf16_t* hp = row + (long)(h0 + u * hs) * D;
+        x1[u] = *reinterpret_cast<const u16x8*>(hp + i);
+        x2[u] = *reinterpret_cast<const u16x8*>(hp + half + i);
+      }
+    }
     float cc[8], ss[8];
 #pragma unroll
     for (int q4 = 0; q4 < 2; ++q4) {
@@ -180,107 +252,47 @@ __global__ void __launch_bounds__(256) rope_cache_tiled_kernel(
       cc[4 * q4] = c.x; cc[4 * q4 + 1] = c.y; cc[4 * q4 + 2] = c.z; cc[4 * q4 + 3] = c.w;
       ss[4 * q4] = sn.x; ss[4 * q4 + 1] = sn.y; ss[4 * q4 + 2] = sn.z; ss[4 * q4 + 3] = sn.w;
     }
-    // skip_q: the prefill attention rotates q itself (paged_prefill rope_cs)
-    for (int h0 = skip_q ? Hq : 0; h0 < H; h0 += HU) {
-      u16x8 x1[HU], x2[HU];
 #pragma unroll
-      for (int u = 0; u < HU; ++u) {
-        if (h0 + u < H) {
-          const bf16_t* hp = row + (long)(h0 + u) * D;
-          x1[u] = *reinterpret_cast<const u16x8*>(hp + i);
-          x2[u] = *reinterpret_cast<const u16x8*>(hp + half + i);
-        }
-      }
+    for (int u = 0; u < HU; ++u) {
+      const int h = h0 + u * hs;
+      if (h >= H) break;
+      bf16_t* hp = row + (long)h * D;
+      const bool is_k = h >= Hq;
+      float a[8], b[8];
 #pragma unroll
-      for (int u = 0; u < HU; ++u) {
-        const int h = h0 + u;
-        if (h >= H) break;
-        bf16_t* hp = row + (long)h * D;
-        const bool is_k = h >= Hq;
-        float a[8], b[8];
+      for (int j = 0; j < 8; ++j) a[j] = bf2f(x1[u].v[j]), b[j] = bf2f(x2[u].v[j]);
+      if (q_norm) {
+        // per-head RMSNorm of q / k (Qwen3): the head's D values are spread
+        // over the 8 consecutive lanes of this (token, head)
+        float sq = 0.f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) a[j] = bf2f(x1[u].v[j]), b[j] = bf2f(x2[u].v[j]);
-        if (q_norm) {
-          // per-head RMSNorm of q / k (Qwen3): the head's D values are spread
-          // over the 8 consecutive lanes of this (token, head)
-          float sq = 0.f;
+        for (int j = 0; j < 8; ++j) sq += a[j] * a[j] + b[j] * b[j];
 #pragma unroll
-          for (int j = 0; j < 8; ++j) sq += a[j] * a[j] + b[j] * b[j];
-#pragma unroll
-          for (int o = 4; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 8);
-          const float r = rsqrtf(sq / (float)D + eps);
-          const bf16_t* w = is_k ? k_norm : q_norm;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            a[j] *= r * bf2f(w[i + j]);
-            b[j] *= r * bf2f(w[half + i + j]);
-          }
-        }
-        u16x8 o1, o2;
+        for (int o = 4; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 8);
+        const float r = rsqrtf(sq / (float)D + eps);
+        const bf16_t* w = is_k ? k_norm : q_norm;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          o1.v[j] = f2bf(a[j] * cc[j] - b[j] * ss[j]);
-          o2.v[j] = f2bf(b[j] * cc[j] + a[j] * ss[j]);
-        }
-        if (!is_k || rotate_k_inplace || slot < 0) {
-          *reinterpret_cast<u16x8*>(hp + i) = o1;
-          *reinterpret_cast<u16x8*>(hp + half + i) = o2;
-        }
-        if (is_k && slot >= 0 && k_cache) {
-          bf16_t* kp = k_cache + (((long)(slot / BS) * Hkv + (h - Hq)) * BS + slot % BS) * D;
-          *reinterpret_cast<u16x8*>(kp + i) = o1;
-          *reinterpret_cast<u16x8*>(kp + half + i) = o2;
+          a[j] *= r * bf2f(w[i + j]);
+          b[j] *= r * bf2f(w[half + i + j]);
         }
       }
-    }
-  }
-  if (!v_cache || !slot_mapping) return;
-  // HG heads per LDS pass (all 8 of Llama-3 at D 128): two barriers per pass
-  // instead of two per head
-  const int HG = RT_VCOLS / D < Hkv ? RT_VCOLS / D : Hkv;
-  const int LD = HG * D + 8, chunks = HG * D / 8;
-  for (int h0 = 0; h0 < Hkv; h0 += HG) {
-    const int hg = Hkv - h0 < HG ? Hkv - h0 : HG;
-    for (int it = threadIdx.x; it < nt * chunks; it += blockDim.x) {
-      const int tt = it / chunks, c = it - tt * chunks;
-      if (8 * c >= hg * D) continue;
-      const bf16_t* src = qkv + (long)(t0 + tt) * qkv_stride + (long)(Hq + Hkv + h0) * D + 8 * c;
-      *reinterpret_cast<u16x8*>(&vt[tt * LD + 8 * c]) = *reinterpret_cast<const u16x8*>(src);
-    }
-    __syncthreads();
-    // one 16-B store per (head, key quad, d pair): 4 tokens x 2 d of the
-    // key-quad page, whenever the quad's 4 slots are consecutive and
-    // 4-aligned (always, inside a prefill chunk's whole pages)
-    const int per_h = (D / 2) * (RT / 4);
-    for (int it = threadIdx.x; it < hg * per_h; it += blockDim.x) {
-      const int hl = it / per_h, r = it - hl * per_h;
-      const int d = 2 * (r % (D / 2)), tt0 = (r / (D / 2)) * 4, h = h0 + hl;
-      if (tt0 >= nt) continue;
-      const int col = hl * D + d;
-      const int s0 = sslot[tt0];
-      bool vec = tt0 + 4 <= nt && s0 >= 0 && (s0 % 4) == 0;
+      u16x8 o1, o2;
 #pragma unroll
-      for (int j = 1; j < 4; ++j) vec = vec && sslot[tt0 + j] == s0 + j;
-      if (vec) {
-        u16x8 w;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          w.v[j] = vt[(tt0 + j) * LD + col];
-          w.v[4 + j] = vt[(tt0 + j) * LD + col + 1];
-        }
-        *reinterpret_cast<u16x8*>(v_cache + ((long)(s0 / BS) * Hkv + h) * BS * D +
-                                  vq_off(d, s0 % BS, D)) = w;
-      } else {
-        for (int j = 0; j < 4 && tt0 + j < nt; ++j) {
-          const int sl = sslot[tt0 + j];
-          if (sl < 0) continue;
-          bf16_t* vp = v_cache + ((long)(sl / BS) * Hkv + h) * BS * D + vq_off(d, sl % BS, D);
-          vp[0] = vt[(tt0 + j) * LD + col];
-          vp[4] = vt[(tt0 + j) * LD + col + 1];
-        }
+      for (int j = 0; j < 8; ++j) {
+        o1.v[j] = f2bf(a[j] * cc[j] - b[j] * ss[j]);
+        o2.v[j] = f2bf(b[j] * cc[j] + a[j] * ss[j]);
+      }
+      if (!is_k || rotate_k_inplace || slot < 0) {
+        *reinterpret_cast<u16x8*>(hp + i) = o1;
+        *reinterpret_cast<u16x8*>(hp + half + i) = o2;
+      }
+      if (is_k && slot >= 0 && k_cache) {
+        bf16_t* kp = k_cache + (((long)(slot / BS) * Hkv + (h - Hq)) * BS + slot % BS) * D;
+        *reinterpret_cast<u16x8*>(kp + i) = o1;
+        *reinterpret_cast<u16x8*>(kp + half + i) = o2;
       }
     }
-    __syncthreads();
   }
 }
 
@@ -310,19 +322,14 @@ int rope_cache(void* qkv, long qkv_stride, const int* positions, const float* co
 #undef LMX_RC
   }
   if (T > n1) {
-    const size_t smem = v_cache && slot_mapping ? rope_tile_smem(Hkv, D) : 0;
-    static size_t attr = 0;
-    if (smem > 65536 && smem > attr) {
-      const hipError_t e = hipFuncSetAttribute((const void*)rope_cache_tiled_kernel,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)smem);
-      if (e != hipSuccess) return (int)e;
-      attr = smem;
-    }
-    rope_cache_tiled_kernel<<<dim3((T - n1 + RT - 1) / RT), dim3(256), smem, stream>>>(
+    const bool v = v_cache && slot_mapping;
+    const int hv = rope_v_heads(D), per = 4 * rope_head_step(D);
+    const int rot = ((skip_q ? Hkv : Hq + Hkv) + per - 1) / per, vg = v ? (Hkv + hv - 1) / hv : 0;
+    const size_t smem = v ? (size_t)RT * (hv * D + 8) * sizeof(bf16_t) : 0;
+    rope_cache_tiled_kernel<<<dim3((T - n1 + RT - 1) / RT, rot + vg), dim3(256), smem, stream>>>(
         (bf16_t*)qkv, qkv_stride, positions, cos_sin, n1, T, Hq, Hkv, D, slot_mapping,
         (bf16_t*)k_cache, (bf16_t*)v_cache, BS, rotate_k_inplace, (const bf16_t*)q_norm,
-        (const bf16_t*)k_norm, eps, skip_q);
+        (const bf16_t*)k_norm, eps, skip_q, rot);
   }
   return (int)hipGetLastError();
 }
@@ -582,8 +589,8 @@ int qkv_norm_rope_cache(const void* p, long p_ld, const float* bias, const float
   return (int)hipGetLastError();
 }
 
-// Plain cache write (no rotation), used by the paged-cache tests and by
-// models without rotary embeddings.
+// Plain cache write (no rotation): models without rotary embeddings.  Any head
+// size and alignment, one token per workgroup.
 __global__ void kv_write_kernel(const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
                                 long kv_stride, const int* __restrict__ slot_mapping, int Hkv,
                                 int D, bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache,
@@ -599,9 +606,51 @@ __global__ void kv_write_kernel(const bf16_t* __restrict__ k, const bf16_t* __re
   }
 }
 
+// The same for rows of whole 16-B pieces: grid (32-token tiles, K groups + V
+// groups) as rope_cache_tiled_kernel, V in key quads through LDS instead of 2-B
+// stores 8 B apart.  19,153 tokens of 16 heads of 64: 53 -> 39 us (157 MB).
+__global__ void __launch_bounds__(256) kv_write_tiled_kernel(
+    const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, long kv_stride,
+    const int* __restrict__ slot_mapping, int T, int Hkv, int D, bf16_t* __restrict__ k_cache,
+    bf16_t* __restrict__ v_cache, int BS, int k_groups) {
+  extern __shared__ __attribute__((aligned(16))) bf16_t vt[];
+  __shared__ int sslot[RT];
+  const int t0 = blockIdx.x * RT, nt = min(RT, T - t0);
+  if (threadIdx.x < RT) sslot[threadIdx.x] = threadIdx.x < nt ? slot_mapping[t0 + threadIdx.x] : -1;
+  __syncthreads();
+  const int hv = rope_v_heads(D);
+  const bool is_k = (int)blockIdx.y < k_groups;
+  const int h0 = ((int)blockIdx.y - (is_k ? 0 : k_groups)) * hv, hg = min(hv, Hkv - h0);
+  if (!is_k) {
+    v_to_pages(v + (long)t0 * kv_stride, kv_stride, nt, h0, hg, Hkv, D, sslot, vt, hv * D + 8, v_cache,
+               BS);
+    return;
+  }
+  const int per = D / 8, chunks = hg * per;
+#pragma unroll 4
+  for (int it = threadIdx.x; it < nt * chunks; it += 256) {
+    const int tt = it / chunks, c = it - tt * chunks, h = h0 + c / per;
+    const int slot = sslot[tt];
+    if (slot < 0) continue;
+    *reinterpret_cast<u16x8*>(k_cache + (((long)(slot / BS) * Hkv + h) * BS + slot % BS) * D +
+                              c % per * 8) =
+        *reinterpret_cast<const u16x8*>(k + (long)(t0 + tt) * kv_stride + (long)h0 * D + 8 * c);
+  }
+}
+
 int kv_write(const void* k, const void* v, long kv_stride, const int* slot_mapping, int T, int Hkv,
              int D, void* k_cache, void* v_cache, int BS, hipStream_t stream) {
   if (T <= 0) return 0;
+  // whole 16-B pieces of rows and pages, whole key quads (BS % 4)
+  if (D % 8 == 0 && D <= 256 && BS % 4 == 0 && kv_stride % 8 == 0 &&
+      (((uintptr_t)k | (uintptr_t)v | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0) {
+    const int hv = rope_v_heads(D), groups = (Hkv + hv - 1) / hv;
+    kv_write_tiled_kernel<<<dim3((T + RT - 1) / RT, 2 * groups), dim3(256),
+                            (size_t)RT * (hv * D + 8) * sizeof(bf16_t), stream>>>(
+        (const bf16_t*)k, (const bf16_t*)v, kv_stride, slot_mapping, T, Hkv, D, (bf16_t*)k_cache,
+        (bf16_t*)v_cache, BS, groups);
+    return (int)hipGetLastError();
+  }
   kv_write_kernel<<<dim3(T), dim3(256), 0, stream>>>((const bf16_t*)k, (const bf16_t*)v,
                                                      kv_stride, slot_mapping, Hkv, D,
                                                      (bf16_t*)k_cache, (bf16_t*)v_cache, BS);
