@@ -13,6 +13,7 @@
 #include <string>
 
 #include "delta.h"
+#include "encoder.h"
 
 namespace lmx {
 int rmsnorm(void*, void*, const void*, const void*, int, int, long, long, float, hipStream_t);
@@ -128,7 +129,11 @@ int gemm_splitk(void*, const void*, const void*, float*, int*, int, int, int, lo
 int gemm_nt(void*, const void*, const void*, const void*, const void*, int, int, int, long, long,
             long, int, hipStream_t);
 int dgemm(void*, const void*, const void*, float*, unsigned*, int, int, int, int, long, long, long,
-          int, int, int, hipStream_t);
+          int, int, int, hipStream_t, const void*);
+int layernorm_slabs(void*, const float*, int, long, const void*, const void*, const void*, const void*,
+                    int, int, float, hipStream_t);
+int embed_layernorm(void*, const int*, const void*, int, const void*, const void*, const int*,
+                    const void*, const void*, int, int, float, hipStream_t);
 int dgemm_num_configs();
 int rsgemm(void*, const void*, const void*, float*, unsigned*, int, int, int, int, long, long, long,
            int, int, int, hipStream_t);
@@ -564,10 +569,43 @@ PYBIND11_MODULE(_lmx_kernels, m) {
   });
   m.def("dgemm", [](uptr C, uptr A, uptr W, uptr slabs, uptr tickets, int n_tickets, int M, int N,
                     int K, long lda, long ldw, long ldc, int cfg, int splits, int epi,
-                    uptr stream) {
+                    uptr stream, uptr bias) {
     check(lmx::dgemm(P<void>(C), P<void>(A), P<void>(W), P<float>(slabs), P<unsigned>(tickets),
-                     n_tickets, M, N, K, lda, ldw, ldc, cfg, splits, epi, S(stream)),
+                     n_tickets, M, N, K, lda, ldw, ldc, cfg, splits, epi, S(stream), P<void>(bias)),
           "dgemm");
+  }, py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(),
+     py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg("bias") = 0);
+  m.def("layernorm_slabs", [](uptr out, uptr slabs, int nsl, long stride, uptr bias, uptr residual,
+                              uptr w, uptr b, int rows, int cols, float eps, uptr stream) {
+    check(lmx::layernorm_slabs(P<void>(out), P<float>(slabs), nsl, stride, P<void>(bias),
+                               P<void>(residual), P<void>(w), P<void>(b), rows, cols, eps, S(stream)),
+          "layernorm_slabs");
+  });
+  m.def("embed_layernorm", [](uptr out, uptr ids, uptr word, int vocab, uptr type, uptr pos,
+                              uptr positions, uptr w, uptr b, int rows, int cols, float eps,
+                              uptr stream) {
+    check(lmx::embed_layernorm(P<void>(out), P<int>(ids), P<void>(word), vocab, P<void>(type),
+                               P<void>(pos), P<int>(positions), P<void>(w), P<void>(b), rows, cols, eps,
+                               S(stream)),
+          "embed_layernorm");
+  });
+  m.def("enc_plan", [](int M, int N, int K, int act, bool partials) {
+    const lmx::EncPlan p = lmx::enc_plan(M, N, K, act, partials);
+    return std::make_pair(p.cfg, p.splits);
+  });
+  m.def("enc_slab_floats", &lmx::enc_slab_floats);
+  m.def("encoder_layers", [](const std::vector<uintptr_t>& w, int T, int d, int I, int H, int D, int page,
+                             bool gelu, float eps, float scale, uptr x, uptr h, uptr qkv, uptr attn,
+                             uptr g, uptr slabs, long slab_floats, uptr kc, uptr vc, uptr slots,
+                             uptr positions, uptr cos_sin, uptr bt, int bt_stride, uptr cu, uptr ctx,
+                             uptr tiles, int ntiles, int q_per_tile, uptr stream) {
+    if (w.size() % lmx::kEncPtrs) throw std::runtime_error("encoder_layers: weights");
+    const lmx::EncArgs a{(int)(w.size() / lmx::kEncPtrs), T, d, I, H, D, page, gelu, eps, scale,
+                         P<void>(x), P<void>(h), P<void>(qkv), P<void>(attn), P<void>(g),
+                         P<float>(slabs), slab_floats, P<void>(kc), P<void>(vc), P<int>(slots),
+                         P<int>(positions), P<float>(cos_sin), P<int>(bt), bt_stride, P<int>(cu),
+                         P<int>(ctx), P<int>(tiles), ntiles, q_per_tile};
+    check(lmx::encoder_layers(a, w.data(), S(stream)), "encoder_layers");
   });
   m.def("rmsnorm_slabs", [](uptr out, uptr residual, uptr slabs, int nsl, long slab_stride,
                             uptr w, int rows, int cols, long out_stride, float eps, uptr stream) {

@@ -90,6 +90,26 @@ __device__ __forceinline__ bf16x8_t load_frag16B(const bf16_t* p) {
   return *reinterpret_cast<const bf16x8_t*>(p);
 }
 
+// x/2 (1 + erf(x / sqrt 2)): erfc(z) = e^(-z^2) t Q(t), t = 1 / (1 + 0.375 z), Q a minimax fit
+// (relative, z to 10) of erfcx(z) / t, so the negative side does not cancel. In fp32 on [-12, 12]:
+// at most 2.4e-7 off (1.3e-6 of the value from -3 up, 2.5e-6 from -6), where 1 + erff(.) is
+// 4.5e-7 off (1.1e-5; all digits). 16 instructions and two special ones, no branch; erff takes
+// both of its branches in a wave.
+__device__ __forceinline__ float gelu_erf(float x) {
+  const float a = fabsf(x);
+  const float t = __builtin_amdgcn_rcpf(fmaf(0.375f * 0.70710678f, a, 1.f));
+  float q = -0.1350931335f;
+  q = fmaf(q, t, 0.3879281462f);
+  q = fmaf(q, t, -0.1295836224f);
+  q = fmaf(q, t, 0.2830515626f);
+  q = fmaf(q, t, 0.1666685279f);
+  q = fmaf(q, t, 0.2156883690f);
+  q = fmaf(q, t, 0.2113395155f);
+  const float e = fast_exp2(x * x * -0.72134752f) * (t * q);
+  const float h = 0.5f * fminf(a, 64.f) * e;            // e is 0 there: no inf * 0
+  return fmaf(0.5f, a, 0.5f * x) - h;
+}
+
 // Two 8-byte halves -> one fragment (used for permuted-k operands).
 // V-cache page layout [BS/4][D][4] ("key-quad"): the 4 consecutive keys of
 // one d are 8 contiguous bytes (the 8-B V^T fragment run of the PV MFMA), and

@@ -189,7 +189,7 @@ template <int BM, int BN, int WM, int NST, int EPI, int ROT, int NT, int BK>
 __global__ void __launch_bounds__(DTHREADS, 2) dgemm_kernel(
     bf16_t* __restrict__ C, const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
     float* __restrict__ slabs, unsigned* __restrict__ tickets, int M, int N, int K, long lda,
-    long ldw, long ldc, int splits) {
+    long ldw, long ldc, int splits, const bf16_t* __restrict__ bias) {
   constexpr int WN = 8 / WM;
   constexpr int WTM = BM / WM, WTN = BN / WN;       // wave tile
   constexpr int TM = WTM / 16, TN = WTN / 16;       // 16x16 MFMA tiles per wave
@@ -293,7 +293,18 @@ __global__ void __launch_bounds__(DTHREADS, 2) dgemm_kernel(
     __syncthreads();            // the SwiGLU hand-off below reuses the LDS word of the flag
   }
 
-  if (EPI == 0) {
+  if (EPI == 0 || EPI == 5 || EPI == 6) {
+    // 5: + bias, 6: gelu(. + bias), the exact form
+    f32x4_t b[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      b[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if constexpr (EPI != 0) {
+        const bf16x4_t v = *reinterpret_cast<const bf16x4_t*>(bias + n0 + wc * WTN + 16 * j + 4 * fg);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) b[j][r] = bf2f((uint16_t)v[r]);
+      }
+    }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int m = m0 + wr * WTM + 16 * i + fr;
@@ -303,7 +314,10 @@ __global__ void __launch_bounds__(DTHREADS, 2) dgemm_kernel(
         const int n = n0 + wc * WTN + 16 * j + 4 * fg;
         bf16x4_t o;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = (short)f2bf(acc[i][j][r]);
+        for (int r = 0; r < 4; ++r) {
+          const float v = EPI == 0 ? acc[i][j][r] : acc[i][j][r] + b[j][r];
+          o[r] = (short)f2bf(EPI == 6 ? gelu_erf(v) : v);
+        }
         *reinterpret_cast<bf16x4_t*>(C + (long)m * ldc + n) = o;
       }
     }
@@ -521,7 +535,7 @@ int dgemm_sk_pieces(int M, int N, int K, int cfg, int groups) {
 template <int BM, int BN, int WM, int NST, int EPI, int ROT, int NT, int BK>
 static int dg_launch(bf16_t* C, const bf16_t* A, const bf16_t* W, float* slabs,
                      unsigned* tickets, int M, int N, int K, long lda, long ldw, long ldc,
-                     int splits, hipStream_t stream) {
+                     int splits, hipStream_t stream, const bf16_t* bias = nullptr) {
   constexpr size_t ring = (size_t)NST * (BM + BN) * BK * sizeof(bf16_t);
   constexpr size_t xchg = EPI == 1 ? (size_t)BM * (BN / 2 + 4) * 4 : 0;   // SwiGLU hand-off
   constexpr size_t smem = ring > xchg ? ring : xchg;
@@ -536,7 +550,7 @@ static int dg_launch(bf16_t* C, const bf16_t* A, const bf16_t* W, float* slabs,
   }
   const int nwg = ((M + BM - 1) / BM) * (N / BN) * splits;
   dgemm_kernel<BM, BN, WM, NST, EPI, ROT, NT, BK><<<dim3(nwg), dim3(DTHREADS), smem, stream>>>(
-      C, A, W, slabs, tickets, M, N, K, lda, ldw, ldc, splits);
+      C, A, W, slabs, tickets, M, N, K, lda, ldw, ldc, splits, bias);
   return (int)hipGetLastError();
 }
 
@@ -564,14 +578,21 @@ static int dg_sk_launch(bf16_t* C, const bf16_t* A, const bf16_t* W, float* slab
   return (int)hipGetLastError();
 }
 
+// tiles with the bias epilogues: those the encoders' rule picks (encoder.hip enc_plan)
+static constexpr bool dg_bias_tile(int bm, int bn, int bk) {
+  return bk == 128 ? bm <= 128 && bn <= 128 : bm == 128 && bn == 256;
+}
+
+// bias (bf16 [N]): with epi 5 (C = A . W^T + bias) and 6 (gelu of it, the exact form)
 int dgemm(void* C, const void* A, const void* W, float* slabs, unsigned* tickets, int n_tickets,
           int M, int N, int K, long lda, long ldw, long ldc, int cfg, int splits, int epi,
-          hipStream_t stream) {
+          hipStream_t stream, const void* bias) {
   if (M <= 0) return 0;
   const int nt = (cfg >> 5) & 1;      // bit 5: non-temporal weight stream
   const int sk = (cfg >> 6) & 1;      // bit 6: stream-K, `splits` = workgroups (0: 256)
   cfg &= 31;
-  if (cfg < 0 || cfg >= kNumDgCfgs || splits < 0 || epi < 0 || epi > 4) return -1;
+  if (cfg < 0 || cfg >= kNumDgCfgs || splits < 0 || epi < 0 || epi > 6) return -1;
+  if ((epi >= 5) != (bias != nullptr) || (epi >= 5 && nt)) return -1;
   const DgCfg c = kDgCfgs[cfg];
   if (sk) {
     if (epi != 0 || N % c.bn != 0 || K % c.bk != 0) return -1;
@@ -587,6 +608,7 @@ int dgemm(void* C, const void* A, const void* W, float* slabs, unsigned* tickets
   auto C_ = (bf16_t*)C;
   auto A_ = (const bf16_t*)A;
   auto W_ = (const bf16_t*)W;
+  auto b_ = (const bf16_t*)bias;
 #define LMX_DG_E(BM, BN, WM, NST, ROT, NT, BK)                                                 \
   if (sk)                                                                                     \
     return dg_sk_launch<BM, BN, WM, NST, NT, BK>(C_, A_, W_, slabs, M, N, K, lda, ldw, ldc,   \
@@ -601,6 +623,16 @@ int dgemm(void* C, const void* A, const void* W, float* slabs, unsigned* tickets
     if constexpr ((BN / (8 / WM)) % 32 == 0)                                                  \
       return dg_launch<BM, BN, WM, NST, 4, ROT, NT, BK>(C_, A_, W_, slabs, tickets, M, N, K, \
                                                         lda, ldw, ldc, splits, stream);       \
+    return -1;                                                                                \
+  }                                                                                           \
+  if (epi >= 5) {                                                                             \
+    if constexpr (!NT && dg_bias_tile(BM, BN, BK)) {                                          \
+      if (epi == 5)                                                                           \
+        return dg_launch<BM, BN, WM, NST, 5, ROT, NT, BK>(C_, A_, W_, slabs, tickets, M, N, K, \
+                                                          lda, ldw, ldc, splits, stream, b_); \
+      return dg_launch<BM, BN, WM, NST, 6, ROT, NT, BK>(C_, A_, W_, slabs, tickets, M, N, K,  \
+                                                        lda, ldw, ldc, splits, stream, b_);   \
+    }                                                                                         \
     return -1;                                                                                \
   }                                                                                           \
   if (epi == 1)                                                                               \

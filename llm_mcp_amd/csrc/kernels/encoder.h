@@ -1,0 +1,37 @@
+// Arguments of encoder_layers (encoder.hip), filled by the bindings.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace lmx {
+
+// weights of a layer, in this order, 0 where there is none: Wqkv, its bias, Wo, bias, the
+// first norm's gain and shift, W1 (gate / up interleaved by 16 rows, or the plain one), bias,
+// W2, bias, the second norm's gain and shift
+constexpr int kEncPtrs = 12;
+
+struct EncArgs {
+  int layers, T, d, I, H, D, page;
+  bool gelu;                       // gelu(h W1 + b) instead of SwiGLU
+  float eps, scale;
+  // rows of T tokens, bf16: x [d] (in: the first norm's output, out: the last one's),
+  // h [d], qkv [3 d], attn [d], g [I]
+  void *x, *h, *qkv, *attn, *g;
+  float* slabs;
+  long slab_floats;
+  void *kc, *vc;                   // pages of this forward
+  const int *slots, *positions;    // per token
+  const float* cos_sin;            // null: no rotation
+  const int* bt;                   // page tables [sequences][bt_stride]
+  int bt_stride;
+  const int *cu, *ctx, *tiles;
+  int ntiles, q_per_tile;
+};
+
+struct EncPlan { int cfg, splits; };   // cfg -1: K13
+
+EncPlan enc_plan(int M, int N, int K, int act, bool partials);
+long enc_slab_floats(int T, int d, int I);
+int encoder_layers(const EncArgs& a, const uintptr_t* w, hipStream_t stream);
+
+}  // namespace lmx

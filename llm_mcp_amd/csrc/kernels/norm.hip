@@ -193,6 +193,103 @@ __global__ void __launch_bounds__(256) layernorm_kernel(
   }
 }
 
+// LayerNorm of a projection whose K reduction is left to it: out = LN(sum of S
+// fp32 slabs + bias + residual), the sum in slab order and unrounded. One row per
+// workgroup as above: memory bound for many rows; for few, the S loads of a chunk
+// are in flight together, so the reduction costs no pass of its own (a 16-row
+// encoder step: 4.0 us with 12 slabs, as the plain LayerNorm).
+template <int S>
+__global__ void __launch_bounds__(256) layernorm_slabs_kernel(
+    bf16_t* __restrict__ out, const float* __restrict__ slabs, long slab_stride,
+    const bf16_t* __restrict__ bias, const bf16_t* __restrict__ residual,
+    const bf16_t* __restrict__ w, const bf16_t* __restrict__ b, int cols, float eps) {
+  __shared__ float scratch[16];
+  const int row = blockIdx.x, c = threadIdx.x * 8;
+  const bool on = c < cols;
+  float v[8], wv[8], bv[8];
+  float s = 0.f;
+  if (on) {
+    const float* x = slabs + (long)row * cols + c;
+    f32x4_t p0[S], p1[S];
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+      p0[k] = *reinterpret_cast<const f32x4_t*>(x + k * slab_stride);
+      p1[k] = *reinterpret_cast<const f32x4_t*>(x + k * slab_stride + 4);
+    }
+    float r[8], pb[8];
+    ldv<8>(r, residual + (long)row * cols + c);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) pb[j] = 0.f;
+    if (bias) ldv<8>(pb, bias + c);
+    ldv<8>(wv, w + c);
+    ldv<8>(bv, b + c);
+#pragma unroll
+    for (int k = 1; k < S; ++k) {
+      p0[0] += p0[k];
+      p1[0] += p1[k];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      v[j] = (j < 4 ? p0[0][j & 3] : p1[0][j & 3]) + pb[j] + r[j];
+      s += v[j];
+    }
+  }
+  const float mean = block_sum(s, scratch) / (float)cols;
+  float sq = 0.f;
+  if (on)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) { const float d = v[j] - mean; sq += d * d; }
+  const float inv = rsqrtf(block_sum(sq, scratch) / (float)cols + eps);
+  if (on) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (v[j] - mean) * inv * wv[j] + bv[j];
+    stv<8>(out + (long)row * cols + c, v);
+  }
+}
+
+// The encoders' input: LN(word[id] + type + pos[position]) of every token, summed in
+// fp32 (ids outside the table count as a zero row). pos: null without absolute positions.
+__global__ void __launch_bounds__(256) embed_layernorm_kernel(
+    bf16_t* __restrict__ out, const int* __restrict__ ids, const bf16_t* __restrict__ word, int vocab,
+    const bf16_t* __restrict__ type, const bf16_t* __restrict__ pos,
+    const int* __restrict__ positions, const bf16_t* __restrict__ w, const bf16_t* __restrict__ b,
+    int cols, float eps) {
+  __shared__ float scratch[16];
+  const int row = blockIdx.x, c = threadIdx.x * 8, id = ids[row];
+  const bool on = c < cols;
+  float v[8], t[8];
+  float s = 0.f;
+  if (on) {
+    ldv<8>(v, type + c);
+    if (pos) {
+      ldv<8>(t, pos + (long)positions[row] * cols + c);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] += t[j];
+    }
+    if (id >= 0 && id < vocab) {
+      ldv<8>(t, word + (long)id * cols + c);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] += t[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s += v[j];
+  }
+  const float mean = block_sum(s, scratch) / (float)cols;
+  float sq = 0.f;
+  if (on)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) { const float d = v[j] - mean; sq += d * d; }
+  const float inv = rsqrtf(block_sum(sq, scratch) / (float)cols + eps);
+  if (on) {
+    float wv[8];
+    ldv<8>(wv, w + c);
+    ldv<8>(t, b + c);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (v[j] - mean) * inv * wv[j] + t[j];
+    stv<8>(out + (long)row * cols + c, v);
+  }
+}
+
 static int pick_threads(int nchunk) {
   int t = ((nchunk + 63) / 64) * 64;
   return t > 256 ? 256 : (t < 64 ? 64 : t);
@@ -342,6 +439,37 @@ int layernorm(void* out, const void* x, const void* residual, const void* w, con
   else if (vpt <= 8) LMX_LN(8);
   else return -2;
 #undef LMX_LN
+  return (int)hipGetLastError();
+}
+
+int layernorm_slabs(void* out, const float* slabs, int S, long slab_stride, const void* bias,
+                    const void* residual, const void* w, const void* b, int rows, int cols, float eps,
+                    hipStream_t stream) {
+  if (rows <= 0) return 0;
+  if (cols % 8 != 0 || cols > 2048 || !slabs || !residual) return -1;
+  const dim3 g(rows), bl(pick_threads(cols / 8));
+#define LMX_LNS(SS)                                                                            \
+  case SS:                                                                                     \
+    layernorm_slabs_kernel<SS><<<g, bl, 0, stream>>>(                                          \
+        (bf16_t*)out, slabs, slab_stride, (const bf16_t*)bias, (const bf16_t*)residual,        \
+        (const bf16_t*)w, (const bf16_t*)b, cols, eps);                                        \
+    break;
+  switch (S) {
+    LMX_LNS(1) LMX_LNS(2) LMX_LNS(3) LMX_LNS(4) LMX_LNS(6) LMX_LNS(8) LMX_LNS(12) LMX_LNS(16)
+    default: return -3;
+  }
+#undef LMX_LNS
+  return (int)hipGetLastError();
+}
+
+int embed_layernorm(void* out, const int* ids, const void* word, int vocab, const void* type,
+                    const void* pos, const int* positions, const void* w, const void* b, int rows,
+                    int cols, float eps, hipStream_t stream) {
+  if (rows <= 0) return 0;
+  if (cols % 8 != 0 || cols > 2048 || (pos && !positions)) return -1;
+  embed_layernorm_kernel<<<dim3(rows), dim3(pick_threads(cols / 8)), 0, stream>>>(
+      (bf16_t*)out, ids, (const bf16_t*)word, vocab, (const bf16_t*)type, (const bf16_t*)pos,
+      positions, (const bf16_t*)w, (const bf16_t*)b, cols, eps);
   return (int)hipGetLastError();
 }
 

@@ -97,7 +97,7 @@ __device__ __forceinline__ float pg_act(float v) {
   } else if constexpr (ACT == 2) {
     return v / (1.f + __expf(-v));
   } else if constexpr (ACT == 4) {
-    return 0.5f * v * (1.f + erff(v * 0.70710678118f));
+    return gelu_erf(v);
   } else if constexpr (ACT == 7) {
     v = fmaxf(v, 0.f);
     return v * v;

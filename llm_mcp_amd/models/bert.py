@@ -28,9 +28,12 @@ import numpy as np
 import torch
 
 from .. import ops
+from ..ops import encoder
 from .config import BertConfig
 
-PAGE = 32
+PAGE = encoder.PAGE
+# a layer's tensors in the order of csrc/kernels/encoder.h
+NATIVE = ("wqkv", "bqkv", "wo", "bo", "ln1_w", "ln1_b", "w1", "b1", "w2", "b2", "ln2_w", "ln2_b")
 
 
 class BertModel:
@@ -99,6 +102,16 @@ class BertModel:
         ln = np.asarray(lens, dtype=np.int64)
         if int(ln.max()) > cfg.max_position:
             raise ValueError(f"sequence longer than {cfg.max_position} positions")
+        if ids.is_cuda and encoder.layers_ok(w["layers"], NATIVE, d, cfg.intermediate_size, H, D):
+            qpt = ops.prefill_q_per_tile(H, H, D)
+            b = encoder.batch(lens, qpt, ids.device)
+            x = encoder.embed_norm(ids, w["word"], w["type"], w["emb_ln_w"], w["emb_ln_b"],
+                                   cfg.ln_eps, w["pos"], b.positions)
+            encoder.layers(x, w["layers"], NATIVE, b, cu, cfg.intermediate_size, H, D, cfg.ln_eps,
+                           self.scale, qpt, True, None)
+            if cfg.pooling == "cls":     # the first tokens' rows as sequences of one
+                x, cu = ops.embed_gather(x, b.first), b.count
+            return ops.mean_pool_l2(x, cu, dims or cfg.embed_dim, normalize)
         pages = np.maximum(1, -(-ln // PAGE))
         page_off = np.concatenate([[0], np.cumsum(pages)])
         NB = int(page_off[-1])

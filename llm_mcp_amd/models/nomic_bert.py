@@ -31,10 +31,13 @@ import numpy as np
 import torch
 
 from .. import ops
-from ..ops import ref
+from ..ops import encoder, ref
 from .config import NomicBertConfig
 
-PAGE = 32
+PAGE = encoder.PAGE
+# a layer's tensors in the order of csrc/kernels/encoder.h (no biases)
+NATIVE = ("wqkv", None, "wo", None, "ln1_w", "ln1_b", "w_gu_il", None, "w_down", None, "ln2_w",
+          "ln2_b")
 
 
 class NomicBertModel:
@@ -107,6 +110,15 @@ class NomicBertModel:
         H, D, d = self.H, self.D, cfg.hidden_size
         T, S = ids.numel(), len(lens)
         dev = self.device
+        if ids.is_cuda and self.gu_k13 and not self.fuse_q_rope and encoder.layers_ok(
+                w["layers"], tuple(n for n in NATIVE if n), d, cfg.intermediate_size, H, D):
+            qpt = ops.prefill_q_per_tile(H, H, D)
+            b = encoder.batch(lens, qpt, ids.device)
+            x = encoder.embed_norm(ids, w["word"], w["type"], w["emb_ln_w"], w["emb_ln_b"],
+                                   cfg.ln_eps)
+            encoder.layers(x, w["layers"], NATIVE, b, cu, cfg.intermediate_size, H, D, cfg.ln_eps,
+                           self.scale, qpt, False, self.cos_sin)
+            return ops.mean_pool_l2(x, cu, dims or cfg.embed_dim, normalize)
         # per-sequence page-aligned slots in a scratch paged K/V cache, built
         # with array ops (no per-token Python work on the host critical path)
         ln = np.asarray(lens, dtype=np.int64)

@@ -91,3 +91,116 @@ def test_conv_parts(C, taps):
     ref.short_conv(u, w, bias, state, cu, ctx, slots, want, True)
     torch.testing.assert_close(y.float().cpu(), want, atol=2e-2, rtol=1e-2)
     assert torch.equal(st.cpu(), state)
+
+
+# ----------------------------------------------------------------- encoders --
+def _values():
+    """bf16 numbers over the range where gelu is neither 0 nor its argument, and far out."""
+    v = torch.cat([torch.linspace(-14, 14, 3800), torch.logspace(-38, 38, 148),
+                   -torch.logspace(-38, 38, 148)])
+    return v.bfloat16()
+
+
+@pytest.mark.parametrize("kernel", ["pgemm", "dgemm"])
+def test_gelu_erf_epilogue(kernel):
+    """gelu of given values (a product with a unit vector): the correctly rounded result
+    or its neighbour -- at most 2.5e-6 of the value off before the rounding."""
+    v, K = _values(), 256
+    N = v.numel() // 256 * 256
+    w = torch.zeros(N, K, dtype=torch.bfloat16)
+    w[:, 3] = v[:N]
+    a = torch.zeros(3, K, dtype=torch.bfloat16)
+    a[:, 3] = 1
+    a, w, b = a.to(DEV), w.to(DEV), torch.zeros(N, device=DEV, dtype=torch.bfloat16)
+    if kernel == "pgemm":
+        y = ops.pgemm(a, w, bias=b, act=ops.ACT_GELU_ERF)
+    else:
+        y = torch.empty(3, N, device=DEV, dtype=torch.bfloat16)
+        ops.native().dgemm(y.data_ptr(), a.data_ptr(), w.data_ptr(), 0, 0, 0, 3, N, K, K, K, N, 31, 1,
+                           6, torch.cuda.current_stream().cuda_stream, b.data_ptr())
+    x = v[:N].double()
+    want = torch.where(x < 0, 0.5 * x * torch.special.erfc(-x / 2 ** 0.5),
+                       x - 0.5 * x * torch.special.erfc(x / 2 ** 0.5)).to(DEV)
+    # half a unit in the last place and the 2.5e-6; below 2^-126 results flush to zero (z over 13)
+    err = (y.double() - want).abs()
+    assert bool((err <= want.abs() * (2.0 ** -8 + 3e-6) + 2.0 ** -125).all())
+
+
+@pytest.mark.parametrize("cfg", [21, 31, 20, 22, 11])
+@pytest.mark.parametrize("M", [1, 63, 64, 129, 300])
+def test_dgemm_bias_epilogues(cfg, M):
+    """Every tile of the encoders' rule: + bias, gelu(+ bias), edges of row tiles."""
+    N, K = 512, 256
+    a, w, b = (torch.randn(M, K, device=DEV).bfloat16(), torch.randn(N, K, device=DEV).bfloat16() * 0.1,
+               torch.randn(N, device=DEV).bfloat16())
+    z = a.float() @ w.float().t() + b.float()
+    for epi, want in ((5, z), (6, torch.nn.functional.gelu(z))):
+        y = torch.full((M, N), 7.0, device=DEV).bfloat16()
+        ops.native().dgemm(y.data_ptr(), a.data_ptr(), w.data_ptr(), 0, 0, 0, M, N, K, K, K, N, cfg, 1,
+                           epi, torch.cuda.current_stream().cuda_stream, b.data_ptr())
+        # one bf16 rounding of an fp32 sum of 256 products
+        torch.testing.assert_close(y.float(), want, atol=2e-3, rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("S", [1, 2, 3, 4, 6, 8, 12, 16])
+@pytest.mark.parametrize("rows,cols,bias", [(1, 768, True), (17, 1024, False), (5, 2048, True),
+                                            (3, 264, True)])
+def test_layernorm_slabs(S, rows, cols, bias):
+    p = torch.randn(S, rows, cols, device=DEV)
+    r, w, b, c = (torch.randn(*s, device=DEV).bfloat16()
+                  for s in ((rows, cols), (cols,), (cols,), (cols,)))
+    y = torch.empty_like(r)
+    ops.native().layernorm_slabs(y.data_ptr(), p.data_ptr(), S, rows * cols,
+                                 c.data_ptr() if bias else 0, r.data_ptr(), w.data_ptr(), b.data_ptr(),
+                                 rows, cols, 1e-12, torch.cuda.current_stream().cuda_stream)
+    x = p.double().sum(0) + r.double() + (c.double() if bias else 0)
+    want = torch.nn.functional.layer_norm(x, (cols,), w.double(), b.double(), 1e-12)
+    torch.testing.assert_close(y.double(), want, atol=1e-4, rtol=2.0 ** -8)
+
+
+def test_embed_norm():
+    from llm_mcp_amd.ops import encoder
+    word, typ, pos = (torch.randn(s, 768, device=DEV).bfloat16() for s in (50, 2, 40))
+    w, b = torch.randn(768, device=DEV).bfloat16(), torch.randn(768, device=DEV).bfloat16()
+    ids, at = _i32([0, 49, 7, 50, -1]), _i32([0, 39, 3, 1, 2])       # two outside the table
+    for p in (None, pos):
+        y = encoder.embed_norm(ids, word, typ, w, b, 1e-12, p, at)
+        x = torch.stack([word[i].double() if 0 <= i < 50 else torch.zeros(768, device=DEV).double()
+                         for i in ids.tolist()]) + typ[0].double()
+        x = x if p is None else x + pos[at.long()].double()
+        want = torch.nn.functional.layer_norm(x, (768,), w.double(), b.double(), 1e-12)
+        torch.testing.assert_close(y.double(), want, atol=1e-4, rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("model", ["nomic-embed-text", "mxbai-embed-large"])
+def test_encoder_batches_agree(model):
+    """One document alone, in a small batch and in a large one: other tiles, slices and
+    kernels, the same vector to bf16 accuracy; and the models' own loop over single ops."""
+    import dataclasses
+
+    from llm_mcp_amd.models import config as mc
+    from llm_mcp_amd.models.bert import BertModel
+    from llm_mcp_amd.models.nomic_bert import NomicBertModel
+    cfg = dataclasses.replace(mc.resolve(model), num_layers=2)
+    m = (NomicBertModel if model.startswith("nomic") else BertModel)(cfg, "cuda", seed=2)
+    g = torch.Generator().manual_seed(0)
+    docs = [torch.randint(0, 30000, (n,), generator=g, dtype=torch.int32)
+            for n in [1, 5, 16, 33] + [500] * 24]
+
+    def run(which):
+        lens = [len(docs[i]) for i in which]
+        cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+        return m.forward(torch.cat([docs[i] for i in which]).to(DEV), cu.to(DEV), lens)
+
+    whole = run(range(len(docs)))
+    small = run([3, 0, 2, 1])
+    from llm_mcp_amd.ops import encoder
+    keep, encoder.layers_ok = encoder.layers_ok, lambda *a: False
+    try:
+        loop = run(range(len(docs)))
+    finally:
+        encoder.layers_ok = keep
+    cos = torch.nn.functional.cosine_similarity
+    assert float(cos(whole[:4], torch.stack([small[1], small[3], small[2], small[0]])).min()) > 0.9995
+    assert float(cos(whole[4:5], run([4])).min()) > 0.9995
+    assert float(cos(whole, loop).min()) > 0.9995
