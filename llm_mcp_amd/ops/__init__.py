@@ -114,6 +114,13 @@ class Partials:
     def sum(self) -> torch.Tensor:
         return self.slabs.sum(0)
 
+    @classmethod
+    def empty(cls, a: torch.Tensor, S: int, N: int) -> "Partials":
+        """Slabs of a product of a's rows, memory of their own: two products may wait
+        for the same consumer (NormedPair)."""
+        M = a.shape[0]
+        return cls(torch.empty((S, M, N), dtype=torch.float32, device=a.device), S, M, N)
+
 
 def rms_norm(x, w: torch.Tensor, eps: float,
              residual: torch.Tensor | None = None,
@@ -1246,11 +1253,11 @@ def dgemm_partials(a: torch.Tensor, w: torch.Tensor, cfg: int, splits: int) -> P
     _chk(w.shape[1] == K and a.stride(1) == 1 and w.stride(1) == 1, "dgemm layout")
     _chk(a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0
          and w.data_ptr() % 16 == 0, "dgemm operands need 16-B aligned rows")
-    slabs, tickets = _dg_workspace(a.device, splits * M * N)
-    native().dgemm(0, _ptr(a), _ptr(w), _ptr(slabs), _ptr(tickets), _DG_TICKETS, M, N, K,
-                   a.stride(0), w.stride(0), N, cfg, splits, 2, _stream())
+    p = Partials.empty(a, splits, N)
+    native().dgemm(0, _ptr(a), _ptr(w), _ptr(p.slabs), 0, 0, M, N, K, a.stride(0), w.stride(0), N, cfg,
+                   splits, 2, _stream())
     DGEMM_CALLS[0] += 1
-    return Partials(slabs[:splits * M * N].view(splits, M, N), splits, M, N)
+    return p
 
 
 # ---------------------------------------------------------------------------
@@ -1572,10 +1579,10 @@ def rsgemm(a: torch.Tensor, w: torch.Tensor, cfg: int, splits: int, epi: int = 0
     _chk(w.shape[1] == K and rsgemm_operands_ok(a, w), "rsgemm operands need 16-B aligned rows")
     RSGEMM_CALLS[0] += 1
     if epi == 2:
-        slabs, cnt = _rs_workspace(a.device, splits * M * N)
-        native().rsgemm(0, _ptr(a), _ptr(w), _ptr(slabs), _ptr(cnt), _RS_CNT, M, N, K,
-                        a.stride(0), w.stride(0), N, cfg, splits, 2, _stream())
-        return Partials(slabs[:splits * M * N].view(splits, M, N), splits, M, N)
+        p = Partials.empty(a, splits, N)
+        native().rsgemm(0, _ptr(a), _ptr(w), _ptr(p.slabs), 0, 0, M, N, K, a.stride(0), w.stride(0), N,
+                        cfg, splits, 2, _stream())
+        return p
     ncols = N // 2 if epi == 3 else N
     if out is None:
         out = torch.empty((M, ncols), dtype=a.dtype, device=a.device)
@@ -1814,10 +1821,10 @@ def pgemm_sk(a: torch.Tensor, w: torch.Tensor, splits: int, act: int = 0, epi: i
     tiles = -(-M // 256) * (N // 256)
     PGEMM_CALLS[0] += 1
     if epi == 2:
-        slabs, cnt = _pg_workspace(a.device, splits * M * N)
-        native().pgemm_sk(0, _ptr(a), _ptr(w), _ptr(slabs), _ptr(cnt), _PG_CNT, M, N, K,
-                          a.stride(0), w.stride(0), N, 0, splits, 2, _stream())
-        return Partials(slabs[:splits * M * N].view(splits, M, N), splits, M, N)
+        p = Partials.empty(a, splits, N)
+        native().pgemm_sk(0, _ptr(a), _ptr(w), _ptr(p.slabs), 0, 0, M, N, K, a.stride(0), w.stride(0), N,
+                          0, splits, 2, _stream())
+        return p
     ncols = N // 2 if act == ACT_SWIGLU else N
     if out is None:
         out = torch.empty((M, ncols), dtype=a.dtype, device=a.device)

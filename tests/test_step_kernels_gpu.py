@@ -204,3 +204,16 @@ def test_encoder_batches_agree(model):
     assert float(cos(whole[:4], torch.stack([small[1], small[3], small[2], small[0]])).min()) > 0.9995
     assert float(cos(whole[4:5], run([4])).min()) > 0.9995
     assert float(cos(whole, loop).min()) > 0.9995
+
+
+# ----------------------------------------------------- products left to a norm --
+@pytest.mark.parametrize("N,K", [(4096, 4096), (4096, 14336)])
+def test_two_deferred_products_keep_their_slabs(N, K):
+    """Two products of one shape whose K reduction waits for the same norm: each has slabs
+    of its own."""
+    x, y = (torch.randn(4, K, device=DEV).bfloat16() for _ in range(2))
+    w = torch.randn(N, K, device=DEV).bfloat16() * K ** -0.5
+    a, b = ops.linear(x, w, defer=True), ops.linear(y, w, defer=True)
+    assert isinstance(a, ops.Partials) and isinstance(b, ops.Partials)
+    for p, r in ((a, x), (b, y)):
+        torch.testing.assert_close(p.sum().double(), r.double() @ w.double().t(), atol=1e-4, rtol=1e-4)
