@@ -13,20 +13,16 @@ constexpr float LOG2E = 1.4426950408889634f;
 // serial chain.  permlane16_swap(x, x) yields {rows 0,0,2,2 ; rows 1,1,3,3} of
 // x (16-lane rows), so op(first, second) is the xor-16 reduction; the 32-lane
 // form does the same across halves.
-// v_max_f32 as one instruction (fmaxf on values hipcc cannot prove canonical
-// -- MFMA results, lane swaps -- gets a canonicalising v_max per operand)
+// Maxima that propagate NaN: gfx950 has them as one instruction of up to three operands
+// (v_maximum3_f32), without the canonicalising v_max per operand that fmaxf gets on values
+// hipcc cannot prove canonical (MFMA results, lane swaps).  Not inline asm: what reads an
+// MFMA's result has to wait for it, and the compiler places those waits only before
+// instructions that it knows.
 __device__ __forceinline__ float max2f(float a, float b) {
-  float r;
-  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
+  return __builtin_elementwise_maximum(a, b);
 }
-
-// v_max3_f32 as one instruction (the same canonicalisation otherwise doubles
-// the row-max VALU of the softmax)
 __device__ __forceinline__ float max3f(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
 }
 
 __device__ __forceinline__ float col4_max(float x) {

@@ -67,11 +67,12 @@ __device__ __forceinline__ void split1(float x, uint16_t& hi, uint16_t& lo) {
   lo = f2bf(x - bf2f(hi));
 }
 
-// two values to packed bf16, one instruction
+// two values to packed bf16 (v_cvt_pk_bf16_f32; a builtin and not asm, so that a value an
+// MFMA has just made is waited for)
 __device__ __forceinline__ uint32_t cvt_pk(float a, float b) {
-  uint32_t r;
-  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf2));
 }
 __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
   hi = cvt_pk(a, b);
