@@ -130,6 +130,8 @@ int gemm_nt(void*, const void*, const void*, const void*, const void*, int, int,
             long, int, hipStream_t);
 int dgemm(void*, const void*, const void*, float*, unsigned*, int, int, int, int, long, long, long,
           int, int, int, hipStream_t, const void*);
+int sgemm(void*, const void*, const void*, int, int, int, long, long, long, int, int, const void*,
+          hipStream_t);
 int layernorm_slabs(void*, const float*, int, long, const void*, const void*, const void*, const void*,
                     int, int, float, hipStream_t);
 int embed_layernorm(void*, const int*, const void*, int, const void*, const void*, const int*,
@@ -575,6 +577,12 @@ PYBIND11_MODULE(_lmx_kernels, m) {
           "dgemm");
   }, py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(),
      py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg("bias") = 0);
+  m.def("sgemm", [](uptr C, uptr A, uptr W, int M, int N, int K, long lda, long ldw, long ldc, int epi,
+                    int splits, uptr bias, uptr stream) {
+    check(lmx::sgemm(P<void>(C), P<void>(A), P<void>(W), M, N, K, lda, ldw, ldc, epi, splits,
+                     P<void>(bias), S(stream)),
+          "sgemm");
+  });
   m.def("layernorm_slabs", [](uptr out, uptr slabs, int nsl, long stride, uptr bias, uptr residual,
                               uptr w, uptr b, int rows, int cols, float eps, uptr stream) {
     check(lmx::layernorm_slabs(P<void>(out), P<float>(slabs), nsl, stride, P<void>(bias),

@@ -28,7 +28,8 @@ struct EncArgs {
   int ntiles, q_per_tile;
 };
 
-struct EncPlan { int cfg, splits; };   // cfg -1: K13
+struct EncPlan { int cfg, splits; };   // cfg: dgemm's, -1: K13, kEncSmall: K23
+constexpr int kEncSmall = 100;
 
 EncPlan enc_plan(int M, int N, int K, int act, bool partials);
 long enc_slab_floats(int T, int d, int I);

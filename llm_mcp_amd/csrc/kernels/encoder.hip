@@ -33,6 +33,8 @@ int dgemm(void*, const void*, const void*, float*, unsigned*, int, int, int, int
           int, int, int, hipStream_t, const void*);
 int pgemm(void*, const void*, const void*, const void*, int, int, int, long, long, long, int, int, int,
           int, float*, hipStream_t);
+int sgemm(void*, const void*, const void*, int, int, int, long, long, long, int, int, const void*,
+          hipStream_t);
 
 namespace {
 
@@ -66,6 +68,10 @@ float k13_us(int M, int N, int K) {
 // product's fp32 slabs go to a LayerNorm (no activation).
 EncPlan enc_plan(int M, int N, int K, int act, bool partials) {
   EncPlan best{-1, 0};
+  // few rows: K23, except where K slices of the 64 x 64 tile fill the chip (at 16 rows:
+  // qkv of nomic 4.5 us against 5.7, gate / up 5.8 against 7.3, but o 3.5 against 3.0 and down 4.6
+  // against 4.0; qkv at 32 rows 5.5 against 5.9, at 64 7.5 against 6.1)
+  if (!partials && M <= 32 && N % 32 == 0 && K % 32 == 0) return {kEncSmall, 1};
   const bool k13 = N % 256 == 0 && K % 64 == 0 && K >= 192;
   float t = k13 ? k13_us(M, N, K) : 1e30f;
   for (const EncTile& c : kTiles) {
@@ -106,6 +112,8 @@ int encoder_layers(const EncArgs& a, const uintptr_t* w, hipStream_t stream) {
     if (p.cfg < 0)
       return pgemm(out, x, (void*)W, (void*)b, T, N, K, K, K, ldc, act, 0, 0, 0, nullptr, stream);
     const int epi = act == 3 ? 3 : act == 4 ? 6 : b ? 5 : 0;
+    if (p.cfg == kEncSmall)
+      return sgemm(out, x, (void*)W, T, N, K, K, K, ldc, epi, 1, (void*)b, stream);
     return dgemm(out, x, (void*)W, nullptr, nullptr, 0, T, N, K, K, K, ldc, p.cfg, 1, epi, stream,
                  (void*)b);
   };

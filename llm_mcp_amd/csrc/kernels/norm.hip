@@ -194,7 +194,9 @@ __global__ void __launch_bounds__(256) layernorm_kernel(
 }
 
 // LayerNorm of a projection whose K reduction is left to it: out = LN(sum of S
-// fp32 slabs + bias + residual), the sum in slab order and unrounded. One row per
+// fp32 slabs + bias + residual), the slabs summed in order. Rounded to bf16 where the
+// separate passes round, the product and its sum with the residual, so that a row's
+// result does not depend on the kernel that the batch's size picks. One row per
 // workgroup as above: memory bound for many rows; for few, the S loads of a chunk
 // are in flight together, so the reduction costs no pass of its own (a 16-row
 // encoder step: 4.0 us with 12 slabs, as the plain LayerNorm).
@@ -230,7 +232,7 @@ __global__ void __launch_bounds__(256) layernorm_slabs_kernel(
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      v[j] = (j < 4 ? p0[0][j & 3] : p1[0][j & 3]) + pb[j] + r[j];
+      v[j] = bf2f(f2bf(bf2f(f2bf((j < 4 ? p0[0][j & 3] : p1[0][j & 3]) + pb[j])) + r[j]));
       s += v[j];
     }
   }
@@ -247,8 +249,9 @@ __global__ void __launch_bounds__(256) layernorm_slabs_kernel(
   }
 }
 
-// The encoders' input: LN(word[id] + type + pos[position]) of every token, summed in
-// fp32 (ids outside the table count as a zero row). pos: null without absolute positions.
+// The encoders' input: LN(word[id] + (pos[position] + type)) of every token, both sums
+// rounded to bf16 (ids outside the table count as a zero row). pos: null without absolute
+// positions.
 __global__ void __launch_bounds__(256) embed_layernorm_kernel(
     bf16_t* __restrict__ out, const int* __restrict__ ids, const bf16_t* __restrict__ word, int vocab,
     const bf16_t* __restrict__ type, const bf16_t* __restrict__ pos,
@@ -264,12 +267,12 @@ __global__ void __launch_bounds__(256) embed_layernorm_kernel(
     if (pos) {
       ldv<8>(t, pos + (long)positions[row] * cols + c);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] += t[j];
+      for (int j = 0; j < 8; ++j) v[j] = bf2f(f2bf(v[j] + t[j]));
     }
     if (id >= 0 && id < vocab) {
       ldv<8>(t, word + (long)id * cols + c);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] += t[j];
+      for (int j = 0; j < 8; ++j) v[j] = bf2f(f2bf(v[j] + t[j]));
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) s += v[j];

@@ -794,9 +794,58 @@ def _into(out: torch.Tensor | None, y: torch.Tensor) -> torch.Tensor:
     return out.copy_(y)
 
 
+# K23 (csrc/kernels/sgemm.hip), few rows and small weights: elements of W up to which it
+# beats the tables' kernels on cold weights. Llama-3.2-1B at 1 / 16 / 32 rows: QKV (6.3 M) 5.4 / 6.7 /
+# 8.7 us against 11.2 / 11.4 / 11.6, O (4.2 M) 4.1 / 4.7 / 5.7 against 7.1 / 7.3 / 7.0, and at 64
+# rows 13.0 against 12.4; Llama-3-8B O (16.8 M) 9.1 at 1 row and 10.6 at 8 against 10.9 and 11.3,
+# 12.8 at 16 against 11.6
+SGEMM_MAX_M, SGEMM_MAX_W = 32, 6_600_000
+SGEMM_MAX_M_WIDE, SGEMM_MAX_W_WIDE = 8, 17_000_000
+SGEMM_CALLS = [0]          # host-side launch count (tests: the K23 path really ran)
+
+
+def sgemm_splits(M: int, N: int, K: int, epi: int = 0) -> int | None:
+    """K slices of this product on K23 (1 except for epi 2, fp32 slabs), or None: not
+    its range.  The larger weights only as slabs (a plain one of them is K11's)."""
+    if N % 32 or K % 32 or M < 1:
+        return None
+    if not (M <= SGEMM_MAX_M and N * K <= SGEMM_MAX_W) and not (
+            epi == 2 and M <= SGEMM_MAX_M_WIDE and N * K <= SGEMM_MAX_W_WIDE):
+        return None
+    if epi != 2:
+        return 1
+    # a workgroup per CU, 4 slices at most (each is read again by the norm)
+    return next(s for s in (4, 2, 1) if s == 1 or (N // 16 * s <= 256 and K // 32 % s == 0))
+
+
+def sgemm(a: torch.Tensor, w: torch.Tensor, epi: int = 0, splits: int = 1,
+          bias: torch.Tensor | None = None, out: torch.Tensor | None = None):
+    """a @ w^T on K23 (1 to 64 rows).  epi 0 plain, 5 with ``bias``, 3 / 4 SwiGLU / ReLU-GLU over
+    16-row pairs ([M, N / 2]), 2 fp32 ``Partials`` [splits, M, N]."""
+    M, K = a.shape
+    N = w.shape[0]
+    _bf16(a, "a"); _bf16(w, "w")
+    _chk(0 < M <= 64 and N % 32 == 0 and K % 32 == 0 and K // 32 % splits == 0
+         and (splits == 1 or epi == 2), f"sgemm shape M={M} N={N} K={K} S={splits}")
+    _chk(w.shape[1] == K and pgemm_operands_ok(a, w), "sgemm operands need 16-B aligned rows")
+    SGEMM_CALLS[0] += 1
+    if epi == 2:
+        p = Partials.empty(a, splits, N)
+        native().sgemm(_ptr(p.slabs), _ptr(a), _ptr(w), M, N, K, a.stride(0), w.stride(0), N, 2, splits,
+                       0, _stream())
+        return p
+    if out is None:
+        out = torch.empty((M, N // 2 if epi in (3, 4) else N), dtype=a.dtype, device=a.device)
+    _chk(out.shape == (M, N // 2 if epi in (3, 4) else N) and out.stride(1) == 1
+         and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0, "sgemm output layout")
+    native().sgemm(_ptr(out), _ptr(a), _ptr(w), M, N, K, a.stride(0), w.stride(0), out.stride(0),
+                   epi if bias is None else 5, 1, _ptr(bias), _stream())
+    return out
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, defer: bool = False,
            bias: torch.Tensor | None = None, out: torch.Tensor | None = None):
-    """x @ w^T (+ bias): the decode GEMM (K11) where the measured table picks
+    """x @ w^T (+ bias): K23 for few rows of small weights, the decode GEMM (K11) where the measured table picks
     it, the older split-K kernel where it was measured faster, the large-M
     GEMM (K13) for prefill-sized M where ``large_gemm_backend`` picks it, else
     hipBLASLt (bias in its epilogue).  ``defer``: the caller feeds the result to
@@ -814,6 +863,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, defer: bool = False,
         return _packed_product(x, w, 2 if defer and x.shape[0] <= 256 else 0, out=out)
     if x.is_cuda and x.dim() == 2:
         M, N, K = x.shape[0], w.shape[0], w.shape[1]
+        s = sgemm_splits(M, N, K, 2 if defer and bias is None else 0)
+        if s is not None and pgemm_operands_ok(x, w) and pgemm_bias_ok(bias, N):
+            return sgemm(x, w, 2 if defer and bias is None else 0, s, bias, out)
         if bias is None:
             rc = rs_choice(M, N, K, epi=2 if defer else 0, w=w)
             if rc is not None and rsgemm_operands_ok(x, w):
@@ -861,6 +913,9 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, block: int,
         return _packed_product(x, w, 3, out=out)
     if x.is_cuda and x.dim() == 2:
         if block == SWIGLU16:
+            if (sgemm_splits(x.shape[0], w.shape[0], w.shape[1], 3) is not None
+                    and pgemm_operands_ok(x, w)):
+                return sgemm(x, w, 3, out=out)
             rc = rs_choice(x.shape[0], w.shape[0], w.shape[1], epi=3, w=w)
             if rc is not None and rsgemm_operands_ok(x, w):
                 return rsgemm(x, w, rc[0], rc[1], epi=3, out=out)     # K14, SwiGLU epilogue
@@ -888,6 +943,8 @@ def linear_relu_glu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     else the product and the GLU kernel."""
     if x.is_cuda and x.dtype == torch.bfloat16:
         M, N, K = x.shape[0], w.shape[0], w.shape[1]
+        if x.dim() == 2 and sgemm_splits(M, N, K, 4) is not None and pgemm_operands_ok(x, w):
+            return sgemm(x, w, 4)
         ch = dgemm_choice(M, N, K, epi=3)
         if ch is not None and ch[0] >= 0 and swiglu16_ok(ch[0]):
             return dgemm(x, w, ch[0], ch[1], epi=4)
