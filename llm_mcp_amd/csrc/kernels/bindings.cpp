@@ -144,8 +144,9 @@ int rmsnorm_slabs(void*, void*, const float*, int, long, const void*, int, int, 
                   hipStream_t);
 int dgemm_config(int, int*, int*);
 int dgemm_sk_pieces(int, int, int, int, int);
-int pgemm(void*, const void*, const void*, const void*, int, int, int, long, long, long, int, int,
-          int, int, float*, hipStream_t);
+int pgemm(void*, const void*, const void*, const void*, int, int, int, long, long, long, int, int, int,
+          int, float*, hipStream_t, float*, unsigned*);
+long pgemm_tail_floats(int, int, int);
 int row_scale(float*, const float*, int, const void*, long, int, int, float, hipStream_t);
 int pgemm_sk(void*, const void*, const void*, void*, void*, int, int, int, int, long, long, long,
              int, int, int, hipStream_t);
@@ -602,17 +603,20 @@ PYBIND11_MODULE(_lmx_kernels, m) {
     return std::make_pair(p.cfg, p.splits);
   });
   m.def("enc_slab_floats", &lmx::enc_slab_floats);
+  m.def("enc_tail_floats", &lmx::enc_tail_floats);
   m.def("encoder_layers", [](const std::vector<uintptr_t>& w, int T, int d, int I, int H, int D, int page,
                              bool gelu, float eps, float scale, uptr x, uptr h, uptr qkv, uptr attn,
                              uptr g, uptr slabs, long slab_floats, uptr kc, uptr vc, uptr slots,
                              uptr positions, uptr cos_sin, uptr bt, int bt_stride, uptr cu, uptr ctx,
-                             uptr tiles, int ntiles, int q_per_tile, uptr stream) {
+                             uptr tiles, int ntiles, int q_per_tile, uptr tail, long tail_floats,
+                             uptr cnt, uptr stream) {
     if (w.size() % lmx::kEncPtrs) throw std::runtime_error("encoder_layers: weights");
     const lmx::EncArgs a{(int)(w.size() / lmx::kEncPtrs), T, d, I, H, D, page, gelu, eps, scale,
                          P<void>(x), P<void>(h), P<void>(qkv), P<void>(attn), P<void>(g),
                          P<float>(slabs), slab_floats, P<void>(kc), P<void>(vc), P<int>(slots),
                          P<int>(positions), P<float>(cos_sin), P<int>(bt), bt_stride, P<int>(cu),
-                         P<int>(ctx), P<int>(tiles), ntiles, q_per_tile};
+                         P<int>(ctx), P<int>(tiles), ntiles, q_per_tile, P<float>(tail), tail_floats,
+                         P<unsigned>(cnt)};
     check(lmx::encoder_layers(a, w.data(), S(stream)), "encoder_layers");
   });
   m.def("rmsnorm_slabs", [](uptr out, uptr residual, uptr slabs, int nsl, long slab_stride,
@@ -646,11 +650,16 @@ PYBIND11_MODULE(_lmx_kernels, m) {
   });
   // ---- K13 large-M GEMM (pgemm.hip) ----
   m.def("pgemm", [](uptr C, uptr A, uptr W, uptr bias, int M, int N, int K, long lda, long ldw,
-                    long ldc, int act, int grid, int res, int wpacked, uptr nrm, uptr stream) {
+                    long ldc, int act, int grid, int res, int wpacked, uptr nrm, uptr stream,
+                    uptr slabs, uptr cnt) {
     check(lmx::pgemm(P<void>(C), P<void>(A), P<void>(W), P<void>(bias), M, N, K, lda, ldw, ldc,
-                     act, grid, res, wpacked, P<float>(nrm), S(stream)),
+                     act, grid, res, wpacked, P<float>(nrm), S(stream), P<float>(slabs),
+                     P<unsigned>(cnt)),
           "pgemm");
-  });
+  }, py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(),
+     py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg("slabs") = 0,
+     py::arg("cnt") = 0);
+  m.def("pgemm_tail_floats", &lmx::pgemm_tail_floats);
   m.def("row_scale", [](uptr s, uptr part, int np, uptr x, long x_stride, int M, int cols,
                         float eps, uptr stream) {
     check(lmx::row_scale(P<float>(s), P<float>(part), np, P<void>(x), x_stride, M, cols, eps,

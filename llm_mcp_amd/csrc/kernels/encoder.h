@@ -26,6 +26,9 @@ struct EncArgs {
   int bt_stride;
   const int *cu, *ctx, *tiles;
   int ntiles, q_per_tile;
+  float* tail;                     // K13's last round in pieces (pgemm): floats and counters
+  long tail_floats;
+  unsigned* cnt;
 };
 
 struct EncPlan { int cfg, splits; };   // cfg: dgemm's, -1: K13, kEncSmall: K23
@@ -33,6 +36,7 @@ constexpr int kEncSmall = 100;
 
 EncPlan enc_plan(int M, int N, int K, int act, bool partials);
 long enc_slab_floats(int T, int d, int I);
+long enc_tail_floats(int T, int d, int I, bool gelu);
 int encoder_layers(const EncArgs& a, const uintptr_t* w, hipStream_t stream);
 
 }  // namespace lmx

@@ -32,7 +32,9 @@ int paged_prefill(const void*, long, const void*, const void*, const int*, int, 
 int dgemm(void*, const void*, const void*, float*, unsigned*, int, int, int, int, long, long, long,
           int, int, int, hipStream_t, const void*);
 int pgemm(void*, const void*, const void*, const void*, int, int, int, long, long, long, int, int, int,
-          int, float*, hipStream_t);
+          int, float*, hipStream_t, float*, unsigned*);
+long pgemm_tail_floats(int, int, int);
+float pgemm_us(int, int, int);
 int sgemm(void*, const void*, const void*, int, int, int, long, long, long, int, int, const void*,
           hipStream_t);
 
@@ -53,15 +55,6 @@ constexpr EncTile kTiles[] = {
 constexpr int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16};      // layernorm_slabs' S
 constexpr float kBytesUs = 4.5e6f;                         // memory traffic, bytes per us
 
-// K13: a 256 x 256 tile takes 5 us + 0.92 (few workgroups) to 1.27 us (a full chip)
-// per 64-deep K-step (measured 16 / 22 us at K 768, 48 / 55 at 3072, 63 / 82 at 4096)
-float k13_us(int M, int N, int K) {
-  const long tiles = (long)((M + 255) / 256) * (N / 256);
-  const long rounds = (tiles + 255) / 256;
-  const float fill = (float)tiles / (256.f * rounds);
-  return rounds * (5.f + K / 64 * (0.92f + 0.35f * fill));
-}
-
 }  // namespace
 
 // act: 0 none, 3 SwiGLU over 16-row pairs, 4 gelu (exact). partials: the
@@ -73,7 +66,7 @@ EncPlan enc_plan(int M, int N, int K, int act, bool partials) {
   // against 4.0; qkv at 32 rows 5.5 against 5.9, at 64 7.5 against 6.1)
   if (!partials && M <= 32 && N % 32 == 0 && K % 32 == 0) return {kEncSmall, 1};
   const bool k13 = N % 256 == 0 && K % 64 == 0 && K >= 192;
-  float t = k13 ? k13_us(M, N, K) : 1e30f;
+  float t = k13 ? pgemm_us(M, N, K) : 1e30f;
   for (const EncTile& c : kTiles) {
     const int bk = c.cfg == 11 ? 64 : 128;
     if (N % c.bn || (act == 3 && c.cfg == 21)) continue;   // a wave holds whole 16-row pairs
@@ -100,17 +93,36 @@ long enc_slab_floats(int T, int d, int I) {
   return (long)std::max(o.splits, m.splits) * T * d;
 }
 
+// floats that K13 takes for the last rounds of the products it runs
+long enc_tail_floats(int T, int d, int I, bool gelu) {
+  long n = 0;
+  auto add = [&](int N, int K, int act, bool partials) {
+    if (enc_plan(T, N, K, act, partials).cfg < 0) n = std::max(n, pgemm_tail_floats(T, N, K));
+  };
+  add(3 * d, d, 0, false);
+  add(d, d, 0, true);
+  add(gelu ? I : 2 * I, d, gelu ? 4 : 3, false);
+  add(d, I, 0, true);
+  return n;
+}
+
 int encoder_layers(const EncArgs& a, const uintptr_t* w, hipStream_t stream) {
   const int T = a.T, d = a.d, I = a.I;
   if (T <= 0) return 0;
   if (d != a.H * a.D || d % 256 || I % 256 || (a.D != 64 && a.D != 128)) return -1;
   for (int i = 0; i < a.layers * kEncPtrs; ++i)
     if (w[i] & 15) return -2;
+  auto k13 = [&](void* out, const void* x, uintptr_t W, uintptr_t b, int N, int K, int ldc, int act) {
+    const long n = pgemm_tail_floats(T, N, K);
+    float* tail = n > 0 && n <= a.tail_floats ? a.tail : nullptr;
+    return pgemm(out, x, (void*)W, (void*)b, T, N, K, K, K, ldc, act, 0, 0, 0, nullptr, stream, tail,
+                 a.cnt);
+  };
   auto full = [&](void* out, const void* x, uintptr_t W, uintptr_t b, int N, int K, int act) {
     const EncPlan p = enc_plan(T, N, K, act, false);
     const int ldc = act == 3 ? N / 2 : N;
     if (p.cfg < 0)
-      return pgemm(out, x, (void*)W, (void*)b, T, N, K, K, K, ldc, act, 0, 0, 0, nullptr, stream);
+      return k13(out, x, W, b, N, K, ldc, act);
     const int epi = act == 3 ? 3 : act == 4 ? 6 : b ? 5 : 0;
     if (p.cfg == kEncSmall)
       return sgemm(out, x, (void*)W, T, N, K, K, K, ldc, epi, 1, (void*)b, stream);
@@ -122,7 +134,7 @@ int encoder_layers(const EncArgs& a, const uintptr_t* w, hipStream_t stream) {
                     uintptr_t g, uintptr_t s, int K, void* tmp) {
     const EncPlan p = enc_plan(T, d, K, 0, true);
     if (p.cfg < 0) {
-      const int e = pgemm(tmp, x, (void*)W, (void*)b, T, d, K, K, K, d, 0, 0, 0, 0, nullptr, stream);
+      const int e = k13(tmp, x, W, b, d, K, d, 0);
       return e ? e : layernorm(out, tmp, residual, (void*)g, (void*)s, T, d, a.eps, stream);
     }
     if ((long)p.splits * T * d > a.slab_floats) return -3;

@@ -58,6 +58,9 @@
 // any) N <= 8192.
 #include "common.h"
 
+#include <algorithm>
+#include <cmath>
+
 namespace lmx {
 namespace {
 
@@ -132,6 +135,15 @@ struct PgGroups {
   const float* limit;            // ACT 6: clamp per group
   float slope, shift;            // ACT 6: g sigmoid(slope g) (u + shift)
   int mtiles;
+};
+
+// the last, partly filled round in pieces (see pg_tail_share): `share` workgroups, of different
+// XCDs, share the K-steps of some tiles; fp32 tiles of pieces, arrival and publication
+// counters per tile
+struct PgTail {
+  int share;
+  float* slabs;
+  unsigned* cnt;
 };
 
 // thread constants
@@ -453,18 +465,87 @@ __device__ __forceinline__ void pp_step(PpRegs& R, char* smem, int stage, const 
   pp_phase<1, MODE, ACT, BIAS, SCHED, WP, NRM>(R, smem, stage, L1, L2, O, T, N);
 }
 
+constexpr int PG_TSLAB = PG_THREADS * 128;        // floats of a piece's tile
+constexpr int PG_TAIL_SLOTS = 16;                 // pieces of the tiles that 8 workgroups share
+
+// Joins the fp32 tiles of np pieces (slabs one after the other, in K order; this
+// workgroup has piece p): all but the last to arrive publish theirs write-through
+// (sc1) in the lane-native order -- accumulator r = ((qm * 2 + qn) * 4 + i) * 2 + j of
+// every lane is float4 r * PG_THREADS + tid -- and leave (false); the last adds them in
+// piece order, so the sum does not depend on who that is, and re-arms the counters
+// [arrivals, publications].  It waits only for pieces that have arrived, whose
+// workgroups are publishing.
+__device__ __forceinline__ bool pg_join(PpRegs& R, char* smem, float* slabs, unsigned* cnt, int p,
+                                        int np) {
+  typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+  unsigned* word = reinterpret_cast<unsigned*>(smem);
+  __syncthreads();                                 // every wave's DMA has landed
+  if (threadIdx.x == 0)
+    word[0] = __hip_atomic_fetch_add(&cnt[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const unsigned order = word[0];
+  const int voff = threadIdx.x * 16;               // float4 r: + 8 KB r, a scalar offset
+  const auto rs = __builtin_amdgcn_make_buffer_rsrc(slabs, (short)0, np * PG_TSLAB * 4, 0x00020000);
+  auto acc = [&](int r) -> f32x4_t& { return R.acc[r >> 4][(r >> 3) & 1][(r >> 1) & 3][r & 1]; };
+  if (order + 1 < (unsigned)np) {
+    // no L2 write-back fence
+#pragma unroll
+    for (int r = 0; r < 32; ++r)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc(r)), rs, voff,
+                                             p * PG_TSLAB * 4 + r * 8192, 16);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+      __hip_atomic_fetch_add(&cnt[1], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return false;
+  }
+  if (threadIdx.x == 0) {
+    while (__hip_atomic_load(&cnt[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < (unsigned)(np - 1))
+      __builtin_amdgcn_s_sleep(2);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __hip_atomic_store(&cnt[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&cnt[1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  // ((p0 + p1) + ...) + p(np - 1), its own at its place; 8 loads of a lane in flight
+  auto in = [&](int s, int r) {
+    return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                           rs, voff, s * PG_TSLAB * 4 + r * 8192, 0));
+  };
+  constexpr int B = 8;
+#pragma unroll
+  for (int h = 0; h < 32; h += B) {
+    f32x4_t v[B];
+    if (p > 0) {
+#pragma unroll
+      for (int r = 0; r < B; ++r) v[r] = in(0, h + r);
+      for (int s = 1; s < p; ++s)
+#pragma unroll
+        for (int r = 0; r < B; ++r) v[r] += in(s, h + r);
+#pragma unroll
+      for (int r = 0; r < B; ++r) acc(h + r) = v[r] + acc(h + r);
+    }
+    for (int s = p + 1; s < np; ++s)
+#pragma unroll
+      for (int r = 0; r < B; ++r) acc(h + r) += in(s, h + r);
+  }
+  return true;
+}
+
 }  // namespace
 
 template <int ACT, int BIAS, int SCHED, int WP = 0, int NRM = 0>
 __global__ void __launch_bounds__(PG_THREADS, 1) pgemm_pp2_kernel(
     bf16_t* __restrict__ C, const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ bias, int M, int N, int K, int lda, int ldw, int ldc,
-    float* __restrict__ nrm, PgGroups grp) {
+    float* __restrict__ nrm, PgGroups grp, PgTail tail) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tiles_m = WP == 2 ? grp.tiles[2 * grp.mtiles] : (M + 255) / 256, tiles_n = N / 256, ntiles = tiles_m * tiles_n;
   const int G = gridDim.x;
   const int r = xcd_remap(blockIdx.x, G);
-  const int my_tiles = (ntiles - r + G - 1) / G;
+  const bool cut = WP != 2 && tail.share > 0;    // the last round's tiles in pieces
+  const int my_tiles = cut ? ntiles / G : (ntiles - r + G - 1) / G;
   const int nk = K / 64;
   if (WP == 2 && my_tiles <= 0) return;      // fewer used tiles than workgroups
 
@@ -516,9 +597,9 @@ __global__ void __launch_bounds__(PG_THREADS, 1) pgemm_pp2_kernel(
     __syncthreads();
   }
 
-  auto set_tile = [&](PgLoad& L, int t) {
+  auto set_tile = [&](PgLoad& L, int lin) {
     int tm, tn;
-    pg_tile_coords(t * G + r, tiles_m, tiles_n, tm, tn);
+    pg_tile_coords(lin, tiles_m, tiles_n, tm, tn);
     if constexpr (WP == 2) {
       const int g = grp.tiles[2 * tm], m0 = grp.tiles[2 * tm + 1], m1 = grp.off[g + 1];
       const int sc = (lane & 7) ^ ((4 * T.wave + (lane >> 4)) & 7);
@@ -543,9 +624,9 @@ __global__ void __launch_bounds__(PG_THREADS, 1) pgemm_pp2_kernel(
     L.rw = __builtin_amdgcn_make_buffer_rsrc((void*)(W + (long)n0 * ldw), (short)0,
                                              (int)(256L * ldw * 2), 0x00020000);
   };
-  auto set_out = [&](PgOut& O, int t) {
+  auto set_out = [&](PgOut& O, int lin) {
     int tm, tn;
-    pg_tile_coords(t * G + r, tiles_m, tiles_n, tm, tn);
+    pg_tile_coords(lin, tiles_m, tiles_n, tm, tn);
     int m0 = tm * 256, m1 = M;
     if constexpr (WP == 2) {
       const int g = grp.tiles[2 * tm];
@@ -565,88 +646,129 @@ __global__ void __launch_bounds__(PG_THREADS, 1) pgemm_pp2_kernel(
                                                (M - m0) * (N / 64) * 4, 0x00020000);
     O.n0 = tn * 256;
   };
+  // A run: `count` tiles lin, lin + G, .., K-steps [kb, ke) of each, as one load stream. The
+  // workgroup's whole tiles are one run; a piece of a tile of the last round is another
+  // (count 1), each behind a drained pipeline.
+  int lin = r, count = my_tiles, kb = 0, ke = nk;
+  // The last round: the workgroups slot, row + slot, .. (one of each XCD j) take the tiles
+  // slot, row + slot, .. of it, the K-steps of those tiles one after the other cut into equal parts.
+  // The workgroups of an XCD are then at the same K of neighbouring tiles, as in
+  // the other rounds, and share their panels in its L2 (parts in tile order, which start at
+  // as many K as there are workgroups, ran slower than whole tiles).
+  const int row = G >> 3, j = r / row, slot = r - j * row;
+  const int first = ntiles / G * G, most = cut ? (ntiles - first + row - 1) / row : 0;
+  const int steps = most * nk, P = tail.share;
+  int s = j < P ? j * steps / P : 0;
+  const int e = j < P ? (j + 1) * steps / P : 0;
   auto advance = [&](PgLoad& L) {
     if (L.done) return;
-    if (++L.k == nk) {
-      if (L.tile + 1 >= my_tiles) {
+    if (++L.k == ke) {
+      if (L.tile + 1 >= count) {
         L.done = true;
-        L.k = nk - 1;
+        L.k = ke - 1;
         return;
       }
       L.k = 0;
       ++L.tile;
-      set_tile(L, L.tile);
+      set_tile(L, lin + L.tile * G);
     }
     L.kbyte = L.k * 128;
   };
 
   PpRegs R;
   PgLoad L1, L2;                    // K-steps s+1 and s+2 of the running K-step s
-  L2.k = 0;
-  L2.tile = 0;
-  L2.kbyte = 0;
-  L2.done = false;
-  set_tile(L2, 0);
   PgOut O;
-  set_out(O, 0);
+  for (bool piece = false;; piece = true) {
+    if (piece || count == 0) {
+      const int t = cut ? s / nk : 0;
+      lin = first + t * row + slot;
+      if (s >= e || lin >= ntiles) return;
+      piece = true;
+      count = 1;
+      kb = s - t * nk;
+      ke = min(nk, kb + e - s);
+      // no load or store of the run before is counted by the waits that follow
+      pg_vmwait<0>();
+      pg_barrier();
+    }
+    L2.k = kb;
+    L2.tile = 0;
+    L2.kbyte = kb * 128;
+    L2.done = false;
+    set_tile(L2, lin);
+    set_out(O, lin);
 
-  // ---- prologue: the DMA of the phases before K-step 0, in loop order
-  if constexpr (SCHED == 0) {
-    pg_issue<HA0, WP>(smem, 0, L2, T);
-    pg_issue<HW0, WP>(smem, 0, L2, T);
-    pg_issue<HW1, WP>(smem, 0, L2, T);
-    pg_issue<HA1, WP>(smem, 0, L2, T);
-    advance(L2);
-    pg_issue<HA0, WP>(smem, 1, L2, T);
-    pg_issue<HW0, WP>(smem, 1, L2, T);
-    pg_issue<HW1, WP>(smem, 1, L2, T);
-    L1 = L2;
-    advance(L2);
-    pg_vmwait<8>();                 // A0, W0, W1 of K-step 0
-  } else {
-    pg_issue<HA0, WP>(smem, 0, L2, T);
-    pg_issue<HW0, WP>(smem, 0, L2, T);
-    pg_issue<HA1, WP>(smem, 0, L2, T);
-    pg_issue<HW1, WP>(smem, 0, L2, T);
-    advance(L2);
-    pg_issue<HA0, WP>(smem, 1, L2, T);
-    pg_issue<HW0, WP>(smem, 1, L2, T);
-    L1 = L2;
-    advance(L2);
-    pg_vmwait<4>();                 // A0, W0, W1 of K-step 0
-  }
-  pg_barrier();
-  if (T.wm == 1) pg_barrier();      // waves 4-7 run one barrier behind
-
-  int stage = 0;
-  auto next = [&]() {
-    L1 = L2;
-    advance(L2);
-    stage ^= 1;
-  };
-  for (int t = 0; t < my_tiles; ++t) {
-    if (t == 0) {
-      pp_step<MODE_FIRST, ACT, BIAS, SCHED, WP, NRM>(R, smem, stage, L1, L2, O, T, N);
-      next();
-      pp_step<MODE_PLAIN, ACT, BIAS, SCHED, WP, NRM>(R, smem, stage, L1, L2, O, T, N);
+    // ---- prologue: the DMA of the phases before K-step 0, in loop order
+    if constexpr (SCHED == 0) {
+      pg_issue<HA0, WP>(smem, 0, L2, T);
+      pg_issue<HW0, WP>(smem, 0, L2, T);
+      pg_issue<HW1, WP>(smem, 0, L2, T);
+      pg_issue<HA1, WP>(smem, 0, L2, T);
+      advance(L2);
+      pg_issue<HA0, WP>(smem, 1, L2, T);
+      pg_issue<HW0, WP>(smem, 1, L2, T);
+      pg_issue<HW1, WP>(smem, 1, L2, T);
+      L1 = L2;
+      advance(L2);
+      pg_vmwait<8>();                 // A0, W0, W1 of K-step 0
     } else {
-      pp_step<MODE_K0, ACT, BIAS, SCHED, WP, NRM>(R, smem, stage, L1, L2, O, T, N);   // stores tile t-1
-      next();
-      set_out(O, t);
-      pp_step<MODE_K1, ACT, BIAS, SCHED, WP, NRM>(R, smem, stage, L1, L2, O, T, N);
+      pg_issue<HA0, WP>(smem, 0, L2, T);
+      pg_issue<HW0, WP>(smem, 0, L2, T);
+      pg_issue<HA1, WP>(smem, 0, L2, T);
+      pg_issue<HW1, WP>(smem, 0, L2, T);
+      advance(L2);
+      pg_issue<HA0, WP>(smem, 1, L2, T);
+      pg_issue<HW0, WP>(smem, 1, L2, T);
+      L1 = L2;
+      advance(L2);
+      pg_vmwait<4>();                 // A0, W0, W1 of K-step 0
     }
-    next();
-    for (int k = 2; k < nk; ++k) {
-      pp_step<MODE_PLAIN, ACT, BIAS, SCHED, WP, NRM>(R, smem, stage, L1, L2, O, T, N);
+    pg_barrier();
+    if (T.wm == 1) pg_barrier();      // waves 4-7 run one barrier behind
+
+    int stage = 0;
+    auto next = [&]() {
+      L1 = L2;
+      advance(L2);
+      stage ^= 1;
+    };
+    for (int t = 0; t < count; ++t) {
+      if (t == 0) {
+        pp_step<MODE_FIRST, ACT, BIAS, SCHED, WP, NRM>(R, smem, stage, L1, L2, O, T, N);
+        next();
+        if (WP == 2 || ke - kb > 1)   // a piece may be one K-step
+          pp_step<MODE_PLAIN, ACT, BIAS, SCHED, WP, NRM>(R, smem, stage, L1, L2, O, T, N);
+      } else {
+        pp_step<MODE_K0, ACT, BIAS, SCHED, WP, NRM>(R, smem, stage, L1, L2, O, T, N);   // stores tile t-1
+        next();
+        set_out(O, lin + t * G);
+        pp_step<MODE_K1, ACT, BIAS, SCHED, WP, NRM>(R, smem, stage, L1, L2, O, T, N);
+      }
       next();
+      for (int k = kb + 2; k < ke; ++k) {
+        pp_step<MODE_PLAIN, ACT, BIAS, SCHED, WP, NRM>(R, smem, stage, L1, L2, O, T, N);
+        next();
+      }
     }
+    if (T.wm == 0) pg_barrier();
+    pg_vmwait<0>();
+    if constexpr (WP != 2) {
+      if (piece) {
+        s += ke - kb;
+        // the tile's pieces: XCDs j0 .. j1 in K order
+        const int t = (lin - first) / row;
+        const int j0 = ((t * nk + 1) * P - 1) / steps, j1 = ((t + 1) * nk * P - 1) / steps;
+        if (j1 > j0 && !pg_join(R, smem, tail.slabs + (long)(slot * PG_TAIL_SLOTS + j0 + t) * PG_TSLAB,
+                                tail.cnt + 2 * (lin - first), j - j0, j1 - j0 + 1))
+          continue;
+      }
+    }
+    pg_store<0, 0, ACT, BIAS, NRM>(R, O, T, smem, N);
+    pg_store<0, 1, ACT, BIAS, NRM>(R, O, T, smem, N);
+    pg_store<1, 0, ACT, BIAS, NRM>(R, O, T, smem, N);
+    pg_store<1, 1, ACT, BIAS, NRM>(R, O, T, smem, N);
+    if constexpr (WP == 2) return;
   }
-  if (T.wm == 0) pg_barrier();
-  pg_vmwait<0>();
-  pg_store<0, 0, ACT, BIAS, NRM>(R, O, T, smem, N);
-  pg_store<0, 1, ACT, BIAS, NRM>(R, O, T, smem, N);
-  pg_store<1, 0, ACT, BIAS, NRM>(R, O, T, smem, N);
-  pg_store<1, 1, ACT, BIAS, NRM>(R, O, T, smem, N);
 }
 
 // ============================================================================
@@ -797,67 +919,8 @@ __global__ void __launch_bounds__(PG_THREADS, 1) pgemm_sk_kernel(
           }
     return;
   } else {
-    if (splits > 1) {
-      typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-      constexpr int TSLAB = PG_THREADS * 128;        // floats of one slice's tile
-      unsigned* word = reinterpret_cast<unsigned*>(smem + PG_RING_B);
-      __syncthreads();                               // every wave's DMA has landed
-      if (threadIdx.x == 0)
-        word[0] = __hip_atomic_fetch_add(&cnt[2 * tile], 1u, __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
-      __syncthreads();
-      const unsigned order = word[0];
-      float* tslab = slabs + (long)tile * splits * TSLAB;
-      // accumulator r = ((qm * 2 + qn) * 4 + i) * 2 + j of every lane is float4
-      // r * PG_THREADS + tid of a slice's slab
-#define PG_FOR_ACC(BODY)                                   \
-  _Pragma("unroll") for (int qm = 0; qm < 2; ++qm)         \
-  _Pragma("unroll") for (int qn = 0; qn < 2; ++qn)         \
-  _Pragma("unroll") for (int i = 0; i < 4; ++i)            \
-  _Pragma("unroll") for (int j = 0; j < 2; ++j) {          \
-    const int r = ((qm * 2 + qn) * 4 + i) * 2 + j;         \
-    f32x4_t& a = R.acc[qm][qn][i][j];                      \
-    BODY                                                   \
-  }
-      if (order + 1 < (unsigned)splits) {
-        // publish write-through (sc1): no L2 write-back fence (wgemm.hip)
-        const auto rs = __builtin_amdgcn_make_buffer_rsrc(tslab + (long)ks * TSLAB, (short)0,
-                                                          TSLAB * 4, 0x00020000);
-        PG_FOR_ACC(__builtin_amdgcn_raw_buffer_store_b128(
-            __builtin_bit_cast(u32x4_t, a), rs, (r * PG_THREADS + (int)threadIdx.x) * 16, 0, 16);)
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (threadIdx.x == 0)
-          __hip_atomic_fetch_add(&cnt[2 * tile + 1], 1u, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
-        return;
-      }
-      if (threadIdx.x == 0) {
-        while (__hip_atomic_load(&cnt[2 * tile + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
-               (unsigned)(splits - 1))
-          __builtin_amdgcn_s_sleep(2);
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __hip_atomic_store(&cnt[2 * tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&cnt[2 * tile + 1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      __syncthreads();
-      // ((p0 + p1) + ...) + p(S-1), own partial at its slice position
-      const f32x4_t* tin = reinterpret_cast<const f32x4_t*>(tslab) + threadIdx.x;
-      PG_FOR_ACC({
-        f32x4_t v;
-        if (ks > 0) {
-          v = tin[r * PG_THREADS];
-          for (int s = 1; s < ks; ++s) v += tin[(long)s * (TSLAB / 4) + r * PG_THREADS];
-          v += a;
-        } else {
-          v = a;
-        }
-        for (int s = ks + 1; s < splits; ++s) v += tin[(long)s * (TSLAB / 4) + r * PG_THREADS];
-        a = v;
-      })
-#undef PG_FOR_ACC
-    }
+    if (splits > 1 && !pg_join(R, smem, slabs + (long)tile * splits * PG_TSLAB, cnt + 2 * tile, ks, splits))
+      return;
     pg_store<0, 0, ACT, 0>(R, O, T, smem);
     pg_store<0, 1, ACT, 0>(R, O, T, smem);
     pg_store<1, 0, ACT, 0>(R, O, T, smem);
@@ -872,7 +935,7 @@ static int g_pg_cus = 0;
 template <int ACT, int BIAS, int WP = 0, int NRM = 0>
 static int pg_launch(bf16_t* C, const bf16_t* A, const bf16_t* W, const bf16_t* bias, int M,
                      int N, int K, int lda, int ldw, int ldc, int grid, hipStream_t stream,
-                     float* nrm = nullptr, PgGroups grp = PgGroups{}) {
+                     float* nrm = nullptr, PgGroups grp = PgGroups{}, PgTail tail = PgTail{}) {
   constexpr size_t smem = PG_RING_B + (BIAS == 1 ? PG_MAX_BIAS * 2 : 0);
   static_assert(smem <= 160 * 1024, "LDS");
   static bool attr = false;
@@ -883,7 +946,7 @@ static int pg_launch(bf16_t* C, const bf16_t* A, const bf16_t* W, const bf16_t* 
     attr = true;
   }
   pgemm_pp2_kernel<ACT, BIAS, 0, WP, NRM><<<dim3(grid), dim3(PG_THREADS), smem, stream>>>(
-      C, A, W, bias, M, N, K, lda, ldw, ldc, nrm, grp);
+      C, A, W, bias, M, N, K, lda, ldw, ldc, nrm, grp, tail);
   return (int)hipGetLastError();
 }
 
@@ -895,6 +958,55 @@ static int pg_cus() {
       g_pg_cus = p.multiProcessorCount;
   }
   return g_pg_cus;
+}
+
+// Workgroups that share the K-steps of each XCD row of the last round's tiles where it
+// leaves compute units idle, 0: the round runs as whole tiles.  The line is a fit to
+// times: whole tiles take 0.92 us a K-step, up to 1.27 as the chip fills; pieces 1.4, and
+// each piece of a tile beyond the first 11 (its fp32 tile of 256 KB out and in again); after
+// whole rounds the cut also hides 10 of their stores.  The workgroups drift apart by about
+// 0.9 us a round, and the pieces of a tile wait for the last of them.
+// Whole and cut, M x N x K: 2048 x 4096 x 4096 87 and 72 us, x 14336 262 and 180; 2048 x
+// 18688 x 4096 (2.3 rounds) 262 and 241; 6464 x 4096 x 14336 (1.6) 600 and 550; 600 x 4096 x
+// 14336 (48 tiles) 214 and 107.  Not cut, since it lost or made no difference: 600 x 6144 x
+// 4096, 5000 x 768 x 3072, 7680 x 4096 x 14336 (1.9), 7680 x 28672 x 4096 (13.1).
+static int pg_tail_share(int M, int N, int K) {
+  if (pg_cus() == 0 || g_pg_cus % 8 || g_pg_cus > 256) return 0;
+  const int row = g_pg_cus / 8, nk = K / 64;
+  const long tiles = (long)((M + 255) / 256) * (N / 256);
+  const int rest = (int)(tiles % g_pg_cus), most = (rest + row - 1) / row;
+  const float whole = nk * (0.92f + 0.35f * rest / g_pg_cus) + (tiles > g_pg_cus ? 3.f : -7.f);
+  int best = 0;
+  float gain = 3.f + 0.9f * (tiles / g_pg_cus);
+  for (int p = most + 1; p <= 8 && p <= 4 * most && most > 0; ++p) {
+    const float per = (float)(most * nk) / p;
+    if (per < 4) break;
+    const int pieces = (p + most - 1) / most + (p % most != 0);     // at most, of a tile
+    const float g = whole - 1.4f * per - 11.f * (pieces - 1);
+    if (g > gain) {
+      gain = g;
+      best = p;
+    }
+  }
+  return best;
+}
+
+// floats of pieces' tiles that pgemm takes for its last round (0: it runs whole tiles only)
+long pgemm_tail_floats(int M, int N, int K) {
+  if (M <= 0 || N % 256 || K % 64 || pg_tail_share(M, N, K) == 0) return 0;
+  return (long)(g_pg_cus / 8) * PG_TAIL_SLOTS * PG_TSLAB;
+}
+
+// Estimated time: a tile takes 5 us + 0.92 (few workgroups) to 1.27 us (a full chip) per
+// K-step (measured 16 / 22 us at K 768, 48 / 55 at 3072, 63 / 82 at 4096)
+float pgemm_us(int M, int N, int K) {
+  const long tiles = (long)((M + 255) / 256) * (N / 256), nk = K / 64;
+  const long whole = tiles / 256, rest = tiles % 256;
+  const float round = 5.f + 1.27f * nk;
+  if (rest == 0) return whole * round;
+  const int p = pg_tail_share(M, N, K);
+  if (p == 0) return whole * round + 5.f + nk * (0.92f + 0.35f * rest / 256.f);
+  return whole * round + 23.f + 1.4f * ((rest + 31) / 32) * nk / p;
 }
 
 // Grouped rows on the persistent 256 x 256 tile: M sorted rows (A rows src[..] or
@@ -927,9 +1039,11 @@ int pgemm_grouped(void* C, const void* A, const void* W, int M, int N, int K, lo
 // nrm (the RMSNorm folded into the projections): with res, the new residual
 // rows' sums of squares per 64-column block go to nrm [M][N / 64]; without,
 // the output rows are scaled by nrm [M] (plain product or SwiGLU, no bias)
+// slabs (pgemm_tail_floats of them) and cnt (512 zeroed counters, zero again
+// afterwards): the last round in pieces; null: whole tiles only
 int pgemm(void* C, const void* A, const void* W, const void* bias, int M, int N, int K, long lda,
           long ldw, long ldc, int act, int grid, int res, int wpacked, float* nrm,
-          hipStream_t stream) {
+          hipStream_t stream, float* slabs, unsigned* cnt) {
   if (M <= 0) return 0;
   if (wpacked && (bias != nullptr || ldw != K || (act != 0 && act != 3) || (res && act != 0)))
     return -1;
@@ -946,8 +1060,12 @@ int pgemm(void* C, const void* A, const void* W, const void* bias, int M, int N,
     return -1;
   if (pg_cus() == 0) return -2;
   const long tiles = (long)((M + 255) / 256) * (N / 256);
-  if (grid <= 0) grid = g_pg_cus;
-  if (grid > tiles) grid = (int)tiles;
+  PgTail tail{};
+  if (grid <= 0) {
+    grid = g_pg_cus;
+    if (slabs && cnt) tail = PgTail{pg_tail_share(M, N, K), slabs, cnt};
+  }
+  if (grid > tiles && tail.share == 0) grid = (int)tiles;
   auto C_ = (bf16_t*)C;
   auto A_ = (const bf16_t*)A;
   auto W_ = (const bf16_t*)W;
@@ -955,11 +1073,11 @@ int pgemm(void* C, const void* A, const void* W, const void* bias, int M, int N,
   const int ia = (int)lda, iw = (int)ldw, ic = (int)ldc;
   if (bias != nullptr) {
     switch (act) {
-      case 0: return pg_launch<0, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
-      case 1: return pg_launch<1, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
-      case 2: return pg_launch<2, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
-      case 4: return pg_launch<4, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
-      case 7: return pg_launch<7, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
+      case 0: return pg_launch<0, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
+      case 1: return pg_launch<1, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
+      case 2: return pg_launch<2, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
+      case 4: return pg_launch<4, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
+      case 7: return pg_launch<7, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
     }
     return -1;
   }
@@ -967,25 +1085,25 @@ int pgemm(void* C, const void* A, const void* W, const void* bias, int M, int N,
     // the folded-norm forms: producer (residual) and consumers (QKV plain,
     // gate/up SwiGLU), row-major or packed W
 #define LMX_PG_N(WPV)                                                                        \
-    if (res) return pg_launch<0, 2, WPV, 2>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nrm); \
-    if (act == 3) return pg_launch<3, 0, WPV, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nrm); \
-    return pg_launch<0, 0, WPV, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nrm);
+    if (res) return pg_launch<0, 2, WPV, 2>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nrm, PgGroups{}, tail); \
+    if (act == 3) return pg_launch<3, 0, WPV, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nrm, PgGroups{}, tail); \
+    return pg_launch<0, 0, WPV, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nrm, PgGroups{}, tail);
     if (wpacked) { LMX_PG_N(1) } else { LMX_PG_N(0) }
 #undef LMX_PG_N
   }
   if (wpacked) {
-    if (res) return pg_launch<0, 2, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
-    if (act == 3) return pg_launch<3, 0, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
-    return pg_launch<0, 0, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
+    if (res) return pg_launch<0, 2, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
+    if (act == 3) return pg_launch<3, 0, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
+    return pg_launch<0, 0, 1>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
   }
-  if (res) return pg_launch<0, 2>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
+  if (res) return pg_launch<0, 2>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
   switch (act) {
-    case 0: return pg_launch<0, 0>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
-    case 1: return pg_launch<1, 0>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
-    case 2: return pg_launch<2, 0>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
-    case 3: return pg_launch<3, 0>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
-    case 4: return pg_launch<4, 0>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
-    case 5: return pg_launch<5, 0>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream);
+    case 0: return pg_launch<0, 0>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
+    case 1: return pg_launch<1, 0>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
+    case 2: return pg_launch<2, 0>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
+    case 3: return pg_launch<3, 0>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
+    case 4: return pg_launch<4, 0>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
+    case 5: return pg_launch<5, 0>(C_, A_, W_, b_, M, N, K, ia, iw, ic, grid, stream, nullptr, PgGroups{}, tail);
   }
   return -1;
 }
@@ -995,7 +1113,7 @@ template <int ACT, int EPI>
 static int pg_sk_launch(bf16_t* C, const bf16_t* A, const bf16_t* W, float* slabs, unsigned* cnt,
                         int M, int N, int K, int lda, int ldw, int ldc, int splits, int grid,
                         hipStream_t stream) {
-  constexpr size_t smem = PG_RING_B + 16;
+  constexpr size_t smem = PG_RING_B;
   static bool attr = false;
   if (!attr) {
     const hipError_t e = hipFuncSetAttribute((const void*)pgemm_sk_kernel<ACT, EPI>,

@@ -1772,10 +1772,31 @@ def pgemm(a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, ac
     _chk(out.shape == (M, ncols) and out.stride(1) == 1 and out.stride(0) % 4 == 0
          and out.data_ptr() % 8 == 0, "pgemm output layout")
     PGEMM_CALLS[0] += 1
+    tail, cnt = pgemm_tail(a.device, M, N, K) if grid == 0 else (None, None)
     native().pgemm(_ptr(out), _ptr(a), _ptr(w), _ptr(bias), M, N, K, a.stride(0), w.stride(0),
                    out.stride(0), act, grid, int(residual is not None), int(packed), _ptr(nrm),
-                   _stream())
+                   _stream(), _ptr(tail), _ptr(cnt))
     return out
+
+
+_PG_COUNTERS: dict = {}    # (device, stream) -> counters of K13's last round, zero between calls
+
+
+def pgemm_counters(dev: torch.device) -> torch.Tensor:
+    key = (dev.index, _stream())
+    if key not in _PG_COUNTERS:
+        _PG_COUNTERS[key] = torch.zeros(512, dtype=torch.int32, device=dev)
+    return _PG_COUNTERS[key]
+
+
+def pgemm_tail(dev: torch.device, M: int, N: int, K: int) -> tuple:
+    """(slabs, counters) of a product whose last round of tiles K13 cuts along K, or
+    (None, None): whole tiles only.  So is every product under capture: a graph may be
+    replayed beside this stream, whose counters it would share."""
+    n = native().pgemm_tail_floats(M, N, K)
+    if n == 0 or torch.cuda.is_current_stream_capturing():
+        return None, None
+    return torch.empty(n, dtype=torch.float32, device=dev), pgemm_counters(dev)
 
 
 def row_scale(eps: float, part: torch.Tensor | None = None,

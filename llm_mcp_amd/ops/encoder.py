@@ -82,13 +82,17 @@ def layers(x: torch.Tensor, weights: list, names: tuple, b: Batch, cu: torch.Ten
            cos_sin: torch.Tensor | None) -> torch.Tensor:
     """All layers over x [T, d], in place.  ``names``: a layer's tensors in the order of
     encoder.h (None: the model has none there)."""
-    from . import PGEMM_CALLS, _ptr, _stream, native
+    from . import PGEMM_CALLS, _ptr, _stream, native, pgemm_counters
     T, d = x.shape
     dev, n = x.device, native().enc_slab_floats(T, d, I)
     rows = torch.empty(T * (5 * d + I), dtype=x.dtype, device=dev)       # h, attn, qkv, g
     at = [0, T * d, 2 * T * d, 5 * T * d]
     h, attn, qkv, g = (_ptr(rows) + 2 * a for a in at)
-    slabs = torch.empty(n, dtype=torch.float32, device=dev)
+    tail = native().enc_tail_floats(T, d, I, gelu)
+    if torch.cuda.is_current_stream_capturing():
+        tail = 0               # see ops.pgemm_tail
+    slabs = torch.empty(n + tail, dtype=torch.float32, device=dev)
+    cnt = pgemm_counters(dev) if tail else None
     # masked keys weigh 0 times V, which must be finite
     kv = torch.zeros(2 * b.pages * H * PAGE * D, dtype=x.dtype, device=dev)
     ptrs = [0 if k is None else L[k].data_ptr() for L in weights for k in names]
@@ -96,6 +100,7 @@ def layers(x: torch.Tensor, weights: list, names: tuple, b: Batch, cu: torch.Ten
         ptrs, T, d, I, H, D, PAGE, gelu, float(eps), float(scale), _ptr(x), h, qkv, attn, g,
         _ptr(slabs), n, _ptr(kv), _ptr(kv) + kv.numel(), _ptr(b.slots), _ptr(b.positions),
         _ptr(cos_sin), _ptr(b.tables), b.tables.stride(0), _ptr(cu), _ptr(b.ctx), _ptr(b.tiles),
-        b.tiles.numel() // 2, q_per_tile, _stream())
+        b.tiles.numel() // 2, q_per_tile, _ptr(slabs) + 4 * n if tail else 0, tail, _ptr(cnt),
+        _stream())
     PGEMM_CALLS[0] += 4 * len(weights)
     return x

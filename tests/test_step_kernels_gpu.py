@@ -264,3 +264,66 @@ def test_linear_of_few_rows(M):
             assert ops.SGEMM_CALLS[0] - n == int(M <= (32 if N == 2048 else 8))
             torch.testing.assert_close(ops.linear(xs, w, bias=b).double(), y + b.double(), atol=2e-2,
                                        rtol=1e-2)
+
+
+# --------------------------------------------- K13: the last round in pieces --
+def _k13(M, N, K, **kw):
+    a = torch.randn(M, K, device=DEV).bfloat16()
+    w = torch.randn(N, K, device=DEV).bfloat16() * K ** -0.5
+    return a, w
+
+
+@pytest.mark.parametrize("M,N,K,cut", [
+    (2048, 4096, 4096, True),      # half a round: two pieces a tile, one a workgroup
+    (2300, 4096, 14336, True),     # 144 tiles: pieces that end inside tiles, ragged rows
+    (257, 512, 6144, True),        # four tiles of four pieces each
+    (100, 256, 8192, True),        # one tile
+    (6500, 3328, 4160, True),      # a whole round, then 82 tiles
+    (7000, 4864, 832, False),      # 532 tiles: 20 of 13 steps
+    (2048, 8192, 512, False)])     # one round, whole
+def test_k13_last_round(M, N, K, cut):
+    """Every form of the epilogue where the last round of tiles is cut along K: the numbers
+    of a product in fp32, the same bits each time, nothing left in the counters."""
+    assert (ops.native().pgemm_tail_floats(M, N, K) > 0) == cut
+    a, w = _k13(M, N, K)
+    z = a.float() @ w.float().t()
+    tol = dict(atol=4e-3, rtol=2.0 ** -7)
+    y = ops.pgemm(a, w)
+    torch.testing.assert_close(y.float(), z, **tol)
+    for _ in range(3):
+        assert torch.equal(ops.pgemm(a, w), y)
+    b = torch.randn(N, device=DEV).bfloat16()
+    torch.testing.assert_close(ops.pgemm(a, w, bias=b).float(), z + b.float(), **tol)
+    torch.testing.assert_close(ops.pgemm(a, w, bias=b, act=ops.ACT_GELU_ERF).float(),
+                               torch.nn.functional.gelu(z + b.float()), **tol)
+    g, u = z.view(M, N // 32, 2, 16).unbind(2)
+    torch.testing.assert_close(ops.pgemm(a, w, act=ops.ACT_SWIGLU).float(),
+                               (torch.nn.functional.silu(g) * u).reshape(M, -1), **tol)
+    r = torch.randn(M, N, device=DEV).bfloat16()
+    want = (r.float() + z.bfloat16().float())
+    ssq = torch.empty(M, N // 64, device=DEV)
+    ops.pgemm(a, w, residual=r, ssq=ssq)
+    torch.testing.assert_close(r.float(), want, atol=4e-2, rtol=2.0 ** -7)
+    torch.testing.assert_close(ssq, r.float().pow(2).view(M, N // 64, 64).sum(-1), atol=1e-3, rtol=1e-5)
+    s = torch.rand(M, device=DEV) + 0.5
+    torch.testing.assert_close(ops.pgemm(a, w, row_scale=s).float(), z * s[:, None], **tol)
+    assert not any(int(c.abs().sum()) for c in ops._PG_COUNTERS.values())
+
+
+def test_k13_under_capture():
+    """A captured product runs whole tiles and replays beside eager ones."""
+    a, w = _k13(2048, 4096, 4096)
+    y, st = ops.pgemm(a, w), torch.cuda.Stream()
+    out = torch.empty_like(y)
+    st.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(st):
+        ops.pgemm(a, w, out=out)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            ops.pgemm(a, w, out=out)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        assert torch.equal(ops.pgemm(a, w), y)
+        torch.cuda.synchronize()
+        torch.testing.assert_close(out.float(), y.float(), atol=4e-3, rtol=2.0 ** -7)
