@@ -19,6 +19,8 @@ namespace lmx {
 int rmsnorm(void*, void*, const void*, const void*, int, int, long, long, float, hipStream_t);
 int layernorm(void*, const void*, const void*, const void*, const void*, int, int, float,
               hipStream_t);
+int enc_attention(const void*, long, int, int, const int*, const int*, int, const float*, void*, long,
+                  float, float, hipStream_t);
 int rope_cache(void*, long, const int*, const float*, int, int, int, int, const int*, void*, void*,
                int, int, int, const void*, const void*, float, int, hipStream_t);
 int kv_write(const void*, const void*, long, const int*, int, int, int, void*, void*, int,
@@ -604,19 +606,21 @@ PYBIND11_MODULE(_lmx_kernels, m) {
   });
   m.def("enc_slab_floats", &lmx::enc_slab_floats);
   m.def("enc_tail_floats", &lmx::enc_tail_floats);
-  m.def("encoder_layers", [](const std::vector<uintptr_t>& w, int T, int d, int I, int H, int D, int page,
-                             bool gelu, float eps, float scale, uptr x, uptr h, uptr qkv, uptr attn,
-                             uptr g, uptr slabs, long slab_floats, uptr kc, uptr vc, uptr slots,
-                             uptr positions, uptr cos_sin, uptr bt, int bt_stride, uptr cu, uptr ctx,
-                             uptr tiles, int ntiles, int q_per_tile, uptr tail, long tail_floats,
-                             uptr cnt, uptr stream) {
+  m.def("enc_attention", [](uptr qkv, long ld, int H, int D, uptr cu, uptr tiles, int ntiles, uptr cos_sin,
+                            uptr out, long ldo, float scale, float rescale_thr, uptr stream) {
+    check(lmx::enc_attention(P<void>(qkv), ld, H, D, P<int>(cu), P<int>(tiles), ntiles, P<float>(cos_sin),
+                             P<void>(out), ldo, scale, rescale_thr, S(stream)),
+          "enc_attention");
+  });
+  m.def("encoder_layers", [](const std::vector<uintptr_t>& w, int T, int d, int I, int H, int D, bool gelu,
+                             float eps, float scale, uptr x, uptr h, uptr qkv, uptr attn, uptr g,
+                             uptr slabs, long slab_floats, uptr cos_sin, uptr cu, uptr tiles,
+                             int ntiles, uptr tail, long tail_floats, uptr cnt, uptr stream) {
     if (w.size() % lmx::kEncPtrs) throw std::runtime_error("encoder_layers: weights");
-    const lmx::EncArgs a{(int)(w.size() / lmx::kEncPtrs), T, d, I, H, D, page, gelu, eps, scale,
+    const lmx::EncArgs a{(int)(w.size() / lmx::kEncPtrs), T, d, I, H, D, gelu, eps, scale,
                          P<void>(x), P<void>(h), P<void>(qkv), P<void>(attn), P<void>(g),
-                         P<float>(slabs), slab_floats, P<void>(kc), P<void>(vc), P<int>(slots),
-                         P<int>(positions), P<float>(cos_sin), P<int>(bt), bt_stride, P<int>(cu),
-                         P<int>(ctx), P<int>(tiles), ntiles, q_per_tile, P<float>(tail), tail_floats,
-                         P<unsigned>(cnt)};
+                         P<float>(slabs), slab_floats, P<float>(cos_sin), P<int>(cu), P<int>(tiles),
+                         ntiles, P<float>(tail), tail_floats, P<unsigned>(cnt)};
     check(lmx::encoder_layers(a, w.data(), S(stream)), "encoder_layers");
   });
   m.def("rmsnorm_slabs", [](uptr out, uptr residual, uptr slabs, int nsl, long slab_stride,

@@ -11,7 +11,7 @@ namespace lmx {
 constexpr int kEncPtrs = 12;
 
 struct EncArgs {
-  int layers, T, d, I, H, D, page;
+  int layers, T, d, I, H, D;
   bool gelu;                       // gelu(h W1 + b) instead of SwiGLU
   float eps, scale;
   // rows of T tokens, bf16: x [d] (in: the first norm's output, out: the last one's),
@@ -19,13 +19,9 @@ struct EncArgs {
   void *x, *h, *qkv, *attn, *g;
   float* slabs;
   long slab_floats;
-  void *kc, *vc;                   // pages of this forward
-  const int *slots, *positions;    // per token
   const float* cos_sin;            // null: no rotation
-  const int* bt;                   // page tables [sequences][bt_stride]
-  int bt_stride;
-  const int *cu, *ctx, *tiles;
-  int ntiles, q_per_tile;
+  const int *cu, *tiles;           // enc_attention's
+  int ntiles;
   float* tail;                     // K13's last round in pieces (pgemm): floats and counters
   long tail_floats;
   unsigned* cnt;

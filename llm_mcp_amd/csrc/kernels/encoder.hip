@@ -2,7 +2,7 @@
 // launch of a forward from here, so that a short request is bound by its kernels
 // and not by the interpreter (96 to 290 launches of 3 to 6 us each).
 //
-//   qkv = x Wqkv^T + b;  rotation (nomic) and K / V pages;  attention
+//   qkv = x Wqkv^T + b;  attention on its rows (K24), with the rotation (nomic)
 //   h = LN(x + attn Wo^T + b);  g = act(h W1^T + b);  x = LN(h + g W2^T + b)
 //
 // Requests range from one query of ten tokens to 64 k tokens, so a projection has
@@ -22,13 +22,8 @@ namespace lmx {
 int layernorm(void*, const void*, const void*, const void*, const void*, int, int, float, hipStream_t);
 int layernorm_slabs(void*, const float*, int, long, const void*, const void*, const void*, const void*,
                     int, int, float, hipStream_t);
-int rope_cache(void*, long, const int*, const float*, int, int, int, int, const int*, void*, void*,
-               int, int, int, const void*, const void*, float, int, hipStream_t);
-int kv_write(const void*, const void*, long, const int*, int, int, int, void*, void*, int,
-             hipStream_t);
-int paged_prefill(const void*, long, const void*, const void*, const int*, int, const int*,
-                  const int*, const int*, int, void*, long, int, int, int, int, float, int, int,
-                  const int*, const float*, const void*, long, int, int, float, hipStream_t);
+int enc_attention(const void*, long, int, int, const int*, const int*, int, const float*, void*, long,
+                  float, float, hipStream_t);
 int dgemm(void*, const void*, const void*, float*, unsigned*, int, int, int, int, long, long, long,
           int, int, int, hipStream_t, const void*);
 int pgemm(void*, const void*, const void*, const void*, int, int, int, long, long, long, int, int, int,
@@ -109,7 +104,7 @@ long enc_tail_floats(int T, int d, int I, bool gelu) {
 int encoder_layers(const EncArgs& a, const uintptr_t* w, hipStream_t stream) {
   const int T = a.T, d = a.d, I = a.I;
   if (T <= 0) return 0;
-  if (d != a.H * a.D || d % 256 || I % 256 || (a.D != 64 && a.D != 128)) return -1;
+  if (d != a.H * a.D || d % 256 || I % 256 || a.D != 64) return -1;
   for (int i = 0; i < a.layers * kEncPtrs; ++i)
     if (w[i] & 15) return -2;
   auto k13 = [&](void* out, const void* x, uintptr_t W, uintptr_t b, int N, int K, int ldc, int act) {
@@ -143,19 +138,12 @@ int encoder_layers(const EncArgs& a, const uintptr_t* w, hipStream_t stream) {
     return e ? e : layernorm_slabs(out, a.slabs, p.splits, (long)T * d, (void*)b, residual, (void*)g,
                                    (void*)s, T, d, a.eps, stream);
   };
-  char* q = (char*)a.qkv;
   for (int l = 0; l < a.layers; ++l, w += kEncPtrs) {
     const bool gelu = a.gelu;
     int e = full(a.qkv, a.x, w[0], w[1], 3 * d, d, 0);
     if (!e)
-      e = a.cos_sin ? rope_cache(a.qkv, 3L * d, a.positions, a.cos_sin, T, a.H, a.H, a.D, a.slots, a.kc,
-                                 a.vc, a.page, 0, 0, nullptr, nullptr, 0.f, 0, stream)
-                    : kv_write(q + 2L * d, q + 4L * d, 3L * d, a.slots, T, a.H, a.D, a.kc, a.vc, a.page,
-                               stream);
-    if (!e)
-      e = paged_prefill(a.qkv, 3L * d, a.kc, a.vc, a.bt, a.bt_stride, a.cu, a.ctx, a.tiles, a.ntiles,
-                        a.attn, d, a.H, a.H, a.D, a.page, a.scale, 0, a.q_per_tile, nullptr, nullptr,
-                        nullptr, 0, 0, 0, 0.f, stream);
+      e = enc_attention(a.qkv, 3L * d, a.H, a.D, a.cu, a.tiles, a.ntiles, a.cos_sin, a.attn, d, a.scale,
+                        8.f, stream);
     if (!e) e = normed(a.h, a.attn, w[2], w[3], a.x, w[4], w[5], d, a.qkv);
     if (!e) e = full(a.g, a.h, w[6], w[7], gelu ? I : 2 * I, d, gelu ? 4 : 3);
     if (!e) e = normed(a.x, a.g, w[8], w[9], a.h, w[10], w[11], I, a.qkv);

@@ -67,13 +67,6 @@ __device__ __forceinline__ void split1(float x, uint16_t& hi, uint16_t& lo) {
   lo = f2bf(x - bf2f(hi));
 }
 
-// two values to packed bf16 (v_cvt_pk_bf16_f32; a builtin and not asm, so that a value an
-// MFMA has just made is waited for)
-__device__ __forceinline__ uint32_t cvt_pk(float a, float b) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf2));
-}
 __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
   hi = cvt_pk(a, b);
   lo = cvt_pk(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u));

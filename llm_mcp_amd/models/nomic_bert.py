@@ -112,12 +112,11 @@ class NomicBertModel:
         dev = self.device
         if ids.is_cuda and self.gu_k13 and not self.fuse_q_rope and encoder.layers_ok(
                 w["layers"], tuple(n for n in NATIVE if n), d, cfg.intermediate_size, H, D):
-            qpt = ops.prefill_q_per_tile(H, H, D)
-            b = encoder.batch(lens, qpt, ids.device)
+            b = encoder.batch(lens, ids.device)
             x = encoder.embed_norm(ids, w["word"], w["type"], w["emb_ln_w"], w["emb_ln_b"],
                                    cfg.ln_eps)
             encoder.layers(x, w["layers"], NATIVE, b, cu, cfg.intermediate_size, H, D, cfg.ln_eps,
-                           self.scale, qpt, False, self.cos_sin)
+                           self.scale, False, self.cos_sin)
             return ops.mean_pool_l2(x, cu, dims or cfg.embed_dim, normalize)
         # per-sequence page-aligned slots in a scratch paged K/V cache, built
         # with array ops (no per-token Python work on the host critical path)

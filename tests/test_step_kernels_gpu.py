@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from llm_mcp_amd import ops
-from llm_mcp_amd.ops import mixers, ref
+from llm_mcp_amd.ops import encoder, mixers, ref
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -327,3 +327,42 @@ def test_k13_under_capture():
         assert torch.equal(ops.pgemm(a, w), y)
         torch.cuda.synchronize()
         torch.testing.assert_close(out.float(), y.float(), atol=4e-3, rtol=2.0 ** -7)
+
+
+# ------------------------------------------------- K24: the encoders' attention --
+@pytest.mark.parametrize("lens", [[1], [16], [33, 1, 2], [64, 65, 63], [127, 128, 129, 5], [700, 31, 32, 256],
+                                  [1, 1024, 3]])
+@pytest.mark.parametrize("H,rope,thr", [(12, True, 8.0), (3, False, 8.0), (16, True, 0.0), (2, False, 0.0)])
+def test_k24_attention(lens, H, rope, thr):
+    """Against softmax(q k^T) v in 64 bits on the same rounded operands; the weights enter the
+    second product as bf16 and the output is bf16: 2^-8 each of sum p |v| and of the output.
+    One sequence is NaN and must not be seen by the others."""
+    D, T = 64, sum(lens)
+    wide = torch.randn(T, 3 * H * D + 8, device=DEV).bfloat16()
+    qkv = wide[:, :3 * H * D]                                   # rows wider than q, k, v
+    qkv[:, :2 * H * D] *= 3                                     # wide scores
+    cu = torch.tensor([0] + lens, device=DEV).cumsum(0).int()
+    cs = None
+    if rope:
+        a = torch.arange(max(lens), device=DEV)[:, None] * 1e4 ** (-torch.arange(32, device=DEV) / 32)
+        cs = torch.cat([a.cos(), a.sin()], 1).float().contiguous()
+    bad = len(lens) // 2 if len(lens) > 1 else -1
+    if bad >= 0:
+        qkv[cu[bad]:cu[bad + 1]] = float("nan")
+    got = encoder.attention(qkv, cu, encoder.batch(lens, torch.device(DEV)), H, D ** -0.5, cs, thr)
+    for i, n in enumerate(lens):
+        lo, o = int(cu[i]), got[int(cu[i]):int(cu[i + 1])]
+        if i == bad:
+            assert o.isnan().all()
+            continue
+        q, k, v = qkv[lo:lo + n].float().view(n, 3, H, D).unbind(1)
+        if rope:
+            c, s = cs[:n, None, :32], cs[:n, None, 32:]
+            q, k = (torch.cat([x[..., :32] * c - x[..., 32:] * s, x[..., 32:] * c + x[..., :32] * s], -1)
+                    .bfloat16().float() for x in (q, k))
+        q, k, v = (x.double().transpose(0, 1) for x in (q, k, v))
+        p = (q @ k.transpose(1, 2) * D ** -0.5).softmax(-1)
+        want, bound = p @ v, 2.0 ** -8 * (p @ v.abs())
+        bound = 1.05 * (bound + 2.0 ** -8 * (want.abs() + bound)) + 1e-4      # fp32 sums and exponents
+        err = (o.double().view(n, H, D).transpose(0, 1) - want).abs()
+        assert (err <= bound).all(), (err - bound).max()
