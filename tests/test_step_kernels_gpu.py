@@ -366,3 +366,36 @@ def test_k24_attention(lens, H, rope, thr):
         bound = 1.05 * (bound + 2.0 ** -8 * (want.abs() + bound)) + 1e-4      # fp32 sums and exponents
         err = (o.double().view(n, H, D).transpose(0, 1) - want).abs()
         assert (err <= bound).all(), (err - bound).max()
+
+
+# ---------------------------------------- K4: short partitions and their sum --
+@pytest.mark.parametrize("ctxs,parts", [([255, 256, 257], 16), ([1, 513, 2049], 8), ([2304], 9), ([6000], 40),
+                                        ([300] * 8, 4), ([700] * 9, 4), ([3000, 40], 17)])
+@pytest.mark.parametrize("Hq,Hkv,D", [(32, 8, 128), (8, 8, 64)])
+def test_k4_partitions(ctxs, parts, Hq, Hkv, D):
+    """Few rows, cut to 256 tokens, up to 24 partitions (sums of 8 at a time): the softmax in
+    64 bits; weights as bf16 and a bf16 output, 2^-8 each of sum p |v| and of the output."""
+    B, pages = len(ctxs), [-(-c // 32) for c in ctxs]
+    NB = sum(pages) + 1
+    kc = torch.randn(NB, Hkv, 32, D, device=DEV).bfloat16() * 2
+    vc = torch.randn(NB, Hkv, 8, D, 4, device=DEV).bfloat16()           # key quads
+    bt = torch.zeros(B, max(pages), dtype=torch.int32, device=DEV)
+    perm = torch.randperm(NB, device=DEV).int()
+    for b in range(B):
+        bt[b, :pages[b]] = perm[sum(pages[:b]):sum(pages[:b + 1])]
+    ctx = torch.tensor(ctxs, dtype=torch.int32, device=DEV)
+    q = torch.randn(B, Hq * D, device=DEV).bfloat16()
+    out = torch.empty(B, Hq * D, dtype=torch.bfloat16, device=DEV)
+    ws = ops.DecodeWorkspace(B, Hq, D, parts, DEV)
+    ws.part_o.fill_(float("nan"))                                       # unused partitions are not read
+    ws.part_ml.fill_(float("nan"))
+    ops.paged_decode_attention(q, kc, vc, bt, ctx, D ** -0.5, out, ws, Hq=Hq)
+    for b, n in enumerate(ctxs):
+        t = bt[b, :pages[b]].long()
+        k = kc[t].transpose(1, 2).reshape(-1, Hkv, D)[:n].double()
+        v = vc[t].permute(0, 2, 4, 1, 3).reshape(-1, Hkv, D)[:n].double()
+        k, v = (x.repeat_interleave(Hq // Hkv, 1).transpose(0, 1) for x in (k, v))
+        p = (q[b].double().view(Hq, 1, D) @ k.transpose(1, 2) * D ** -0.5).softmax(-1)
+        want, bound = p @ v, 2.0 ** -8 * (p @ v.abs())
+        bound = 1.05 * (bound + 2.0 ** -8 * (want.abs() + bound)) + 1e-4
+        assert ((out[b].double().view(Hq, 1, D) - want).abs() <= bound).all()
