@@ -32,7 +32,7 @@ KERNEL_SOURCES = ["norm.hip", "rope_cache.hip", "attention.hip", "sampling.hip",
                   "elementwise.hip", "gemm.hip", "dgemm.hip", "pgemm.hip",
                   "rsgemm.hip", "allreduce.hip", "conv.hip", "linscan.hip",
                   "grouped.hip", "moe.hip", "rglru.hip", "latent.hip", "delta.hip", "talk.hip",
-                  "encoder.hip", "encattn.hip", "sgemm.hip"]
+                  "encoder.hip", "encattn.hip", "sgemm.hip", "gemv.hip"]
 RUNTIME_SOURCES = ["job_queue.cpp", "block_manager.cpp", "scheduler.cpp", "bindings.cpp"]
 
 

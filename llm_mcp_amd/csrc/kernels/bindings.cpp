@@ -134,6 +134,8 @@ int dgemm(void*, const void*, const void*, float*, unsigned*, int, int, int, int
           int, int, int, hipStream_t, const void*);
 int sgemm(void*, const void*, const void*, int, int, int, long, long, long, int, int, const void*,
           hipStream_t);
+int gemv(void*, const void*, const void*, int, int, int, long, long, long, int, int, const void*,
+         hipStream_t);
 int layernorm_slabs(void*, const float*, int, long, const void*, const void*, const void*, const void*,
                     int, int, float, hipStream_t);
 int embed_layernorm(void*, const int*, const void*, int, const void*, const void*, const int*,
@@ -585,6 +587,12 @@ PYBIND11_MODULE(_lmx_kernels, m) {
     check(lmx::sgemm(P<void>(C), P<void>(A), P<void>(W), M, N, K, lda, ldw, ldc, epi, splits,
                      P<void>(bias), S(stream)),
           "sgemm");
+  });
+  m.def("gemv", [](uptr C, uptr A, uptr W, int M, int N, int K, long lda, long ldw, long ldc, int epi,
+                   int splits, uptr bias, uptr stream) {
+    check(lmx::gemv(P<void>(C), P<void>(A), P<void>(W), M, N, K, lda, ldw, ldc, epi, splits,
+                    P<void>(bias), S(stream)),
+          "gemv");
   });
   m.def("layernorm_slabs", [](uptr out, uptr slabs, int nsl, long stride, uptr bias, uptr residual,
                               uptr w, uptr b, int rows, int cols, float eps, uptr stream) {

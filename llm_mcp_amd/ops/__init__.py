@@ -818,6 +818,50 @@ def sgemm_splits(M: int, N: int, K: int, epi: int = 0) -> int | None:
     return next(s for s in (4, 2, 1) if s == 1 or (N // 16 * s <= 256 and K // 32 % s == 0))
 
 
+# K25 (csrc/kernels/gemv.hip), one or two rows: whole weight rows streamed. Faster than
+# the other kernels at every size but where K14 has packed weights (4096 x 14336: 21.7 us
+# against 20.7) and one near 16384 x 4096 (25.9 against 24.3; 15360 and 17408 columns 23.0
+# and 26.5 against 29.5 and 51); at four rows its FMAs take as long as the stream.
+GEMV_MAX_M, GEMV_K = 2, 1024
+GEMV_CALLS = [0]           # host-side launch count (tests: the K25 path really ran)
+
+
+def gemv_splits(x: torch.Tensor, w: torch.Tensor, epi: int = 0, out: torch.Tensor | None = None) -> int | None:
+    """K slices of this product on K25 (1 except for epi 2, fp32 slabs), or None: not its range."""
+    M, N, K = x.shape[0], w.shape[0], w.shape[1]
+    if not (0 < M <= GEMV_MAX_M) or N % 32 or K % GEMV_K or not pgemm_operands_ok(x, w):
+        return None
+    if out is not None and (out.stride(1) != 1 or out.stride(0) % 2 or out.data_ptr() % 4):
+        return None
+    if epi != 4 and rs_choice(M, N, K, epi=epi, w=w) is not None:
+        return None
+    # 2048 waves (two a SIMD) at least
+    return 2 if epi == 2 and N < 4096 and K // GEMV_K % 2 == 0 else 1
+
+
+def gemv(a: torch.Tensor, w: torch.Tensor, epi: int = 0, splits: int = 1,
+         bias: torch.Tensor | None = None, out: torch.Tensor | None = None):
+    """a @ w^T on K25 (1 or 2 rows), epilogues as ``sgemm``'s (no gelu)."""
+    M, K = a.shape
+    N = w.shape[0]
+    _bf16(a, "a"); _bf16(w, "w")
+    _chk(0 < M <= GEMV_MAX_M and N % 32 == 0 and K % GEMV_K == 0 and K // GEMV_K % splits == 0
+         and (splits == 1 or epi == 2), f"gemv shape M={M} N={N} K={K} S={splits}")
+    _chk(w.shape[1] == K and pgemm_operands_ok(a, w), "gemv operands need 16-B aligned rows")
+    GEMV_CALLS[0] += 1
+    if epi == 2:
+        p = Partials.empty(a, splits, N)
+        native().gemv(_ptr(p.slabs), _ptr(a), _ptr(w), M, N, K, a.stride(0), w.stride(0), N, 2, splits, 0,
+                      _stream())
+        return p
+    if out is None:
+        out = torch.empty((M, N // 2 if epi in (3, 4) else N), dtype=a.dtype, device=a.device)
+    _chk(out.shape == (M, N // 2 if epi in (3, 4) else N) and out.stride(1) == 1, "gemv output")
+    native().gemv(_ptr(out), _ptr(a), _ptr(w), M, N, K, a.stride(0), w.stride(0), out.stride(0),
+                  5 if bias is not None else epi, 1, _ptr(bias), _stream())
+    return out
+
+
 def sgemm(a: torch.Tensor, w: torch.Tensor, epi: int = 0, splits: int = 1,
           bias: torch.Tensor | None = None, out: torch.Tensor | None = None):
     """a @ w^T on K23 (1 to 64 rows).  epi 0 plain, 5 with ``bias``, 3 / 4 SwiGLU / ReLU-GLU over
@@ -845,8 +889,9 @@ def sgemm(a: torch.Tensor, w: torch.Tensor, epi: int = 0, splits: int = 1,
 
 def linear(x: torch.Tensor, w: torch.Tensor, defer: bool = False,
            bias: torch.Tensor | None = None, out: torch.Tensor | None = None):
-    """x @ w^T (+ bias): K23 for few rows of small weights, the decode GEMM (K11) where the measured table picks
-    it, the older split-K kernel where it was measured faster, the large-M
+    """x @ w^T (+ bias): K25 for one or two rows, K23 for few rows of small weights,
+    the decode GEMM (K11) where the measured table picks it, the older split-K
+    kernel where it was measured faster, the large-M
     GEMM (K13) for prefill-sized M where ``large_gemm_backend`` picks it, else
     hipBLASLt (bias in its epilogue).  ``defer``: the caller feeds the result to
     ``rms_norm(..., residual=)``, so a table entry for the partials-only form
@@ -863,6 +908,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, defer: bool = False,
         return _packed_product(x, w, 2 if defer and x.shape[0] <= 256 else 0, out=out)
     if x.is_cuda and x.dim() == 2:
         M, N, K = x.shape[0], w.shape[0], w.shape[1]
+        s = gemv_splits(x, w, 2 if defer and bias is None else 0, out)
+        if s is not None and pgemm_bias_ok(bias, N):
+            return gemv(x, w, 2 if defer and bias is None else 0, s, bias, out)
         s = sgemm_splits(M, N, K, 2 if defer and bias is None else 0)
         if s is not None and pgemm_operands_ok(x, w) and pgemm_bias_ok(bias, N):
             return sgemm(x, w, 2 if defer and bias is None else 0, s, bias, out)
@@ -913,6 +961,8 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, block: int,
         return _packed_product(x, w, 3, out=out)
     if x.is_cuda and x.dim() == 2:
         if block == SWIGLU16:
+            if gemv_splits(x, w, 3, out) is not None:
+                return gemv(x, w, 3, out=out)
             if (sgemm_splits(x.shape[0], w.shape[0], w.shape[1], 3) is not None
                     and pgemm_operands_ok(x, w)):
                 return sgemm(x, w, 3, out=out)
@@ -943,6 +993,8 @@ def linear_relu_glu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     else the product and the GLU kernel."""
     if x.is_cuda and x.dtype == torch.bfloat16:
         M, N, K = x.shape[0], w.shape[0], w.shape[1]
+        if x.dim() == 2 and gemv_splits(x, w, 4) is not None:
+            return gemv(x, w, 4)
         if x.dim() == 2 and sgemm_splits(M, N, K, 4) is not None and pgemm_operands_ok(x, w):
             return sgemm(x, w, 4)
         ch = dgemm_choice(M, N, K, epi=3)

@@ -249,7 +249,7 @@ def test_sgemm(M, N, K):
             torch.testing.assert_close(p.slabs.double().sum(0), y, atol=2e-5, rtol=2e-5)
 
 
-@pytest.mark.parametrize("M", [1, 8, 9, 32, 33])
+@pytest.mark.parametrize("M", [2, 3, 8, 9, 32, 33])
 def test_linear_of_few_rows(M):
     """The rule of ops.linear: both sides of its lines, with bias, deferred, strided rows."""
     for N, K in ((2048, 2048), (4096, 4096)):
@@ -261,7 +261,7 @@ def test_linear_of_few_rows(M):
             got = ops.linear(xs, w, defer=True)
             got = got.sum() if isinstance(got, ops.Partials) else got
             torch.testing.assert_close(got.double(), y, atol=2e-2, rtol=1e-2)
-            assert ops.SGEMM_CALLS[0] - n == int(M <= (32 if N == 2048 else 8))
+            assert ops.SGEMM_CALLS[0] - n == int(2 < M <= (32 if N == 2048 else 8))
             torch.testing.assert_close(ops.linear(xs, w, bias=b).double(), y + b.double(), atol=2e-2,
                                        rtol=1e-2)
 
@@ -399,3 +399,37 @@ def test_k4_partitions(ctxs, parts, Hq, Hkv, D):
         want, bound = p @ v, 2.0 ** -8 * (p @ v.abs())
         bound = 1.05 * (bound + 2.0 ** -8 * (want.abs() + bound)) + 1e-4
         assert ((out[b].double().view(Hq, 1, D) - want).abs() <= bound).all()
+
+
+# ------------------------------------------------------------ K25: one or two rows --
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("N,K", [(32, 1024), (96, 3072), (3072, 2048), (2048, 8192), (4128, 14336)])
+def test_k25(M, N, K):
+    """Every epilogue against 64 bits: fp32 sums of K products (K / 64 in turn, then 64 by halves:
+    an error of K / 64 + 6 roundings of sum |a w| at most), bf16 results."""
+    a = torch.randn(M, K + 8, device=DEV).bfloat16()[:, :K]              # rows wider than K
+    w = torch.randn(N, K, device=DEV).bfloat16() * K ** -0.5
+    z, size = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    slack = (K / 64 + 6) * 2.0 ** -24 * size
+    calls = ops.GEMV_CALLS[0]
+
+    def close(got, want, bound):
+        assert ((got.double() - want).abs() <= bound + 2.0 ** -8 * want.abs() + 1e-30).all()
+
+    close(ops.linear(a, w), z, slack)
+    b = torch.randn(N, device=DEV).bfloat16()
+    close(ops.linear(a, w, bias=b), z + b.double(), slack + 2.0 ** -23 * (z + b.double()).abs())
+    p = ops.linear(a, w, defer=True)
+    assert p.slabs.numel() == (2 if N < 4096 and K // 1024 % 2 == 0 else 1) * M * N
+    assert ((p.slabs.view(-1, M, N).double().sum(0) - z).abs() <= slack).all()
+    g, u = z.view(M, N // 32, 2, 16).unbind(2)
+    gs, us = slack.view(M, N // 32, 2, 16).unbind(2)
+    for got, act in ((ops.linear_swiglu(a, w, ops.SWIGLU16), torch.nn.functional.silu),
+                     (ops.linear_relu_glu(a, w), torch.relu)):
+        bound = 1.1 * gs * u.abs() + act(g).abs() * us + 2.0 ** -20 * (act(g) * u).abs() + 2 * gs * us
+        close(got, (act(g) * u).reshape(M, -1), bound.reshape(M, -1))
+    out = torch.zeros(M, N + 2, device=DEV).bfloat16()[:, :N]            # any even row stride
+    close(ops.linear(a, w, out=out), z, slack)
+    assert ops.GEMV_CALLS[0] == calls + 6
+    a[0, 5] = float("inf")
+    assert not ops.linear(a, w)[0].isfinite().any()
