@@ -1,4 +1,5 @@
-// K23: projection of a few rows (1 to 64) with weights of up to some tens of MB:
+// K23: projection of a few rows (1 to 64; one and two of long K: gemv.hip) with weights of up to
+// some tens of MB:
 //     C[M, N] = epi(A[M, K] . W[N, K]^T)      bf16 in, fp32 accumulate
 //
 // Such a product is bound by latencies, not by its weight stream: the decode GEMM
