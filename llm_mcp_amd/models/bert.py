@@ -102,12 +102,9 @@ class BertModel:
         ln = np.asarray(lens, dtype=np.int64)
         if int(ln.max()) > cfg.max_position:
             raise ValueError(f"sequence longer than {cfg.max_position} positions")
-        if ids.is_cuda and encoder.layers_ok(w["layers"], NATIVE, d, cfg.intermediate_size, H, D):
-            b = encoder.batch(lens, ids.device)
-            x = encoder.embed_norm(ids, w["word"], w["type"], w["emb_ln_w"], w["emb_ln_b"],
-                                   cfg.ln_eps, w["pos"], b.positions)
-            encoder.layers(x, w["layers"], NATIVE, b, cu, cfg.intermediate_size, H, D, cfg.ln_eps,
-                           self.scale, True, None)
+        r = encoder.encode(ids, cu, lens, w, NATIVE, cfg, self.scale, True) if ids.is_cuda else None
+        if r is not None:
+            x, b = r
             if cfg.pooling == "cls":     # the first tokens' rows as sequences of one
                 x, cu = ops.embed_gather(x, b.first), b.count
             return ops.mean_pool_l2(x, cu, dims or cfg.embed_dim, normalize)

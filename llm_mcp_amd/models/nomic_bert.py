@@ -110,13 +110,10 @@ class NomicBertModel:
         H, D, d = self.H, self.D, cfg.hidden_size
         T, S = ids.numel(), len(lens)
         dev = self.device
-        if ids.is_cuda and self.gu_k13 and not self.fuse_q_rope and encoder.layers_ok(
-                w["layers"], tuple(n for n in NATIVE if n), d, cfg.intermediate_size, H, D):
-            b = encoder.batch(lens, ids.device)
-            x = encoder.embed_norm(ids, w["word"], w["type"], w["emb_ln_w"], w["emb_ln_b"],
-                                   cfg.ln_eps)
-            encoder.layers(x, w["layers"], NATIVE, b, cu, cfg.intermediate_size, H, D, cfg.ln_eps,
-                           self.scale, False, self.cos_sin)
+        r = (encoder.encode(ids, cu, lens, w, NATIVE, cfg, self.scale, False, self.cos_sin)
+             if ids.is_cuda and self.gu_k13 and not self.fuse_q_rope else None)
+        if r is not None:
+            x, _ = r
             return ops.mean_pool_l2(x, cu, dims or cfg.embed_dim, normalize)
         # per-sequence page-aligned slots in a scratch paged K/V cache, built
         # with array ops (no per-token Python work on the host critical path)

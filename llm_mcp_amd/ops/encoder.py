@@ -1,11 +1,16 @@
 """The layers of an embedding encoder in one native call (csrc/kernels/encoder.hip).
 
-``batch`` lays a batch of packed sequences out (positions, attention tiles), ``layers``
-runs all layers.  The models keep their own
-loop over single ops for the CPU and for shapes and switches this one does not take.
+``encode`` is a whole forward up to the pooling: ``batch`` lays the packed sequences out
+(positions, attention tiles), ``embed_norm`` makes their rows, ``layers`` runs all layers.  The
+kernels get addresses and the configuration's sizes, so everything they read is checked
+first (``layers_ok``, ``embed_ok``).  The models keep their own loop over single ops
+for the CPU and for operands and switches this one does not take.
 """
 from __future__ import annotations
 
+import functools
+import itertools
+import operator
 import os
 from dataclasses import dataclass
 
@@ -35,9 +40,9 @@ def batch(lens, device) -> Batch:
     row0, tile0 = np.cumsum(ln) - ln, np.cumsum(nt) - nt
     NT = int(nt.sum())
     sizes = (T, 2 * NT, S, S + 1)
-    at = np.concatenate([[0], np.cumsum([-(-n // 4) * 4 for n in sizes])])
+    at = [0, *itertools.accumulate(-(-n // 4) * 4 for n in sizes)]
     cuda = device.type == "cuda"
-    host = torch.empty(int(at[-1]), dtype=torch.int32, pin_memory=cuda)
+    host = torch.empty(at[-1], dtype=torch.int32, pin_memory=cuda)
     h = host.numpy()
     pos, tiles, first, count = (h[a:a + n] for a, n in zip(at, sizes))
     pos[:] = np.arange(T, dtype=np.int32)
@@ -46,22 +51,73 @@ def batch(lens, device) -> Batch:
     tiles[1::2] = (np.arange(NT, dtype=np.int32) - np.repeat(tile0, nt)) * QUERIES
     first[:], count[:] = row0, np.arange(S + 1)
     dev = host.to(device, non_blocking=True) if cuda else host
-    return Batch(*(dev[a:a + n] for a, n in zip(at.tolist(), sizes)), int(ln.max(initial=0)))
+    return Batch(*(dev[a:a + n] for a, n in zip(at, sizes)), int(ln.max(initial=0)))
 
 
-def layers_ok(layers: list, names: tuple, d: int, I: int, H: int, D: int) -> bool:
-    """Whether the native layers run these weights: whole 256-column tiles, bf16 rows
-    as they are stored, no switch that asks for the library."""
-    if (d % 256 or I % 256 or d > 2048 or d != H * D or D != 64
-            or os.environ.get("LMX_ENCODER_LIBRARY", "0") == "1"):
-        return False
-    return all(t is not None and t.dtype is torch.bfloat16 and t.is_contiguous()
-               for L in layers for t in (L.get(n) for n in names))
+def _shapes(d: int, I: int, gelu: bool) -> tuple:
+    """Shapes of a layer's tensors in the order of encoder.h."""
+    v, w1 = (d,), I if gelu else 2 * I
+    return tuple(torch.Size(s) for s in ((3 * d, d), (3 * d,), (d, d), v, v, v, (w1, d), (w1,), (d, I),
+                                         v, v, v))
+
+
+def sizes_ok(d: int, I: int, H: int, D: int, gelu: bool) -> bool:
+    """Whether the native layers run an encoder of these sizes: whole 256-column tiles, a bias
+    that K13 holds, no switch that asks for the library."""
+    from . import PGEMM_MAX_BIAS
+    return (d % 256 == 0 and I % 256 == 0 and d <= 2048 and d == H * D and D == 64
+            and not (gelu and I > PGEMM_MAX_BIAS) and os.environ.get("LMX_ENCODER_LIBRARY", "0") != "1")
+
+
+def layers_ok(layers: list, names: tuple, d: int, I: int, gelu: bool) -> list | None:
+    """Addresses of the layers' weights, ``names`` of them a layer (None: the model has none
+    there), if all are bf16 tensors of the configuration's shapes as they are stored, on 16
+    bytes.  Else None: the models' own loop takes or refuses them."""
+    want, bf16, out = list(zip(names, _shapes(d, I, gelu))), torch.bfloat16, []
+    for L in layers:
+        for n, shape in want:
+            if n is None:
+                out.append(0)
+                continue
+            t = L.get(n)
+            if t is None or t.dtype is not bf16 or t.shape != shape or not t.is_contiguous():
+                return None
+            out.append(t.data_ptr())
+    return None if functools.reduce(operator.or_, out, 0) & 15 else out
+
+
+def _rows_ok(t: torch.Tensor, cols: int, dims: int = 2) -> bool:
+    return (t.dtype is torch.bfloat16 and t.dim() == dims and t.shape[-1] == cols and t.is_contiguous()
+            and t.data_ptr() % 16 == 0)
+
+
+def _index_ok(t: torch.Tensor, n: int, device: torch.device) -> bool:
+    return (t.dtype is torch.int32 and t.dim() == 1 and t.numel() == n and t.is_contiguous()
+            and t.device == device)
+
+
+def embed_ok(ids: torch.Tensor, word: torch.Tensor, type_row: torch.Tensor, w, b,
+             pos: torch.Tensor | None = None, positions: torch.Tensor | None = None) -> bool:
+    """Whether ``embed_norm`` reads these: int32 indices, contiguous bf16 tables and vectors of
+    one width on 16 bytes."""
+    d = word.shape[-1]
+    return (_index_ok(ids, ids.numel(), word.device) and _rows_ok(word, d) and d % 8 == 0 and d <= 2048
+            and _rows_ok(type_row, d) and type_row.shape[0] > 0 and _rows_ok(w, d, 1) and _rows_ok(b, d, 1)
+            and (pos is None or _rows_ok(pos, d))
+            and (positions is None or _index_ok(positions, ids.numel(), word.device)))
 
 
 def embed_norm(ids: torch.Tensor, word: torch.Tensor, type_row: torch.Tensor, w, b, eps: float,
                pos: torch.Tensor | None = None, positions: torch.Tensor | None = None) -> torch.Tensor:
-    """LayerNorm(word[ids] + type (+ pos[positions])), bf16 rows."""
+    """LayerNorm(word[ids] + type (+ pos[positions])), bf16 rows.  ``positions`` are the caller's
+    to keep below pos's rows."""
+    from . import _chk
+    _chk(embed_ok(ids, word, type_row, w, b, pos, positions)
+         and (pos is None or positions is not None), "embed_norm operands")
+    return _embed_norm(ids, word, type_row, w, b, eps, pos, positions)
+
+
+def _embed_norm(ids, word, type_row, w, b, eps, pos, positions) -> torch.Tensor:
     from . import _ptr, _stream, native
     out = torch.empty((ids.numel(), word.shape[1]), dtype=word.dtype, device=word.device)
     native().embed_layernorm(_ptr(out), _ptr(ids), _ptr(word), word.shape[0], _ptr(type_row), _ptr(pos),
@@ -70,14 +126,33 @@ def embed_norm(ids: torch.Tensor, word: torch.Tensor, type_row: torch.Tensor, w,
     return out
 
 
-def layers(x: torch.Tensor, weights: list, names: tuple, b: Batch, cu: torch.Tensor, I: int, H: int,
-           D: int, eps: float, scale: float, gelu: bool,
-           cos_sin: torch.Tensor | None) -> torch.Tensor:
-    """All layers over x [T, d], in place.  ``names``: a layer's tensors in the order of
-    encoder.h (None: the model has none there)."""
-    from . import PGEMM_CALLS, _chk, _ptr, _stream, native, pgemm_counters
+def encode(ids: torch.Tensor, cu: torch.Tensor, lens: list, w: dict, names: tuple, cfg, scale: float,
+           gelu: bool, cos_sin: torch.Tensor | None = None) -> tuple | None:
+    """(rows [T, d] after all layers, their ``Batch``) of packed sequences, or None where the
+    native layers do not take these operands (the models' own loop takes or refuses them).
+    ``cos_sin``: rotary tables; without them w["pos"] holds a row for every position."""
+    from . import _chk
+    d, I, H, D = cfg.hidden_size, cfg.intermediate_size, cfg.num_heads, cfg.head_dim
+    word, pos = w["word"], None if cos_sin is not None else w["pos"]
+    if not (sizes_ok(d, I, H, D, gelu) and word.shape[-1] == d and sum(lens) == ids.numel()
+            and _index_ok(cu, len(lens) + 1, ids.device)
+            and embed_ok(ids, word, w["type"], w["emb_ln_w"], w["emb_ln_b"], pos)):
+        return None
+    b = batch(lens, ids.device)
+    _chk(b.longest <= (pos if cos_sin is None else cos_sin).shape[0],
+         "a sequence is longer than the position table")
+    x = _embed_norm(ids, word, w["type"], w["emb_ln_w"], w["emb_ln_b"], cfg.ln_eps, pos,
+                    b.positions if pos is not None else None)
+    # here, while the upload and the first norm run (50 us for 12 layers)
+    ptrs = layers_ok(w["layers"], names, d, I, gelu)
+    return (layers(x, ptrs, b, cu, I, H, D, cfg.ln_eps, scale, gelu, cos_sin), b) if ptrs else None
+
+
+def layers(x: torch.Tensor, ptrs: list, b: Batch, cu: torch.Tensor, I: int, H: int, D: int, eps: float,
+           scale: float, gelu: bool, cos_sin: torch.Tensor | None) -> torch.Tensor:
+    """All layers over x [T, d], in place.  ``ptrs``: ``layers_ok``'s."""
+    from . import PGEMM_CALLS, _ptr, _stream, native, pgemm_counters
     T, d = x.shape
-    _chk(cos_sin is None or b.longest <= cos_sin.shape[0], "a sequence is longer than cos_sin")
     dev, n = x.device, native().enc_slab_floats(T, d, I)
     rows = torch.empty(T * (5 * d + I), dtype=x.dtype, device=dev)       # h, attn, qkv, g
     at = [0, T * d, 2 * T * d, 5 * T * d]
@@ -87,12 +162,11 @@ def layers(x: torch.Tensor, weights: list, names: tuple, b: Batch, cu: torch.Ten
         tail = 0               # see ops.pgemm_tail
     slabs = torch.empty(n + tail, dtype=torch.float32, device=dev)
     cnt = pgemm_counters(dev) if tail else None
-    ptrs = [0 if k is None else L[k].data_ptr() for L in weights for k in names]
     native().encoder_layers(
         ptrs, T, d, I, H, D, gelu, float(eps), float(scale), _ptr(x), h, qkv, attn, g, _ptr(slabs), n,
         _ptr(cos_sin), _ptr(cu), _ptr(b.tiles), b.tiles.numel() // 2,
         _ptr(slabs) + 4 * n if tail else 0, tail, _ptr(cnt), _stream())
-    PGEMM_CALLS[0] += 4 * len(weights)
+    PGEMM_CALLS[0] += 4 * (len(ptrs) // 12)
     return x
 
 

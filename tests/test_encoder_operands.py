@@ -1,0 +1,118 @@
+"""Which operands the encoders' native layers take (ops.encoder): the kernels get addresses and the
+configuration's sizes, so all others go to the models' own loop or are refused."""
+import types
+
+import pytest
+import torch
+
+from llm_mcp_amd.models import bert, nomic_bert
+from llm_mcp_amd.ops import encoder
+
+D, I, V, P = 256, 512, 40, 20
+LENS = [7, 1, 12]
+
+
+def _zeros(*shape):
+    return torch.zeros(shape, dtype=torch.bfloat16)
+
+
+def _model(gelu):
+    names = bert.NATIVE if gelu else nomic_bert.NATIVE
+    shapes = encoder._shapes(D, I, gelu)
+    return names, dict(word=_zeros(V, D), type=_zeros(2, D), pos=_zeros(P, D), emb_ln_w=_zeros(D),
+                       emb_ln_b=_zeros(D),
+                       layers=[{n: _zeros(*s) for n, s in zip(names, shapes) if n} for _ in range(2)])
+
+
+def _ok(names, w, gelu):
+    return encoder.layers_ok(w["layers"], names, D, I, gelu)
+
+
+def _encode(names, w, gelu, ids=None, cu=None, lens=LENS, rows=P):
+    cfg = types.SimpleNamespace(hidden_size=D, intermediate_size=I, num_heads=D // 64, head_dim=64,
+                                ln_eps=1e-12)
+    ids = torch.zeros(sum(LENS), dtype=torch.int32) if ids is None else ids
+    cu = torch.tensor([0, 7, 8, 20], dtype=torch.int32) if cu is None else cu
+    return encoder.encode(ids, cu, lens, w, names, cfg, 0.125, gelu,
+                          None if gelu else torch.zeros(rows, 64))
+
+
+class _Reached(Exception):
+    pass
+
+
+@pytest.fixture
+def reached(monkeypatch):
+    """The kernels' place: says that all checks were passed."""
+    def stop(*a):
+        raise _Reached
+    monkeypatch.setattr(encoder, "_embed_norm", lambda *a: None)
+    monkeypatch.setattr(encoder, "layers", stop)
+
+
+@pytest.mark.parametrize("gelu", [True, False])
+def test_layers(gelu, reached):
+    names, w = _model(gelu)
+    addresses = _ok(names, w, gelu)
+    assert addresses == [0 if n is None else L[n].data_ptr() for L in w["layers"] for n in names]
+    with pytest.raises(_Reached):
+        _encode(names, w, gelu)
+    for n in filter(None, names):
+        t = w["layers"][1][n]
+        small = t[:-16].clone()                                    # fewer rows than the configuration says
+        off = torch.zeros(t.numel() + 8, dtype=t.dtype)
+        off = off[-off.data_ptr() // 2 % 8 + 1:][:t.numel()].view(t.shape)          # 2 bytes off a boundary
+        bad = [None, small, t.float(), off]
+        if t.dim() == 2:
+            bad += [t[:, :-64].contiguous(), _zeros(t.shape[1], t.shape[0]).t(), t[:, :-64]]
+        for b in bad:
+            w["layers"][1][n] = b
+            assert _ok(names, w, gelu) is None and _encode(names, w, gelu) is None, n
+        w["layers"][1][n] = t
+
+
+def test_bias_wider_than_k13_holds():
+    assert encoder.sizes_ok(D, 14336, D // 64, 64, True) and not encoder.sizes_ok(D, 14592, D // 64, 64, True)
+    assert encoder.sizes_ok(D, 14592, D // 64, 64, False)
+
+
+@pytest.mark.parametrize("gelu", [True, False])
+def test_embedding_and_indices(gelu, reached):
+    names, w = _model(gelu)
+    wide = torch.zeros(V, D + 8, dtype=torch.bfloat16)[:, :D]
+    for n, bad in (("word", [w["word"].float(), wide, _zeros(V, D - 8)]), ("type", [w["type"].float()]),
+                   ("emb_ln_w", [w["emb_ln_w"].float(), _zeros(D - 8)]), ("emb_ln_b", [_zeros(D + 8)]),
+                   ("pos", [w["pos"].float(), wide])):
+        if n == "pos" and not gelu:
+            continue
+        keep = w[n]
+        for b in bad:
+            w[n] = b
+            assert _encode(names, w, gelu) is None, n
+        w[n] = keep
+    ids, cu = torch.zeros(sum(LENS), dtype=torch.int32), torch.tensor([0, 7, 8, 20], dtype=torch.int32)
+    for kw in (dict(ids=ids.long()), dict(ids=ids[:-1]), dict(ids=torch.zeros(40, dtype=torch.int32)[::2]),
+               dict(cu=cu.long()), dict(cu=cu[:-1]), dict(lens=[7, 1, 13])):
+        assert _encode(names, w, gelu, **kw) is None, kw
+
+
+@pytest.mark.parametrize("gelu", [True, False])
+def test_positions_within_their_table(gelu, reached):
+    """A sequence longer than the positions' table is refused, not read past the table's end."""
+    names, w = _model(gelu)
+    w["pos"] = _zeros(11, D)
+    with pytest.raises(ValueError):
+        _encode(names, w, gelu, rows=11)
+    w["pos"] = _zeros(12, D)
+    with pytest.raises(_Reached):
+        _encode(names, w, gelu, rows=12)
+
+
+def test_embed_norm_refuses():
+    _, w = _model(True)
+    ids = torch.zeros(5, dtype=torch.int32)
+    args = [ids, w["word"], w["type"], w["emb_ln_w"], w["emb_ln_b"], 1e-12, w["pos"], ids]
+    for i, bad in ((0, ids.long()), (1, w["word"].float()), (2, w["type"][:0]), (3, w["emb_ln_w"][1:]),
+                   (6, w["pos"].float()), (7, ids.long()), (7, ids[:-1]), (7, None)):
+        with pytest.raises(ValueError):
+            encoder.embed_norm(*args[:i], bad, *args[i + 1:])
