@@ -794,6 +794,51 @@ def _into(out: torch.Tensor | None, y: torch.Tensor) -> torch.Tensor:
     return out.copy_(y)
 
 
+def _by_address(*ts) -> bool:
+    """Kernels may take these tensors by address: plain ones that no gradient, functorch transform
+    or tracer follows."""
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts):
+        return False
+    return (torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0
+            and torch.autograd.forward_ad._current_level < 0
+            and all(t is None or type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts))
+
+
+def few_rows_ok(x: torch.Tensor, w: torch.Tensor, epi: int = 0, bias: torch.Tensor | None = None,
+                out: torch.Tensor | None = None, step: int = 4) -> bool:
+    """Operands that K25 and K23 read and a destination that they write in pieces of ``step``
+    elements.  All others keep the route they have without these kernels."""
+    M, N = x.shape[0], w.shape[0]
+    if (N == 0 or w.shape[1] == 0 or x.shape[1] != w.shape[1] or not _by_address(x, w, bias, out)
+            or not pgemm_operands_ok(x, w) or not pgemm_bias_ok(bias, N)
+            or any(t is not None and t.device != x.device for t in (w, bias, out))):
+        return False
+    if out is None:
+        return True
+    ncols = N // 2 if epi in (3, 4) else N
+    return (out.dtype == x.dtype and out.shape == (M, ncols) and out.stride(1) == 1
+            and out.stride(0) % step == 0 and (M == 1 or out.stride(0) >= ncols)
+            and out.data_ptr() % (2 * step) == 0
+            and not any(t is not None and t.untyped_storage().data_ptr() == out.untyped_storage().data_ptr()
+                        for t in (x, w, bias)))     # read while it is written
+
+
+def few_rows(x: torch.Tensor, w: torch.Tensor, epi: int = 0, bias: torch.Tensor | None = None,
+             out: torch.Tensor | None = None):
+    """x @ w^T on K25 or K23 (``epi``: theirs) where they take it, else None."""
+    M, N, K = x.shape[0], w.shape[0], w.shape[1]
+    if M > SGEMM_MAX_M:
+        return None
+    s = gemv_splits(x, w, epi, out)
+    if s is not None and few_rows_ok(x, w, epi, bias, out, 2):
+        return gemv(x, w, epi, s, bias, out)
+    s = sgemm_splits(M, N, K, epi)
+    if s is not None and few_rows_ok(x, w, epi, bias, out):
+        return sgemm(x, w, epi, s, bias, out)
+    return None
+
+
 # K23 (csrc/kernels/sgemm.hip), few rows and small weights: elements of W up to which it
 # beats the tables' kernels on cold weights. Llama-3.2-1B at 1 / 16 / 32 rows: QKV (6.3 M) 5.4 / 6.7 /
 # 8.7 us against 11.2 / 11.4 / 11.6, O (4.2 M) 4.1 / 4.7 / 5.7 against 7.1 / 7.3 / 7.0, and at 64
@@ -908,12 +953,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, defer: bool = False,
         return _packed_product(x, w, 2 if defer and x.shape[0] <= 256 else 0, out=out)
     if x.is_cuda and x.dim() == 2:
         M, N, K = x.shape[0], w.shape[0], w.shape[1]
-        s = gemv_splits(x, w, 2 if defer and bias is None else 0, out)
-        if s is not None and pgemm_bias_ok(bias, N):
-            return gemv(x, w, 2 if defer and bias is None else 0, s, bias, out)
-        s = sgemm_splits(M, N, K, 2 if defer and bias is None else 0)
-        if s is not None and pgemm_operands_ok(x, w) and pgemm_bias_ok(bias, N):
-            return sgemm(x, w, 2 if defer and bias is None else 0, s, bias, out)
+        y = few_rows(x, w, 2 if defer and bias is None else 0, bias, out)
+        if y is not None:
+            return y
         if bias is None:
             rc = rs_choice(M, N, K, epi=2 if defer else 0, w=w)
             if rc is not None and rsgemm_operands_ok(x, w):
@@ -961,11 +1003,9 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, block: int,
         return _packed_product(x, w, 3, out=out)
     if x.is_cuda and x.dim() == 2:
         if block == SWIGLU16:
-            if gemv_splits(x, w, 3, out) is not None:
-                return gemv(x, w, 3, out=out)
-            if (sgemm_splits(x.shape[0], w.shape[0], w.shape[1], 3) is not None
-                    and pgemm_operands_ok(x, w)):
-                return sgemm(x, w, 3, out=out)
+            y = few_rows(x, w, 3, out=out)
+            if y is not None:
+                return y
             rc = rs_choice(x.shape[0], w.shape[0], w.shape[1], epi=3, w=w)
             if rc is not None and rsgemm_operands_ok(x, w):
                 return rsgemm(x, w, rc[0], rc[1], epi=3, out=out)     # K14, SwiGLU epilogue
@@ -993,10 +1033,9 @@ def linear_relu_glu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     else the product and the GLU kernel."""
     if x.is_cuda and x.dtype == torch.bfloat16:
         M, N, K = x.shape[0], w.shape[0], w.shape[1]
-        if x.dim() == 2 and gemv_splits(x, w, 4) is not None:
-            return gemv(x, w, 4)
-        if x.dim() == 2 and sgemm_splits(M, N, K, 4) is not None and pgemm_operands_ok(x, w):
-            return sgemm(x, w, 4)
+        y = few_rows(x, w, 4) if x.dim() == 2 else None
+        if y is not None:
+            return y
         ch = dgemm_choice(M, N, K, epi=3)
         if ch is not None and ch[0] >= 0 and swiglu16_ok(ch[0]):
             return dgemm(x, w, ch[0], ch[1], epi=4)

@@ -34,3 +34,39 @@ def test_layouts():
     assert ops.gemv_splits(x, w, 0, _rows(2, 64, 67)) is None
     assert ops.gemv_splits(x, w, 0, _rows(2, 64, 66, offset=1)) is None
     assert ops.gemv_splits(x, w, 0, _rows(64, 2).t()) is None
+
+
+@pytest.mark.parametrize("step", [2, 4])
+def test_operands_and_destinations(step):
+    """What K25 and K23 leave to the routes that stood before them: other types, layouts and devices,
+    destinations that they cannot write whole or that are read meanwhile, empty products."""
+    x, w = _rows(2, 1024), _rows(64, 1024)
+    ok = lambda *a, **k: ops.few_rows_ok(*a, **k, step=step)
+    assert ok(x, w) and ok(x, w, 0, _rows(1, 64)[0], _rows(2, 64, 72))
+    assert ok(x, w, 3, None, _rows(2, 32, 36)) and not ok(x, w, 3, None, _rows(2, 64))
+    assert not ok(x, w, 0, torch.zeros(64)) and not ok(x, w, 0, _rows(1, 32)[0])
+    assert not ok(_rows(2, 512), w)
+    assert not ok(x, w[:0]) and not ok(x[:, :0], w[:, :0])
+    for out in (torch.zeros(2, 64), _rows(2, 64, 65), _rows(2, 64, offset=1), _rows(64, 2).t(),
+                _rows(1, 64).expand(2, 64), _rows(3, 64), torch.empty(2, 64, dtype=torch.bfloat16, device="meta")):
+        assert not ok(x, w, 0, None, out)
+    assert ok(x, w, 0, None, _rows(2, 64, 66)) == (step == 2)
+    assert ok(x, w, 0, None, _rows(2, 64, offset=2)) == (step == 2)
+    assert not ok(x, w, 0, None, x[:, :64]) and not ok(x, w, 0, None, w[:2, :64])      # read meanwhile
+    assert not ok(x, w.to("meta"))
+
+
+def test_gradients_and_transforms():
+    x, w = _rows(2, 1024), _rows(64, 1024)
+    g = w.clone().requires_grad_()
+    assert not ops.few_rows_ok(x, g) and not ops.few_rows_ok(x.clone().requires_grad_(), w)
+    with torch.no_grad():
+        assert ops.few_rows_ok(x, torch.nn.Parameter(w))
+    assert ops.few_rows_ok(x, torch.nn.Parameter(w, requires_grad=False))
+    seen = []
+    torch.vmap(lambda a: (seen.append(ops.few_rows_ok(a, w)), a)[1])(x[None])
+    with torch._subclasses.fake_tensor.FakeTensorMode() as mode:
+        seen.append(ops.few_rows_ok(torch.empty(2, 1024, dtype=torch.bfloat16), mode.from_tensor(w)))
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(ops.few_rows_ok(torch.autograd.forward_ad.make_dual(x, x), w))
+    assert seen == [False] * 3

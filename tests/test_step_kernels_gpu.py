@@ -433,3 +433,32 @@ def test_k25(M, N, K):
     assert ops.GEMV_CALLS[0] == calls + 6
     a[0, 5] = float("inf")
     assert not ops.linear(a, w)[0].isfinite().any()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 96, 1024), (2, 96, 1024), (3, 96, 1024), (32, 96, 96), (4, 96, 160)])
+def test_few_rows_destinations(M, N, K):
+    """Any destination that torch writes: odd rows and offsets, other types, the operands' own memory;
+    gradients; empty products.  Two roundings to bf16 at most (product, sum with a bias)."""
+    a, w = torch.randn(M, K, device=DEV).bfloat16(), torch.randn(N, K, device=DEV).bfloat16() * K ** -0.5
+    y, tol = a.double() @ w.double().t(), dict(atol=4e-3, rtol=2.0 ** -8)
+    buf = torch.zeros(M, N + 3, device=DEV).bfloat16()
+    wide = torch.zeros(M, 2 * N, device=DEV).bfloat16()
+    for out in (buf[:, 1:N + 1], buf[:, :N], buf[:, 2:N + 2], wide[:, ::2], torch.zeros(M, N, device=DEV),
+                torch.zeros(N, M, device=DEV).bfloat16().t()):
+        got = ops.linear(a, w, out=out)
+        torch.testing.assert_close(got.double(), y, **tol)
+        torch.testing.assert_close(out.double(), y, **tol)
+    both = torch.cat([a, torch.zeros(M, N, device=DEV).bfloat16()], 1)
+    at = both.clone()
+    ops.linear(at[:, :K], w, out=at[:, :N])                        # over its own rows
+    torch.testing.assert_close(at[:, :N].double(), y, **tol)
+    g = torch.zeros(M, N // 2 + 1, device=DEV).bfloat16()[:, 1:]
+    p, q = y.view(M, N // 32, 2, 16).unbind(2)
+    ops.linear_swiglu(a, w, ops.SWIGLU16, out=g)
+    torch.testing.assert_close(g.double(), (torch.nn.functional.silu(p) * q).reshape(M, -1), atol=2e-2,
+                               rtol=2.0 ** -6)
+    v = w.clone().requires_grad_()
+    ops.linear(a, v).float().sum().backward()
+    torch.testing.assert_close(v.grad.double(), a.double().sum(0).expand(N, K), atol=1e-2 * M, rtol=1e-2)
+    assert ops.linear(a, w[:0]).shape == (M, 0)
+    assert not ops.linear(a[:, :0], w[:, :0]).any()
