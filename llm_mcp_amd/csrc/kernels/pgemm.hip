@@ -59,7 +59,9 @@
 #include "common.h"
 
 #include <algorithm>
+#include <array>
 #include <cmath>
+#include <vector>
 
 namespace lmx {
 namespace {
@@ -468,6 +470,40 @@ __device__ __forceinline__ void pp_step(PpRegs& R, char* smem, int stage, const 
 constexpr int PG_TSLAB = PG_THREADS * 128;        // floats of a piece's tile
 constexpr int PG_TAIL_SLOTS = 16;                 // pieces of the tiles that 8 workgroups share
 
+// The last round in pieces: the workgroups slot, row + slot, .. (one of each XCD j) take the
+// tiles slot, row + slot, .. of it, the K-steps of those tiles one after the other cut into
+// `share` equal parts, the j-th one [s, e).  The workgroups of an XCD are then at the
+// same K of neighbouring tiles, as in the other rounds, and share their panels in its L2 (parts in
+// tile order, which start at as many K as there are workgroups, ran slower than whole tiles).
+struct PgLast {
+  int row, j, slot, first;       // first: the round's first tile
+  int steps, s, e;
+};
+__host__ __device__ inline PgLast pg_last(int G, int r, int ntiles, int nk, int share) {
+  PgLast l;
+  l.row = G >> 3;                // launched on whole XCDs (pg_tail_share)
+  l.j = r / l.row;
+  l.slot = r - l.j * l.row;
+  l.first = ntiles / G * G;
+  l.steps = (ntiles - l.first + l.row - 1) / l.row * nk;
+  l.s = l.j < share ? l.j * l.steps / share : 0;
+  l.e = l.j < share ? (l.j + 1) * l.steps / share : 0;
+  return l;
+}
+// the piece of a part that starts at its step s: K-steps [kb, ke) of tile lin (>= ntiles: none)
+struct PgPiece { int lin, kb, ke; };
+__host__ __device__ inline PgPiece pg_piece(const PgLast& l, int s, int nk) {
+  const int t = s / nk, kb = s - t * nk, left = l.e - s;
+  return {l.first + t * l.row + l.slot, kb, nk - kb < left ? nk : kb + left};
+}
+// the parts j0 .. j1 that hold pieces of tile lin, in K order, and the slab of the first
+struct PgPieces { int j0, j1, slab; };
+__host__ __device__ inline PgPieces pg_pieces(const PgLast& l, int lin, int nk, int share) {
+  const int t = (lin - l.first) / l.row;
+  const int j0 = ((t * nk + 1) * share - 1) / l.steps, j1 = ((t + 1) * nk * share - 1) / l.steps;
+  return {j0, j1, l.slot * PG_TAIL_SLOTS + j0 + t};
+}
+
 // Joins the fp32 tiles of np pieces (slabs one after the other, in K order; this
 // workgroup has piece p): all but the last to arrive publish theirs write-through
 // (sc1) in the lane-native order -- accumulator r = ((qm * 2 + qn) * 4 + i) * 2 + j of
@@ -650,16 +686,10 @@ __global__ void __launch_bounds__(PG_THREADS, 1) pgemm_pp2_kernel(
   // workgroup's whole tiles are one run; a piece of a tile of the last round is another
   // (count 1), each behind a drained pipeline.
   int lin = r, count = my_tiles, kb = 0, ke = nk;
-  // The last round: the workgroups slot, row + slot, .. (one of each XCD j) take the tiles
-  // slot, row + slot, .. of it, the K-steps of those tiles one after the other cut into equal parts.
-  // The workgroups of an XCD are then at the same K of neighbouring tiles, as in
-  // the other rounds, and share their panels in its L2 (parts in tile order, which start at
-  // as many K as there are workgroups, ran slower than whole tiles).
-  const int row = G >> 3, j = r / row, slot = r - j * row;
-  const int first = ntiles / G * G, most = cut ? (ntiles - first + row - 1) / row : 0;
-  const int steps = most * nk, P = tail.share;
-  int s = j < P ? j * steps / P : 0;
-  const int e = j < P ? (j + 1) * steps / P : 0;
+  // an uncut product may run on fewer than 8 workgroups: no rows of XCDs there
+  PgLast last{};
+  if (cut) last = pg_last(G, r, ntiles, nk, tail.share);
+  int s = last.s;
   auto advance = [&](PgLoad& L) {
     if (L.done) return;
     if (++L.k == ke) {
@@ -680,13 +710,14 @@ __global__ void __launch_bounds__(PG_THREADS, 1) pgemm_pp2_kernel(
   PgOut O;
   for (bool piece = false;; piece = true) {
     if (piece || count == 0) {
-      const int t = cut ? s / nk : 0;
-      lin = first + t * row + slot;
-      if (s >= e || lin >= ntiles) return;
+      if (!cut || s >= last.e) return;
+      const PgPiece p = pg_piece(last, s, nk);
+      if (p.lin >= ntiles) return;
       piece = true;
       count = 1;
-      kb = s - t * nk;
-      ke = min(nk, kb + e - s);
+      lin = p.lin;
+      kb = p.kb;
+      ke = p.ke;
       // no load or store of the run before is counted by the waits that follow
       pg_vmwait<0>();
       pg_barrier();
@@ -755,11 +786,9 @@ __global__ void __launch_bounds__(PG_THREADS, 1) pgemm_pp2_kernel(
     if constexpr (WP != 2) {
       if (piece) {
         s += ke - kb;
-        // the tile's pieces: XCDs j0 .. j1 in K order
-        const int t = (lin - first) / row;
-        const int j0 = ((t * nk + 1) * P - 1) / steps, j1 = ((t + 1) * nk * P - 1) / steps;
-        if (j1 > j0 && !pg_join(R, smem, tail.slabs + (long)(slot * PG_TAIL_SLOTS + j0 + t) * PG_TSLAB,
-                                tail.cnt + 2 * (lin - first), j - j0, j1 - j0 + 1))
+        const PgPieces p = pg_pieces(last, lin, nk, tail.share);
+        if (p.j1 > p.j0 && !pg_join(R, smem, tail.slabs + (long)p.slab * PG_TSLAB,
+                                    tail.cnt + 2 * (lin - last.first), last.j - p.j0, p.j1 - p.j0 + 1))
           continue;
       }
     }
@@ -989,6 +1018,23 @@ static int pg_tail_share(int M, int N, int K) {
     }
   }
   return best;
+}
+
+// every piece of the last round as the kernel walks it: {workgroup, tile, first K-step, end, slab,
+// its place among the tile's pieces, their number} (for tests)
+std::vector<std::array<int, 7>> pgemm_last_round(int G, int ntiles, int nk, int share) {
+  std::vector<std::array<int, 7>> out;
+  for (int r = 0; r < G && share > 0; ++r) {
+    const PgLast l = pg_last(G, r, ntiles, nk, share);
+    for (int s = l.s; s < l.e;) {
+      const PgPiece p = pg_piece(l, s, nk);
+      if (p.lin >= ntiles) break;
+      const PgPieces q = pg_pieces(l, p.lin, nk, share);
+      out.push_back({r, p.lin, p.kb, p.ke, q.slab + l.j - q.j0, l.j - q.j0, q.j1 - q.j0 + 1});
+      s += p.ke - p.kb;
+    }
+  }
+  return out;
 }
 
 // floats of pieces' tiles that pgemm takes for its last round (0: it runs whole tiles only)

@@ -310,6 +310,14 @@ def test_k13_last_round(M, N, K, cut):
     assert not any(int(c.abs().sum()) for c in ops._PG_COUNTERS.values())
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 256, 192), (300, 256, 256), (513, 512, 768), (257, 768, 832)])
+def test_k13_on_fewer_workgroups_than_xcds(M, N, K):
+    """1 to 6 whole tiles, a workgroup each."""
+    assert ops.native().pgemm_tail_floats(M, N, K) == 0 and -(-M // 256) * (N // 256) < 8
+    a, w = _k13(M, N, K)
+    torch.testing.assert_close(ops.pgemm(a, w).float(), a.float() @ w.float().t(), atol=4e-3, rtol=2.0 ** -7)
+
+
 def test_k13_under_capture():
     """A captured product runs whole tiles and replays beside eager ones."""
     a, w = _k13(2048, 4096, 4096)
