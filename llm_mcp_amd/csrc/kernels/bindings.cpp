@@ -151,6 +151,7 @@ int dgemm_sk_pieces(int, int, int, int, int);
 int pgemm(void*, const void*, const void*, const void*, int, int, int, long, long, long, int, int, int,
           int, float*, hipStream_t, float*, unsigned*);
 long pgemm_tail_floats(int, int, int);
+std::pair<int, long> pgemm_tail_plan(int, int, int, int);
 std::vector<std::array<int, 7>> pgemm_last_round(int, int, int, int);
 int row_scale(float*, const float*, int, const void*, long, int, int, float, hipStream_t);
 int pgemm_sk(void*, const void*, const void*, void*, void*, int, int, int, int, long, long, long,
@@ -673,6 +674,7 @@ PYBIND11_MODULE(_lmx_kernels, m) {
      py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg("slabs") = 0,
      py::arg("cnt") = 0);
   m.def("pgemm_tail_floats", &lmx::pgemm_tail_floats);
+  m.def("pgemm_tail_plan", &lmx::pgemm_tail_plan);
   m.def("pgemm_last_round", &lmx::pgemm_last_round);
   m.def("row_scale", [](uptr s, uptr part, int np, uptr x, long x_stride, int M, int cols,
                         float eps, uptr stream) {

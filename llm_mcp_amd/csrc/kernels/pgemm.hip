@@ -468,7 +468,6 @@ __device__ __forceinline__ void pp_step(PpRegs& R, char* smem, int stage, const 
 }
 
 constexpr int PG_TSLAB = PG_THREADS * 128;        // floats of a piece's tile
-constexpr int PG_TAIL_SLOTS = 16;                 // pieces of the tiles that 8 workgroups share
 
 // The last round in pieces: the workgroups slot, row + slot, .. (one of each XCD j) take the
 // tiles slot, row + slot, .. of it, the K-steps of those tiles one after the other cut into
@@ -477,7 +476,7 @@ constexpr int PG_TAIL_SLOTS = 16;                 // pieces of the tiles that 8 
 // tile order, which start at as many K as there are workgroups, ran slower than whole tiles).
 struct PgLast {
   int row, j, slot, first;       // first: the round's first tile
-  int steps, s, e;
+  int most, steps, s, e;         // most: tiles of a row of workgroups
 };
 __host__ __device__ inline PgLast pg_last(int G, int r, int ntiles, int nk, int share) {
   PgLast l;
@@ -485,7 +484,8 @@ __host__ __device__ inline PgLast pg_last(int G, int r, int ntiles, int nk, int 
   l.j = r / l.row;
   l.slot = r - l.j * l.row;
   l.first = ntiles / G * G;
-  l.steps = (ntiles - l.first + l.row - 1) / l.row * nk;
+  l.most = (ntiles - l.first + l.row - 1) / l.row;
+  l.steps = l.most * nk;
   l.s = l.j < share ? l.j * l.steps / share : 0;
   l.e = l.j < share ? (l.j + 1) * l.steps / share : 0;
   return l;
@@ -496,12 +496,15 @@ __host__ __device__ inline PgPiece pg_piece(const PgLast& l, int s, int nk) {
   const int t = s / nk, kb = s - t * nk, left = l.e - s;
   return {l.first + t * l.row + l.slot, kb, nk - kb < left ? nk : kb + left};
 }
+// slabs of a row of workgroups: a tile after the first shares a part with the one before it,
+// each with a piece of its own
+__host__ __device__ inline int pg_row_slabs(int most, int share) { return share + most - 1; }
 // the parts j0 .. j1 that hold pieces of tile lin, in K order, and the slab of the first
 struct PgPieces { int j0, j1, slab; };
 __host__ __device__ inline PgPieces pg_pieces(const PgLast& l, int lin, int nk, int share) {
   const int t = (lin - l.first) / l.row;
   const int j0 = ((t * nk + 1) * share - 1) / l.steps, j1 = ((t + 1) * nk * share - 1) / l.steps;
-  return {j0, j1, l.slot * PG_TAIL_SLOTS + j0 + t};
+  return {j0, j1, l.slot * pg_row_slabs(l.most, share) + j0 + t};
 }
 
 // Joins the fp32 tiles of np pieces (slabs one after the other, in K order; this
@@ -999,14 +1002,14 @@ static int pg_cus() {
 // 18688 x 4096 (2.3 rounds) 262 and 241; 6464 x 4096 x 14336 (1.6) 600 and 550; 600 x 4096 x
 // 14336 (48 tiles) 214 and 107.  Not cut, since it lost or made no difference: 600 x 6144 x
 // 4096, 5000 x 768 x 3072, 7680 x 4096 x 14336 (1.9), 7680 x 28672 x 4096 (13.1).
-static int pg_tail_share(int M, int N, int K) {
-  if (pg_cus() == 0 || g_pg_cus % 8 || g_pg_cus > 256) return 0;
-  const int row = g_pg_cus / 8, nk = K / 64;
+static int pg_tail_share(int M, int N, int K, int cus) {
+  if (cus <= 0 || cus % 8 || cus > 256) return 0;
+  const int row = cus / 8, nk = K / 64;
   const long tiles = (long)((M + 255) / 256) * (N / 256);
-  const int rest = (int)(tiles % g_pg_cus), most = (rest + row - 1) / row;
-  const float whole = nk * (0.92f + 0.35f * rest / g_pg_cus) + (tiles > g_pg_cus ? 3.f : -7.f);
+  const int rest = (int)(tiles % cus), most = (rest + row - 1) / row;
+  const float whole = nk * (0.92f + 0.35f * rest / cus) + (tiles > cus ? 3.f : -7.f);
   int best = 0;
-  float gain = 3.f + 0.9f * (tiles / g_pg_cus);
+  float gain = 3.f + 0.9f * (tiles / cus);
   for (int p = most + 1; p <= 8 && p <= 4 * most && most > 0; ++p) {
     const float per = (float)(most * nk) / p;
     if (per < 4) break;
@@ -1037,11 +1040,16 @@ std::vector<std::array<int, 7>> pgemm_last_round(int G, int ntiles, int nk, int 
   return out;
 }
 
-// floats of pieces' tiles that pgemm takes for its last round (0: it runs whole tiles only)
-long pgemm_tail_floats(int M, int N, int K) {
-  if (M <= 0 || N % 256 || K % 64 || pg_tail_share(M, N, K) == 0) return 0;
-  return (long)(g_pg_cus / 8) * PG_TAIL_SLOTS * PG_TSLAB;
+// {parts (0: whole tiles only), floats of pieces' tiles} of a product's last round on so many
+// compute units: 1 MB for one tile in four pieces, 92 MB for 128 tiles in eight parts, 117 MB at most
+std::pair<int, long> pgemm_tail_plan(int M, int N, int K, int cus) {
+  const int share = M > 0 && N % 256 == 0 && K % 64 == 0 ? pg_tail_share(M, N, K, cus) : 0;
+  if (share == 0) return {0, 0};
+  const int row = cus / 8, rest = (int)((long)((M + 255) / 256) * (N / 256) % cus);
+  return {share, (long)std::min(rest, row) * pg_row_slabs((rest + row - 1) / row, share) * PG_TSLAB};
 }
+
+long pgemm_tail_floats(int M, int N, int K) { return pgemm_tail_plan(M, N, K, pg_cus()).second; }
 
 // Estimated time: a tile takes 5 us + 0.92 (few workgroups) to 1.27 us (a full chip) per
 // K-step (measured 16 / 22 us at K 768, 48 / 55 at 3072, 63 / 82 at 4096)
@@ -1050,7 +1058,7 @@ float pgemm_us(int M, int N, int K) {
   const long whole = tiles / 256, rest = tiles % 256;
   const float round = 5.f + 1.27f * nk;
   if (rest == 0) return whole * round;
-  const int p = pg_tail_share(M, N, K);
+  const int p = pg_tail_share(M, N, K, pg_cus());
   if (p == 0) return whole * round + 5.f + nk * (0.92f + 0.35f * rest / 256.f);
   return whole * round + 23.f + 1.4f * ((rest + 31) / 32) * nk / p;
 }
@@ -1109,7 +1117,7 @@ int pgemm(void* C, const void* A, const void* W, const void* bias, int M, int N,
   PgTail tail{};
   if (grid <= 0) {
     grid = g_pg_cus;
-    if (slabs && cnt) tail = PgTail{pg_tail_share(M, N, K), slabs, cnt};
+    if (slabs && cnt) tail = PgTail{pg_tail_share(M, N, K, grid), slabs, cnt};
   }
   if (grid > tiles && tail.share == 0) grid = (int)tiles;
   auto C_ = (bf16_t*)C;

@@ -1882,12 +1882,20 @@ def pgemm_counters(dev: torch.device) -> torch.Tensor:
 
 def pgemm_tail(dev: torch.device, M: int, N: int, K: int) -> tuple:
     """(slabs, counters) of a product whose last round of tiles K13 cuts along K, or
-    (None, None): whole tiles only.  So is every product under capture: a graph may be
-    replayed beside this stream, whose counters it would share."""
-    n = native().pgemm_tail_floats(M, N, K)
+    (None, None): whole tiles only."""
+    return pgemm_tail_memory(dev, native().pgemm_tail_floats(M, N, K))
+
+
+def pgemm_tail_memory(dev: torch.device, n: int) -> tuple:
+    """n floats of slabs and the stream's counters, or (None, None): nothing to cut, no memory left
+    for the slabs (whole tiles need none), or a product under capture (a graph may be replayed
+    beside this stream, whose counters it would share)."""
     if n == 0 or torch.cuda.is_current_stream_capturing():
         return None, None
-    return torch.empty(n, dtype=torch.float32, device=dev), pgemm_counters(dev)
+    try:
+        return torch.empty(n, dtype=torch.float32, device=dev), pgemm_counters(dev)
+    except torch.cuda.OutOfMemoryError:
+        return None, None
 
 
 def row_scale(eps: float, part: torch.Tensor | None = None,

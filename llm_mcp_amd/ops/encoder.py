@@ -151,21 +151,18 @@ def encode(ids: torch.Tensor, cu: torch.Tensor, lens: list, w: dict, names: tupl
 def layers(x: torch.Tensor, ptrs: list, b: Batch, cu: torch.Tensor, I: int, H: int, D: int, eps: float,
            scale: float, gelu: bool, cos_sin: torch.Tensor | None) -> torch.Tensor:
     """All layers over x [T, d], in place.  ``ptrs``: ``layers_ok``'s."""
-    from . import PGEMM_CALLS, _ptr, _stream, native, pgemm_counters
+    from . import PGEMM_CALLS, _ptr, _stream, native, pgemm_tail_memory
     T, d = x.shape
     dev, n = x.device, native().enc_slab_floats(T, d, I)
     rows = torch.empty(T * (5 * d + I), dtype=x.dtype, device=dev)       # h, attn, qkv, g
     at = [0, T * d, 2 * T * d, 5 * T * d]
     h, attn, qkv, g = (_ptr(rows) + 2 * a for a in at)
-    tail = native().enc_tail_floats(T, d, I, gelu)
-    if torch.cuda.is_current_stream_capturing():
-        tail = 0               # see ops.pgemm_tail
-    slabs = torch.empty(n + tail, dtype=torch.float32, device=dev)
-    cnt = pgemm_counters(dev) if tail else None
+    slabs = torch.empty(n, dtype=torch.float32, device=dev)
+    tail, cnt = pgemm_tail_memory(dev, native().enc_tail_floats(T, d, I, gelu))
     native().encoder_layers(
         ptrs, T, d, I, H, D, gelu, float(eps), float(scale), _ptr(x), h, qkv, attn, g, _ptr(slabs), n,
         _ptr(cos_sin), _ptr(cu), _ptr(b.tiles), b.tiles.numel() // 2,
-        _ptr(slabs) + 4 * n if tail else 0, tail, _ptr(cnt), _stream())
+        _ptr(tail), 0 if tail is None else tail.numel(), _ptr(cnt), _stream())
     PGEMM_CALLS[0] += 4 * (len(ptrs) // 12)
     return x
 
