@@ -610,10 +610,10 @@ PYBIND11_MODULE(_lmx_kernels, m) {
                                S(stream)),
           "embed_layernorm");
   });
-  m.def("enc_plan", [](int M, int N, int K, int act, bool partials) {
-    const lmx::EncPlan p = lmx::enc_plan(M, N, K, act, partials);
+  m.def("enc_plan", [](int M, int N, int K, int act, bool partials, int cus) {
+    const lmx::EncPlan p = lmx::enc_plan(M, N, K, act, partials, cus);
     return std::make_pair(p.cfg, p.splits);
-  });
+  }, py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg("cus") = 0);
   m.def("enc_slab_floats", &lmx::enc_slab_floats);
   m.def("enc_tail_floats", &lmx::enc_tail_floats);
   m.def("enc_attention", [](uptr qkv, long ld, int H, int D, uptr cu, uptr tiles, int ntiles, uptr cos_sin,

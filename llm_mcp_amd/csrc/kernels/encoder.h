@@ -30,7 +30,7 @@ struct EncArgs {
 struct EncPlan { int cfg, splits; };   // cfg: dgemm's, -1: K13, kEncSmall: K23
 constexpr int kEncSmall = 100;
 
-EncPlan enc_plan(int M, int N, int K, int act, bool partials);
+EncPlan enc_plan(int M, int N, int K, int act, bool partials, int cus = 0);
 long enc_slab_floats(int T, int d, int I);
 long enc_tail_floats(int T, int d, int I, bool gelu);
 int encoder_layers(const EncArgs& a, const uintptr_t* w, hipStream_t stream);

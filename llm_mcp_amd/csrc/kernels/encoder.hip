@@ -29,14 +29,15 @@ int dgemm(void*, const void*, const void*, float*, unsigned*, int, int, int, int
 int pgemm(void*, const void*, const void*, const void*, int, int, int, long, long, long, int, int, int,
           int, float*, hipStream_t, float*, unsigned*);
 long pgemm_tail_floats(int, int, int);
-float pgemm_us(int, int, int);
+float pgemm_us(int, int, int, int);
+int pgemm_cus();
 int sgemm(void*, const void*, const void*, int, int, int, long, long, long, int, int, const void*,
           hipStream_t);
 
 namespace {
 
 // Time of a decode-GEMM tile configuration in us: base + rounds x (start + step x
-// K / 64), rounds of 256 workgroups (one per CU); fill: the slabs' writes at a full
+// K / 64), rounds of a workgroup per CU; fill: the slabs' writes at a full
 // round. Least squares over 12 shapes (N 384 to 6144, K 384 to 4096) x 16 row counts
 // (16 to 12288) x slices, each within 5 to 8 % rms of the measured time.
 struct EncTile { int cfg, bm, bn; float base, start, step, fill; };
@@ -53,15 +54,16 @@ constexpr float kBytesUs = 4.5e6f;                         // memory traffic, by
 }  // namespace
 
 // act: 0 none, 3 SwiGLU over 16-row pairs, 4 gelu (exact). partials: the
-// product's fp32 slabs go to a LayerNorm (no activation).
-EncPlan enc_plan(int M, int N, int K, int act, bool partials) {
+// product's fp32 slabs go to a LayerNorm (no activation). cus: compute units (0: the device's).
+EncPlan enc_plan(int M, int N, int K, int act, bool partials, int cus) {
+  if (cus <= 0) cus = pgemm_cus();
   EncPlan best{-1, 0};
   // few rows: K23, except where K slices of the 64 x 64 tile fill the chip (at 16 rows:
   // qkv of nomic 4.5 us against 5.7, gate / up 5.8 against 7.3, but o 3.5 against 3.0 and down 4.6
   // against 4.0; qkv at 32 rows 5.5 against 5.9, at 64 7.5 against 6.1)
   if (!partials && M <= 32 && N % 32 == 0 && K % 32 == 0) return {kEncSmall, 1};
   const bool k13 = N % 256 == 0 && K % 64 == 0 && K >= 192;
-  float t = k13 ? pgemm_us(M, N, K) : 1e30f;
+  float t = k13 ? pgemm_us(M, N, K, cus) : 1e30f;
   for (const EncTile& c : kTiles) {
     const int bk = c.cfg == 11 ? 64 : 128;
     if (N % c.bn || (act == 3 && c.cfg == 21)) continue;   // a wave holds whole 16-row pairs
@@ -69,10 +71,10 @@ EncPlan enc_plan(int M, int N, int K, int act, bool partials) {
     if (tiles > 4096) continue;
     for (int s : kSlices) {
       if ((s > 1 && !partials) || K % (bk * s)) continue;
-      const long wgs = tiles * s, rounds = (wgs + 255) / 256;
+      const long wgs = tiles * s, rounds = (wgs + cus - 1) / cus;
       float u = c.base + rounds * (c.start + c.step * (K / 64.f / s));
       if (partials)      // the slabs' writes and reads against bf16 rows
-        u += c.fill * wgs / 256.f + (4.f * s - 2.f) * M * N / kBytesUs;
+        u += c.fill * wgs / cus + (4.f * s - 2.f) * M * N / kBytesUs;
       if (u < t) {
         t = u;
         best = {c.cfg, s};

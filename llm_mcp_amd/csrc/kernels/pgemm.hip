@@ -1051,16 +1051,19 @@ std::pair<int, long> pgemm_tail_plan(int M, int N, int K, int cus) {
 
 long pgemm_tail_floats(int M, int N, int K) { return pgemm_tail_plan(M, N, K, pg_cus()).second; }
 
+// the device's compute units (those of a whole MI355X where there is no device)
+int pgemm_cus() { return pg_cus() > 0 ? g_pg_cus : 256; }
+
 // Estimated time: a tile takes 5 us + 0.92 (few workgroups) to 1.27 us (a full chip) per
 // K-step (measured 16 / 22 us at K 768, 48 / 55 at 3072, 63 / 82 at 4096)
-float pgemm_us(int M, int N, int K) {
+float pgemm_us(int M, int N, int K, int cus) {
   const long tiles = (long)((M + 255) / 256) * (N / 256), nk = K / 64;
-  const long whole = tiles / 256, rest = tiles % 256;
+  const long whole = tiles / cus, rest = tiles % cus;
   const float round = 5.f + 1.27f * nk;
   if (rest == 0) return whole * round;
-  const int p = pg_tail_share(M, N, K, pg_cus());
-  if (p == 0) return whole * round + 5.f + nk * (0.92f + 0.35f * rest / 256.f);
-  return whole * round + 23.f + 1.4f * ((rest + 31) / 32) * nk / p;
+  const int p = pg_tail_share(M, N, K, cus);
+  if (p == 0) return whole * round + 5.f + nk * (0.92f + 0.35f * rest / cus);
+  return whole * round + 23.f + 1.4f * ((rest + cus / 8 - 1) / (cus / 8)) * nk / p;
 }
 
 // Grouped rows on the persistent 256 x 256 tile: M sorted rows (A rows src[..] or
