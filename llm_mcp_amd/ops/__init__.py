@@ -1750,9 +1750,7 @@ def rsgemm(a: torch.Tensor, w: torch.Tensor, cfg: int, splits: int, epi: int = 0
 # K13: large-M GEMM (csrc/kernels/pgemm.hip): prefill chunks, encoder batches
 # ---------------------------------------------------------------------------
 PGEMM_MAX_BIAS = 14336
-# host-side count of products on the hand-written prompt path (tests: no library kernel ran): K13,
-# and the encoders' native layers (encoder.hip: K13 or the decode GEMM's tiles, by rows)
-PGEMM_CALLS = [0]
+PGEMM_CALLS = [0]          # host-side launch count (tests: the K13 path really ran)
 RESIDUAL_EPILOGUE = os.environ.get("LMX_RESIDUAL_EPILOGUE", "1") != "0"
 
 

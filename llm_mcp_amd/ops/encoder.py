@@ -19,6 +19,7 @@ import torch
 
 PAGE = 32                      # of the models' own loops
 QUERIES = 128                  # EA_Q in csrc/kernels/encattn.hip
+LAYER_CALLS = [0]              # host-side count of layers run natively (enc_plan: on which kernels)
 
 
 @dataclass
@@ -151,7 +152,7 @@ def encode(ids: torch.Tensor, cu: torch.Tensor, lens: list, w: dict, names: tupl
 def layers(x: torch.Tensor, ptrs: list, b: Batch, cu: torch.Tensor, I: int, H: int, D: int, eps: float,
            scale: float, gelu: bool, cos_sin: torch.Tensor | None) -> torch.Tensor:
     """All layers over x [T, d], in place.  ``ptrs``: ``layers_ok``'s."""
-    from . import PGEMM_CALLS, _ptr, _stream, native, pgemm_tail_memory
+    from . import _ptr, _stream, native, pgemm_tail_memory
     T, d = x.shape
     dev, n = x.device, native().enc_slab_floats(T, d, I)
     rows = torch.empty(T * (5 * d + I), dtype=x.dtype, device=dev)       # h, attn, qkv, g
@@ -163,7 +164,7 @@ def layers(x: torch.Tensor, ptrs: list, b: Batch, cu: torch.Tensor, I: int, H: i
         ptrs, T, d, I, H, D, gelu, float(eps), float(scale), _ptr(x), h, qkv, attn, g, _ptr(slabs), n,
         _ptr(cos_sin), _ptr(cu), _ptr(b.tiles), b.tiles.numel() // 2,
         _ptr(tail), 0 if tail is None else tail.numel(), _ptr(cnt), _stream())
-    PGEMM_CALLS[0] += 4 * (len(ptrs) // 12)
+    LAYER_CALLS[0] += len(ptrs) // 12
     return x
 
 

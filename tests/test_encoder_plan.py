@@ -1,7 +1,12 @@
 """The encoders' choice of a product's kernel (csrc/kernels/encoder.hip enc_plan), on the host."""
+import dataclasses
+
 import pytest
+import torch
 
 from llm_mcp_amd import native, ops
+from llm_mcp_amd.models import config as mc
+from llm_mcp_amd.ops import encoder
 
 SMALL, K13 = 100, -1            # EncPlan's cfg for K23 and K13
 
@@ -40,3 +45,51 @@ def test_rounds_are_of_the_device(cus):
         if cfg >= 0 and cfg != SMALL:
             bm, bn = ops.DGEMM_CONFIGS[cfg]
             assert -(-M // bm) * (1024 // bn) * s <= max(cus, -(-M // bm) * (1024 // bn))
+
+
+# rows of a request between which every kernel, tile and slice that the choice has for a product
+# of the model up to 8,192 rows occurs
+ROWS = {"nomic-embed-text": [1, 65, 155, 193, 321, 449, 641, 897, 1345, 1793, 2689, 3585, 4030, 5377, 5441],
+        "mxbai-embed-large": [1, 75, 129, 156, 321, 513, 641, 668, 1345, 2689, 4097]}
+
+
+def _plans(cfg, M):
+    d, I, gelu = cfg.hidden_size, cfg.intermediate_size, cfg.family == "bert"
+    return {(i, *native.kernels().enc_plan(M, *x, 256)) for i, x in enumerate(
+        ((3 * d, d, 0, False), (d, d, 0, True), (I if gelu else 2 * I, d, 4 if gelu else 3, False),
+         (d, I, 0, True)))}
+
+
+@pytest.mark.parametrize("model", ROWS)
+def test_rows_below_reach_every_plan(model):
+    cfg = mc.resolve(model)
+    every = set().union(*(_plans(cfg, M) for M in range(1, 8193)))
+    assert set().union(*(_plans(cfg, M) for M in ROWS[model])) == every
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model,rows", [(m, r) for m in ROWS for r in ROWS[m]])
+def test_every_plan_against_the_models_own_loop(model, rows):
+    """One layer of the model's sizes on every kernel, tile and slice that it is planned on: the
+    vectors of the loop over single ops, which runs K13 alone."""
+    from llm_mcp_amd.models.bert import BertModel
+    from llm_mcp_amd.models.nomic_bert import NomicBertModel
+    cfg = dataclasses.replace(mc.resolve(model), num_layers=1)
+    m = (BertModel if cfg.family == "bert" else NomicBertModel)(cfg, "cuda", seed=4)
+    g = torch.Generator().manual_seed(rows)
+    longest, lens = 500, []
+    while sum(lens) < rows:
+        lens.append(min(rows - sum(lens), longest))
+    ids = torch.randint(0, 30000, (rows,), generator=g, dtype=torch.int32).cuda()
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+    calls = encoder.LAYER_CALLS[0]
+    a = m.forward(ids, cu, lens)
+    assert encoder.LAYER_CALLS[0] == calls + 1
+    keep, encoder.layers_ok = encoder.layers_ok, lambda *x: None
+    try:
+        b = m.forward(ids, cu, lens)
+    finally:
+        encoder.layers_ok = keep
+    # bf16 rows through one layer and its two norms: 2^-8 of a row's length at each of some ten
+    # roundings, at random, against the other's
+    assert float((a - b).norm(dim=1).max()) < 10 ** 0.5 * 2 ** 0.5 * 2.0 ** -8
