@@ -839,34 +839,51 @@ def few_rows(x: torch.Tensor, w: torch.Tensor, epi: int = 0, bias: torch.Tensor 
     return None
 
 
-# K23 (csrc/kernels/sgemm.hip), few rows and small weights: elements of W up to which it
-# beats the tables' kernels on cold weights. Llama-3.2-1B at 1 / 16 / 32 rows: QKV (6.3 M) 5.4 / 6.7 /
-# 8.7 us against 11.2 / 11.4 / 11.6, O (4.2 M) 4.1 / 4.7 / 5.7 against 7.1 / 7.3 / 7.0, and at 64
-# rows 13.0 against 12.4; Llama-3-8B O (16.8 M) 9.1 at 1 row and 10.6 at 8 against 10.9 and 11.3,
-# 12.8 at 16 against 11.6
+# K23 (csrc/kernels/sgemm.hip), few rows and small weights: where it beats the routes below on
+# cold weights.  Measured at 1 to 32 rows, 32 to 24,576 columns, K 64 to 14,336 (450 products):
+#  - weights: 6.6 M elements, left as slabs to 8 rows of 17 M.  Llama-3.2-1B at 3 / 16 / 32 rows: QKV (6.3 M) 1.7
+#    / 1.5 / 1.2 times as fast; Llama-3-8B O as slabs (16.8 M) 1.1 at 3 rows, 1.02 at 8;
+#  - rows by K (plain, pair epilogues): a workgroup walks all of K and reads all rows' activations, the split-K
+#    library kernels do not.  64 columns, K23 as fast as the library times: K 2048 at 32 rows 1.26, 2560 at
+#    16 1.14 and at 24 0.88, 4096 at 16 1.38 and at 32 0.79, 5120 at 8 1.6 and at 12 0.77, 6144 at 8 0.87, 12288
+#    at 24 0.46; pairs 2560 at 8 1.08 and at 16 0.94.  K 1280 (5 steps a wave, loaded by fours) at 32 0.95;
+#  - more than 4096 columns are more than a workgroup per CU: 512 to 1024 of K only (5120 columns, K 768 at 32 rows
+#    1.09, K 1280 0.61, K 256 0.69); pairs to 12288 columns (24576 x 256 0.83 at 16 rows);
+#  - slabs: K slices bound a workgroup's K (64 columns, K 12288 at 24 rows 1.32); without slices K 2048, to 16 rows
+#    4096 (2304 columns, K 2560 at 16 / 24 rows 1.18 / 0.91).  6144 columns at 8 rows: K 2048 1.31, 2560 0.90.
 SGEMM_MAX_M, SGEMM_MAX_W = 32, 6_600_000
 SGEMM_MAX_M_WIDE, SGEMM_MAX_W_WIDE = 8, 17_000_000
+SGEMM_ROWS = ((1152, 32, 32), (1535, 24, 32), (2048, 32, 32), (4096, 16, 8), (5120, 8, 8))
 SGEMM_CALLS = [0]          # host-side launch count (tests: the K23 path really ran)
 
 
 def sgemm_splits(M: int, N: int, K: int, epi: int = 0) -> int | None:
     """K slices of this product on K23 (1 except for epi 2, fp32 slabs), or None: not
     its range.  The larger weights only as slabs (a plain one of them is K11's)."""
-    if N % 32 or K % 32 or M < 1:
+    if N % 32 or K % 32 or not 0 < M <= SGEMM_MAX_M or table_keeps(M, N, K, epi):
         return None
-    if not (M <= SGEMM_MAX_M and N * K <= SGEMM_MAX_W) and not (
-            epi == 2 and M <= SGEMM_MAX_M_WIDE and N * K <= SGEMM_MAX_W_WIDE):
+    if N * K > SGEMM_MAX_W and not (epi == 2 and M <= SGEMM_MAX_M_WIDE and N * K <= SGEMM_MAX_W_WIDE):
         return None
-    if epi != 2:
-        return 1
-    # a workgroup per CU, 4 slices at most (each is read again by the norm)
-    return next(s for s in (4, 2, 1) if s == 1 or (N // 16 * s <= 256 and K // 32 % s == 0))
+    if epi == 2:
+        # a workgroup per CU, 4 slices at most (each is read again by the norm)
+        s = next(s for s in (4, 2, 1) if s == 1 or (N // 16 * s <= 256 and K // 32 % s == 0))
+        if N > 4096:
+            ok = 512 <= K <= 1024 or (K < 512 and M <= 16) or (K <= 2048 and M <= 8 and N <= 8192)
+        else:
+            ok = s > 1 or K <= (2048 if M > 16 else 4096)
+        return s if ok else None
+    rows = next((r for k, *r in SGEMM_ROWS if K <= k), (0, 0))[epi in (3, 4)]
+    wide = 512 <= K <= 1024 if epi == 0 else N <= 12288
+    return 1 if M <= rows and (N <= 4096 or wide) else None
 
 
 # K25 (csrc/kernels/gemv.hip), one or two rows: whole weight rows streamed. Faster than
-# the other kernels at every size but where K14 has packed weights (4096 x 14336: 21.7 us
-# against 20.7) and one near 16384 x 4096 (25.9 against 24.3; 15360 and 17408 columns 23.0
-# and 26.5 against 29.5 and 51); at four rows its FMAs take as long as the stream.
+# the other kernels at every size without a table entry (1,024 to 40,960 columns, K 1024 to 24,576: 1.0 to 3.5 times),
+# and at 55 of the table's 64 shapes; the others (``table_keeps``) are those where an entry of K11 reads
+# at 5 TB/s or more and K25's activations do not fit the vector L1 (8192 x 28672 at two rows 86.5 us
+# against 82.0), or its rows a power of two apart share channels (16384 x 4096 26.9 against 25.0).  K14 has
+# packed weights where it is picked (4096 x 14336: 20.7 against 21.7).  At four rows the FMAs take as
+# long as the stream.
 GEMV_MAX_M, GEMV_K = 2, 1024
 GEMV_CALLS = [0]           # host-side launch count (tests: the K25 path really ran)
 
@@ -878,7 +895,7 @@ def gemv_splits(x: torch.Tensor, w: torch.Tensor, epi: int = 0, out: torch.Tenso
         return None
     if out is not None and (out.stride(1) != 1 or out.stride(0) % 2 or out.data_ptr() % 4):
         return None
-    if epi != 4 and rs_choice(M, N, K, epi=epi, w=w) is not None:
+    if (epi != 4 and rs_choice(M, N, K, epi=epi, w=w) is not None) or table_keeps(M, N, K, epi):
         return None
     # 2048 waves (two a SIMD) at least
     return 2 if epi == 2 and N < 4096 and K // GEMV_K % 2 == 0 else 1
@@ -1301,6 +1318,32 @@ def _sk_table() -> dict:
                     _SK_TABLE.setdefault((int(e["N"]), int(e["K"]), int(e.get("epi", 0))), []).append(
                         (int(e["m_min"]), int(e["m_max"]), int(e["splits"])))
     return _SK_TABLE
+
+
+_KEEP_TABLE: dict | None = None
+
+
+def _keep_table() -> dict:
+    """{(N, K, epi): [(m_min, m_max), ...]} from config/dgemm_gfx950.json "keep": few-row products
+    whose table kernel was measured faster than K25 or K23 on cold weights (every tabled
+    shape at 1 to 32 rows, twice; partials with the norm that sums them)."""
+    global _KEEP_TABLE
+    if _KEEP_TABLE is None:
+        import json
+        _KEEP_TABLE = {}
+        path = os.environ.get("LMX_DGEMM_TABLE") or os.path.join(
+            os.path.dirname(os.path.dirname(__file__)), "config", "dgemm_gfx950.json")
+        if os.environ.get("LMX_DGEMM", "1") == "1" and os.path.exists(path):
+            with open(path) as f:
+                for e in json.load(f).get("keep", []):
+                    _KEEP_TABLE.setdefault((int(e["N"]), int(e["K"]), int(e["epi"])), []).append(
+                        (int(e["m_min"]), int(e["m_max"])))
+    return _KEEP_TABLE
+
+
+def table_keeps(M: int, N: int, K: int, epi: int = 0) -> bool:
+    """This product stays on the kernel that the measured table names for it."""
+    return any(a <= M <= b for a, b in _keep_table().get((N, K, 3 if epi == 4 else epi), ()))
 
 
 def sk_choice(M: int, N: int, K: int, epi: int = 0) -> int | None:

@@ -70,3 +70,33 @@ def test_gradients_and_transforms():
     with torch.autograd.forward_ad.dual_level():
         seen.append(ops.few_rows_ok(torch.autograd.forward_ad.make_dual(x, x), w))
     assert seen == [False] * 3
+
+
+@pytest.mark.parametrize("M,N,K,epi,splits", [
+    (32, 2048, 2048, 0, 1), (33, 2048, 2048, 0, None), (32, 32, 1152, 0, 1), (24, 64, 1280, 0, 1),
+    (25, 64, 1280, 0, None), (32, 64, 1280, 3, 1), (17, 64, 2080, 0, None), (16, 64, 4096, 0, 1),
+    (9, 64, 4128, 0, None), (8, 64, 5120, 0, 1), (1, 64, 5152, 0, None), (8, 512, 4096, 3, 1),
+    (9, 512, 4096, 4, None), (32, 4096, 256, 0, 1), (1, 4128, 480, 0, None), (32, 6144, 768, 0, 1),
+    (1, 6144, 1056, 0, None), (32, 12288, 256, 3, 1), (1, 12320, 256, 3, None), (3, 3072, 4096, 0, None),
+    (32, 64, 14336, 2, 4), (32, 1024, 6144, 2, 4), (32, 2048, 2048, 2, 2), (17, 2304, 2560, 2, None),
+    (16, 2304, 2560, 2, 1), (8, 4096, 4096, 2, 1), (9, 4096, 4096, 2, None), (8, 2560, 4608, 2, None),
+    (8, 6144, 2048, 2, 1), (8, 6144, 2560, 2, None), (8, 12288, 1280, 2, None), (9, 6144, 1056, 2, None),
+    (3, 96, 48, 0, None), (3, 48, 96, 0, None), (0, 96, 96, 0, None)])
+def test_shapes_of_k23(M, N, K, epi, splits):
+    assert ops.sgemm_splits(M, N, K, epi) == splits
+
+
+def test_products_that_the_table_keeps(monkeypatch):
+    """Shapes whose table kernel was measured faster: they have one, and neither kernel takes them."""
+    keep, taken = ops._keep_table(), 0
+    cases = [(M, *k) for k, ranges in keep.items() for a, b in ranges for M in range(a, b + 1)]
+    assert cases and all(1 <= M <= ops.SGEMM_MAX_M and ops.dgemm_choice(M, *k) for M, *k in cases)
+    for off in (False, True):
+        if off:
+            monkeypatch.setattr(ops, "_KEEP_TABLE", {})
+        for M, N, K, epi in cases:
+            x, w = torch.zeros(M, K).bfloat16(), torch.empty(N, K, dtype=torch.bfloat16, device="meta")
+            got = ops.gemv_splits(x, w, epi), ops.sgemm_splits(M, N, K, epi)
+            assert off or got == (None, None)
+            taken += got != (None, None)
+    assert taken == len(cases)               # without the list one of them takes each
