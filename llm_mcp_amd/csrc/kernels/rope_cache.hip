@@ -590,7 +590,8 @@ int qkv_norm_rope_cache(const void* p, long p_ld, const float* bias, const float
 }
 
 // Plain cache write (no rotation): models without rotary embeddings.  Any head
-// size and alignment, one token per workgroup.
+// size and alignment, one token per workgroup: few tokens are bound by latency, and this is one
+// trip to memory and no barrier (a token of 8 heads of 128 3.4 us, 600 tokens 5.4).
 __global__ void kv_write_kernel(const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
                                 long kv_stride, const int* __restrict__ slot_mapping, int Hkv,
                                 int D, bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache,
@@ -608,7 +609,8 @@ __global__ void kv_write_kernel(const bf16_t* __restrict__ k, const bf16_t* __re
 
 // The same for rows of whole 16-B pieces: grid (32-token tiles, K groups + V
 // groups) as rope_cache_tiled_kernel, V in key quads through LDS instead of 2-B
-// stores 8 B apart.  19,153 tokens of 16 heads of 64: 53 -> 39 us (157 MB).
+// stores 8 B apart: many tokens, bound by the stores.  19,153 tokens of 16 heads of 64: 53 -> 39 us
+// (157 MB); 600 of 8 heads of 128 6.0, longer than a workgroup a token.
 __global__ void __launch_bounds__(256) kv_write_tiled_kernel(
     const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, long kv_stride,
     const int* __restrict__ slot_mapping, int T, int Hkv, int D, bf16_t* __restrict__ k_cache,
@@ -641,8 +643,10 @@ __global__ void __launch_bounds__(256) kv_write_tiled_kernel(
 int kv_write(const void* k, const void* v, long kv_stride, const int* slot_mapping, int T, int Hkv,
              int D, void* k_cache, void* v_cache, int BS, hipStream_t stream) {
   if (T <= 0) return 0;
-  // whole 16-B pieces of rows and pages, whole key quads (BS % 4)
-  if (D % 8 == 0 && D <= 256 && BS % 4 == 0 && kv_stride % 8 == 0 &&
+  // whole 16-B pieces of rows and pages, whole key quads (BS % 4).  The line is where both take the same time:
+  // 800,000 elements at 4 to 16 heads (1600 tokens of 4 heads of 128 5.9 / 6.0 us, 600 of 8 5.4 / 6.0, 1200
+  // of 8 7.2 / 6.6), 4096 tokens at one or two (of one of 128 5.2 / 4.8, 3000 4.5 / 4.9)
+  if ((T >= 4096 || (long)T * Hkv * D >= 800000) && D % 8 == 0 && D <= 256 && BS % 4 == 0 && kv_stride % 8 == 0 &&
       (((uintptr_t)k | (uintptr_t)v | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0) {
     const int hv = rope_v_heads(D), groups = (Hkv + hv - 1) / hv;
     kv_write_tiled_kernel<<<dim3((T + RT - 1) / RT, 2 * groups), dim3(256),

@@ -56,8 +56,27 @@ def test_rope_head_groups(Hq, Hkv, D, T, skip_q):
 @pytest.mark.parametrize("T", [1, 31, 32, 65])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_kv_write(H, D, T, shift):
-    """Aligned rows (key quads) and rows that no 16-byte load reads."""
+    """Few tokens, a workgroup each: aligned rows and rows that no 16-byte load reads."""
     NB = 6
+    kv = torch.randn(T, 2 * H * D + 8, device=DEV).bfloat16()
+    k = kv[:, shift:shift + H * D].view(T, H, D)
+    v = kv[:, shift + H * D:shift + 2 * H * D].view(T, H, D)
+    slots = _slots(T, NB).to(DEV)
+    kc = torch.zeros(NB, H, 32, D, device=DEV, dtype=torch.bfloat16)
+    vc = torch.zeros(NB, H, 8, D, 4, device=DEV, dtype=torch.bfloat16)
+    k0, v0 = kc.cpu(), vc.cpu()
+    ref.write_cache(k.cpu(), v.cpu(), slots.cpu(), k0, v0)
+    ops.kv_write(k, v, slots, kc, vc)
+    assert torch.equal(kc.cpu(), k0) and torch.equal(vc.cpu(), v0)
+
+
+@pytest.mark.parametrize("H,D", [(16, 64), (3, 128), (5, 48), (2, 256), (1, 8), (3, 20)])
+@pytest.mark.parametrize("T", [1601, 4096, 4097, 4127])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_kv_write_of_many_tokens(H, D, T, shift):
+    """Both sides of the line between a workgroup a token and 32-token tiles: tiles of 1, 31 and 32
+    tokens, head groups that do not divide the heads, rows that no 16-byte load reads."""
+    NB = T // 32 + 8
     kv = torch.randn(T, 2 * H * D + 8, device=DEV).bfloat16()
     k = kv[:, shift:shift + H * D].view(T, H, D)
     v = kv[:, shift + H * D:shift + 2 * H * D].view(T, H, D)
