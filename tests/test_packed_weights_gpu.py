@@ -44,6 +44,29 @@ def test_pgemm_packed_w_matches_row_major(M, N, K):
     torch.testing.assert_close(r1.float(), (r0.float() + y.float()), atol=3e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("M,N,K", [(100, 256, 8192), (257, 512, 6144), (600, 4096, 14336), (2300, 4096, 14336),
+                                   (6464, 4096, 14336), (2048, 18688, 4096)])
+def test_last_round_in_pieces_on_packed_w(M, N, K):
+    """The cut of K13's last round is by shape alone, so packed W gives the bits of row-major W there
+    too, in every form of the epilogue that the prompts of packed weights use; pieces start inside K."""
+    assert ops.native().pgemm_tail_floats(M, N, K) > 0
+    a, w, s = _bf(M, K), _bf(N, K, scale=K ** -0.5), torch.rand(M, device=DEV) + 0.5
+    wp, ran = ops.rsgemm_pack(w), []
+    for kw in (dict(), dict(act=ops.ACT_SWIGLU), dict(row_scale=s), dict(act=ops.ACT_SWIGLU, row_scale=s)):
+        ran.append(ops.pgemm(a, w, **kw))
+        assert torch.equal(ops.pgemm(a, wp, packed=True, **kw), ran[-1])
+    torch.testing.assert_close(ran[0].float(), a.float() @ w.float().t(), atol=4e-3, rtol=2.0 ** -7)
+    r0 = _bf(M, N)
+    for sums in (False, True):
+        got = []
+        for x, packed in ((w, False), (wp, True)):
+            r, q = r0.clone(), torch.empty(M, N // 64, device=DEV) if sums else None
+            ops.pgemm(a, x, residual=r, ssq=q, packed=packed)
+            got.append((r, q))
+        assert torch.equal(got[0][0], got[1][0]) and (not sums or torch.equal(got[0][1], got[1][1]))
+        torch.testing.assert_close(got[1][0].float(), r0.float() + ran[0].float(), atol=3e-2, rtol=2.0 ** -7)
+
+
 @pytest.mark.parametrize("M", [1, 16, 64, 100, 200, 256, 300, 700])
 def test_packed_only_weights_every_batch_size(M):
     """linear / linear_swiglu / the residual product on packed-only weights of

@@ -301,8 +301,8 @@ def _k13(M, N, K, **kw):
     (7000, 4864, 832, False),      # 532 tiles: 20 of 13 steps
     (2048, 8192, 512, False)])     # one round, whole
 def test_k13_last_round(M, N, K, cut):
-    """Every form of the epilogue where the last round of tiles is cut along K: the numbers
-    of a product in fp32, the same bits each time, nothing left in the counters."""
+    """Every form of the epilogue on row-major W where the last round of tiles is cut along K: the
+    numbers of a product in fp32, the same bits each time, nothing left in the counters."""
     assert (ops.native().pgemm_tail_floats(M, N, K) > 0) == cut
     a, w = _k13(M, N, K)
     z = a.float() @ w.float().t()
