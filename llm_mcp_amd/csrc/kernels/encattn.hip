@@ -13,8 +13,8 @@
 // LDS read, from the same row-major image that the rows arrive in).  K / V rows go through
 // registers (they are rotated there) into a double buffer: the next tile's loads are in flight
 // while a tile is computed, one barrier a tile.
-// The grid has the heads innermost: the workgroups of a head are spread over one XCD (H % 8
-// == 0) or two, which read its K / V through their L2, and the longest sequences start first.
+// The grid has the heads innermost: the workgroups of a head run on 8 / gcd(H, 8) XCDs (one for 16 heads,
+// two for 12), which read its K / V through their L2, and the longest sequences start first.
 // Bound by vector instructions (150 a wave and tile, 32 of them exponentials, 56 more for the
 // rotation): 16 heads, 48 sequences of 512: 70 us, 739 TF/s; 12 heads, 16 of 735, rotated: 58 us.
 // Cache pages written by one kernel and read by the prompt attention took 85 + 40 us for 19153

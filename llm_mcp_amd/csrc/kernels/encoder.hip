@@ -60,7 +60,9 @@ EncPlan enc_plan(int M, int N, int K, int act, bool partials, int cus) {
   EncPlan best{-1, 0};
   // few rows: K23, except where K slices of the 64 x 64 tile fill the chip (at 16 rows:
   // qkv of nomic 4.5 us against 5.7, gate / up 5.8 against 7.3, but o 3.5 against 3.0 and down 4.6
-  // against 4.0; qkv at 32 rows 5.5 against 5.9, at 64 7.5 against 6.1)
+  // against 4.0; qkv at 32 rows 5.5 against 5.9, at 64 7.5 against 6.1). K is d, 2048 at most. Weights
+  // over 12 M elements, which no preset has, would do better on the 64 x 64 tile from 17 rows on (6144 x 2048 at
+  // 16 / 32 rows 12.2 / 17.1 us against 12.2 / 12.4; K13 36.4)
   if (!partials && M <= 32 && N % 32 == 0 && K % 32 == 0) return {kEncSmall, 1};
   const bool k13 = N % 256 == 0 && K % 64 == 0 && K >= 192;
   float t = k13 ? pgemm_us(M, N, K, cus) : 1e30f;

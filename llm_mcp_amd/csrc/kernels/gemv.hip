@@ -9,9 +9,11 @@
 // no LDS, no barrier. The activations (8 KB a row at K = 4096) come from the vector L1.
 // Measured, cold weights, one row (before: the fastest of K11 and K23): 16384 x 2048 with the
 // SwiGLU 12.3 us (18.0), 6144 x 4096 10.4 (13.7), 3072 x 2048 4.5 (5.5), 4096 x 4096 7.8 (9.2), 2048 x
-// 8192 in two slices 7.9 (9.3), 28672 x 4096 37.8 (39.2), 128256 x 4096 151 (160): 5 to 6.9 TB/s.
-// Two rows 0.4 to 2 us more, four no better than before. A read of the same bytes that does
-// nothing else takes 11.5, 9.3, 3.4 and 6.8. Blocks in plain order (not a range of rows per XCD)
+// 8192 in two slices 7.9 (9.3), 28672 x 4096 37.8 (39.2), 128256 x 4096 151 (160): 2.8 TB/s for 13 MB, 4.2
+// to 4.8 for 34 to 50, 5.5 for 67, 6.2 to 7 from 235 on. Two rows 0.4 to 2 us more up to 150 MB, beyond 2
+// to 10 % (17 % at K = 25600, where the rows pass the vector L1), four no better than before. A read of the
+// same bytes that does nothing else takes 11.5, 9.3, 3.4 and 6.8 for the first four. Where a measured
+// kernel of the table is faster the product stays there (ops.table_keeps). Blocks in plain order (not a range of rows per XCD)
 // cost 10 % at K = 4096.
 #include "common.h"
 

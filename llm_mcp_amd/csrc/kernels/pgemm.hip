@@ -10,7 +10,8 @@
 // The structure is chosen for one 512-thread workgroup per CU holding a
 // 256 x 256 output tile (cdna guide §5 "the 256² 8-phase template", MI355X
 // microarch guide §LDS / MFMA):
-//   * persistent: gridDim = min(tiles, CUs); a workgroup walks its tiles
+//   * persistent: gridDim = min(tiles, CUs), or all CUs where the last round is cut
+//     along K (pg_tail_share); a workgroup walks its tiles
 //     (linear id i * grid + xcd_remap(block), grouped 8 M-tiles x N so one XCD's
 //     32 concurrent tiles share 8 A panels and 4 W panels in its L2) and the
 //     k-steps of consecutive tiles form ONE load stream: the next tile's first
@@ -1041,7 +1042,7 @@ std::vector<std::array<int, 7>> pgemm_last_round(int G, int ntiles, int nk, int 
 }
 
 // {parts (0: whole tiles only), floats of pieces' tiles} of a product's last round on so many
-// compute units: 1 MB for one tile in four pieces, 92 MB for 128 tiles in eight parts, 117 MB at most
+// compute units: 1 MB for one tile in four pieces, 92 MB for 128 tiles in eight parts, 109 MB at most
 std::pair<int, long> pgemm_tail_plan(int M, int N, int K, int cus) {
   const int share = M > 0 && N % 256 == 0 && K % 64 == 0 ? pg_tail_share(M, N, K, cus) : 0;
   if (share == 0) return {0, 0};

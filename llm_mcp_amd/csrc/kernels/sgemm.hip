@@ -1,5 +1,5 @@
-// K23: projection of a few rows (1 to 64; one and two of long K: gemv.hip) with weights of up to
-// some tens of MB:
+// K23: projection of a few rows (1 to 64; ops.sgemm_splits and the encoders take it to 32, and one and
+// two rows of K in whole thousands go to gemv.hip) with small weights:
 //     C[M, N] = epi(A[M, K] . W[N, K]^T)      bf16 in, fp32 accumulate
 //
 // Such a product is bound by latencies, not by its weight stream: the decode GEMM
@@ -8,7 +8,8 @@
 // another kernel has to sum. Here a workgroup owns 16 NT columns over all of K (or
 // a slice) and its 8 waves share K: a wave loads its fragments straight to registers,
 // U K32 steps (16 B a lane) at a time and the next U behind them, so the whole
-// workgroup has 64 KB of weights in flight without a barrier; one exchange through LDS
+// workgroup has 64 KB of weights in flight without a barrier (128 with one row tile and two column
+// tiles, 32 with four row tiles and one column tile); one exchange through LDS
 // adds the 8 partial tiles. Every weight is read once, the activations once per
 // workgroup from L2.
 //
@@ -18,7 +19,8 @@
 // Measured (cold weights, one row / 16 rows; before: K11 with its slices): 3072 x 2048 5.4 / 6.7 us
 // (11.2 / 11.4), 2048 x 2048 as two slabs 4.1 / 4.7 (7.1 / 7.3), 2304 x 768 4.0 / 4.5 (- / 5.7),
 // 4096 x 4096 9.1 / 12.8 (10.9 / 11.6): above 32 rows and some 20 MB the ring kernels are the better
-// ones, since every workgroup reads all activations (28672 x 4096 50.9 / 62.2 against 38.8).
+// ones, since every workgroup reads all activations (28672 x 4096 50.9 / 62.2 against 38.8). Long K
+// needs slices: a workgroup walks all of its K alone (the lines, measured: ops.sgemm_splits).
 #include "common.h"
 
 namespace lmx {

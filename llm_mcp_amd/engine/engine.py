@@ -128,7 +128,7 @@ class EngineConfig:
     prefix_cache: bool = field(
         default_factory=lambda: _env_int("LMX_PREFIX_CACHE", 1) != 0)
     use_graphs: bool = True
-    part_tokens: int = 512
+    part_tokens: int = 512          # of a partition in decode attention (ops.paged_decode_attention)
     seed: int = 0
     # a KV pool of this many tokens (whole pages) instead of a share of HBM
     kv_cache_tokens: int | None = None

@@ -248,7 +248,10 @@ def paged_decode_attention(q: torch.Tensor, k_cache, v_cache, block_tables, cont
     registers and writes the step's rotated k and v into the cache at
     ``slots`` itself (K2 + K5 fused into K4: ``rope_and_cache`` is skipped for
     these rows; no q/k-norm models).  ``gate`` ([B, Hq*D] rows): the output is
-    multiplied by sigmoid(gate).  ``precise``: softmax weights enter the PV
+    multiplied by sigmoid(gate).  ``part_tokens``: tokens of a partition of the
+    context, at most: 256 are taken where the rows' kv heads fill less than a quarter of
+    the compute units, and more than either where the workspace has too few
+    partitions for the context.  ``precise``: softmax weights enter the PV
     product with fp32 precision (a bf16 pair) instead of one bf16.  ``window``
     (0: all): only that many last positions are seen; ``cap`` (0: none): scores
     become cap tanh(score / cap); both with ``precise``."""
