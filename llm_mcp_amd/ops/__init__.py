@@ -797,31 +797,34 @@ def _into(out: torch.Tensor | None, y: torch.Tensor) -> torch.Tensor:
     return out.copy_(y)
 
 
-def _by_address(*ts) -> bool:
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _by_address(x: torch.Tensor, w: torch.Tensor, *more) -> bool:
     """Kernels may take these tensors by address: plain ones that no gradient, functorch transform
     or tracer follows."""
-    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts):
-        return False
-    return (torch._C._functorch.peek_interpreter_stack() is None
-            and torch._C._len_torch_dispatch_stack() == 0
-            and torch.autograd.forward_ad._current_level < 0
-            and all(t is None or type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts))
+    return not (type(x) not in _PLAIN or type(w) not in _PLAIN
+                or ((x.requires_grad or w.requires_grad or any(t is not None and t.requires_grad for t in more))
+                    and torch.is_grad_enabled())
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch._C._len_torch_dispatch_stack() or torch.autograd.forward_ad._current_level >= 0)
 
 
 def few_rows_ok(x: torch.Tensor, w: torch.Tensor, epi: int = 0, bias: torch.Tensor | None = None,
                 out: torch.Tensor | None = None, step: int = 4) -> bool:
     """Operands that K25 and K23 read and a destination that they write in pieces of ``step``
     elements.  All others keep the route they have without these kernels."""
-    M, N = x.shape[0], w.shape[0]
-    if (N == 0 or w.shape[1] == 0 or x.shape[1] != w.shape[1] or not _by_address(x, w, bias, out)
-            or not pgemm_operands_ok(x, w) or not pgemm_bias_ok(bias, N)
-            or any(t is not None and t.device != x.device for t in (w, bias, out))):
+    N, K = w.shape
+    if (N == 0 or K == 0 or x.shape[1] != K or not _by_address(x, w, bias, out)
+            or not pgemm_operands_ok(x, w) or w.device != x.device):
+        return False
+    if bias is not None and (not pgemm_bias_ok(bias, N) or bias.device != x.device):
         return False
     if out is None:
         return True
-    ncols = N // 2 if epi in (3, 4) else N
-    return (out.dtype == x.dtype and out.shape == (M, ncols) and out.stride(1) == 1
-            and out.stride(0) % step == 0 and (M == 1 or out.stride(0) >= ncols)
+    M, ncols = x.shape[0], N // 2 if epi in (3, 4) else N
+    return (out.dtype == x.dtype and out.device == x.device and out.shape == (M, ncols)
+            and out.stride(1) == 1 and out.stride(0) % step == 0 and (M == 1 or out.stride(0) >= ncols)
             and out.data_ptr() % (2 * step) == 0
             and not any(t is not None and t.untyped_storage().data_ptr() == out.untyped_storage().data_ptr()
                         for t in (x, w, bias)))     # read while it is written
@@ -835,11 +838,27 @@ def few_rows(x: torch.Tensor, w: torch.Tensor, epi: int = 0, bias: torch.Tensor 
         return None
     s = gemv_splits(x, w, epi, out)
     if s is not None and few_rows_ok(x, w, epi, bias, out, 2):
-        return gemv(x, w, epi, s, bias, out)
+        GEMV_CALLS[0] += 1
+        return _few_rows_launch(native().gemv, x, w, epi, s, bias, out)
     s = sgemm_splits(M, N, K, epi)
     if s is not None and few_rows_ok(x, w, epi, bias, out):
-        return sgemm(x, w, epi, s, bias, out)
+        SGEMM_CALLS[0] += 1
+        return _few_rows_launch(native().sgemm, x, w, epi, s, bias, out)
     return None
+
+
+def _few_rows_launch(kernel, a, w, epi, splits, bias, out):
+    """K25 or K23 on checked operands: rows, or ``Partials`` with epi 2."""
+    M, N, K = a.shape[0], w.shape[0], w.shape[1]
+    if epi == 2:
+        p = Partials.empty(a, splits, N)
+        kernel(_ptr(p.slabs), _ptr(a), _ptr(w), M, N, K, a.stride(0), w.stride(0), N, 2, splits, 0, _stream())
+        return p
+    if out is None:
+        out = torch.empty((M, N // 2 if epi in (3, 4) else N), dtype=a.dtype, device=a.device)
+    kernel(_ptr(out), _ptr(a), _ptr(w), M, N, K, a.stride(0), w.stride(0), out.stride(0),
+           epi if bias is None else 5, 1, _ptr(bias), _stream())
+    return out
 
 
 # K23 (csrc/kernels/sgemm.hip), few rows and small weights: where it beats the routes below on
@@ -913,18 +932,9 @@ def gemv(a: torch.Tensor, w: torch.Tensor, epi: int = 0, splits: int = 1,
     _chk(0 < M <= GEMV_MAX_M and N % 32 == 0 and K % GEMV_K == 0 and K // GEMV_K % splits == 0
          and (splits == 1 or epi == 2), f"gemv shape M={M} N={N} K={K} S={splits}")
     _chk(w.shape[1] == K and pgemm_operands_ok(a, w), "gemv operands need 16-B aligned rows")
+    _chk(out is None or (out.shape == (M, N // 2 if epi in (3, 4) else N) and out.stride(1) == 1), "gemv output")
     GEMV_CALLS[0] += 1
-    if epi == 2:
-        p = Partials.empty(a, splits, N)
-        native().gemv(_ptr(p.slabs), _ptr(a), _ptr(w), M, N, K, a.stride(0), w.stride(0), N, 2, splits, 0,
-                      _stream())
-        return p
-    if out is None:
-        out = torch.empty((M, N // 2 if epi in (3, 4) else N), dtype=a.dtype, device=a.device)
-    _chk(out.shape == (M, N // 2 if epi in (3, 4) else N) and out.stride(1) == 1, "gemv output")
-    native().gemv(_ptr(out), _ptr(a), _ptr(w), M, N, K, a.stride(0), w.stride(0), out.stride(0),
-                  5 if bias is not None else epi, 1, _ptr(bias), _stream())
-    return out
+    return _few_rows_launch(native().gemv, a, w, epi, splits, bias, out)
 
 
 def sgemm(a: torch.Tensor, w: torch.Tensor, epi: int = 0, splits: int = 1,
@@ -937,19 +947,10 @@ def sgemm(a: torch.Tensor, w: torch.Tensor, epi: int = 0, splits: int = 1,
     _chk(0 < M <= 64 and N % 32 == 0 and K % 32 == 0 and K // 32 % splits == 0
          and (splits == 1 or epi == 2), f"sgemm shape M={M} N={N} K={K} S={splits}")
     _chk(w.shape[1] == K and pgemm_operands_ok(a, w), "sgemm operands need 16-B aligned rows")
+    _chk(out is None or (out.shape == (M, N // 2 if epi in (3, 4) else N) and out.stride(1) == 1
+                         and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0), "sgemm output layout")
     SGEMM_CALLS[0] += 1
-    if epi == 2:
-        p = Partials.empty(a, splits, N)
-        native().sgemm(_ptr(p.slabs), _ptr(a), _ptr(w), M, N, K, a.stride(0), w.stride(0), N, 2, splits,
-                       0, _stream())
-        return p
-    if out is None:
-        out = torch.empty((M, N // 2 if epi in (3, 4) else N), dtype=a.dtype, device=a.device)
-    _chk(out.shape == (M, N // 2 if epi in (3, 4) else N) and out.stride(1) == 1
-         and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0, "sgemm output layout")
-    native().sgemm(_ptr(out), _ptr(a), _ptr(w), M, N, K, a.stride(0), w.stride(0), out.stride(0),
-                   epi if bias is None else 5, 1, _ptr(bias), _stream())
-    return out
+    return _few_rows_launch(native().sgemm, a, w, epi, splits, bias, out)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, defer: bool = False,
