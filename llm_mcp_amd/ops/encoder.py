@@ -135,7 +135,7 @@ def encode(ids: torch.Tensor, cu: torch.Tensor, lens: list, w: dict, names: tupl
     from . import _chk
     d, I, H, D = cfg.hidden_size, cfg.intermediate_size, cfg.num_heads, cfg.head_dim
     word, pos = w["word"], None if cos_sin is not None else w["pos"]
-    if not (sizes_ok(d, I, H, D, gelu) and word.shape[-1] == d and sum(lens) == ids.numel()
+    if not (sizes_ok(d, I, H, D, gelu) and word.shape[-1] == d and sum(lens) == ids.numel() > 0
             and _index_ok(cu, len(lens) + 1, ids.device)
             and embed_ok(ids, word, w["type"], w["emb_ln_w"], w["emb_ln_b"], pos)):
         return None

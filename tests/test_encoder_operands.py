@@ -92,7 +92,7 @@ def test_embedding_and_indices(gelu, reached):
         w[n] = keep
     ids, cu = torch.zeros(sum(LENS), dtype=torch.int32), torch.tensor([0, 7, 8, 20], dtype=torch.int32)
     for kw in (dict(ids=ids.long()), dict(ids=ids[:-1]), dict(ids=torch.zeros(40, dtype=torch.int32)[::2]),
-               dict(cu=cu.long()), dict(cu=cu[:-1]), dict(lens=[7, 1, 13])):
+               dict(cu=cu.long()), dict(cu=cu[:-1]), dict(lens=[7, 1, 13]), dict(ids=ids[:0], cu=cu[:1], lens=[])):
         assert _encode(names, w, gelu, **kw) is None, kw
 
 
