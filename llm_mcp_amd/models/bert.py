@@ -108,6 +108,8 @@ class BertModel:
             if cfg.pooling == "cls":     # the first tokens' rows as sequences of one
                 x, cu = ops.embed_gather(x, b.first), b.count
             return ops.mean_pool_l2(x, cu, dims or cfg.embed_dim, normalize)
+        if dev.type == "cuda":
+            encoder.weights_on(ids, cu, w)
         pages = np.maximum(1, -(-ln // PAGE))
         page_off = np.concatenate([[0], np.cumsum(pages)])
         NB = int(page_off[-1])

@@ -3,8 +3,8 @@
 ``encode`` is a whole forward up to the pooling: ``batch`` lays the packed sequences out
 (positions, attention tiles), ``embed_norm`` makes their rows, ``layers`` runs all layers.  The
 kernels get addresses and the configuration's sizes, so everything they read is checked
-first (``layers_ok``, ``embed_ok``).  The models keep their own loop over single ops
-for the CPU and for operands and switches this one does not take.
+first (``layers_ok``, ``embed_ok``); operands of several devices are refused.  The models keep
+their own loop over single ops for the CPU and for operands and switches this one does not take.
 """
 from __future__ import annotations
 
@@ -70,10 +70,26 @@ def sizes_ok(d: int, I: int, H: int, D: int, gelu: bool) -> bool:
             and not (gelu and I > PGEMM_MAX_BIAS) and os.environ.get("LMX_ENCODER_LIBRARY", "0") != "1")
 
 
-def layers_ok(layers: list, names: tuple, d: int, I: int, gelu: bool) -> list | None:
+def _one_device(device: int, *tensors) -> None:
+    """All are on the device of this index (-1: host)."""
+    for t in tensors:
+        if t is not None and t.get_device() != device:
+            raise ValueError(f"an encoder operand on {t.device}, its rows on device {device}")
+
+
+def weights_on(ids: torch.Tensor, cu: torch.Tensor, w: dict, cos_sin: torch.Tensor | None = None) -> None:
+    """Everything that a forward reads is on the rows' device.  Before the models' own loop, whose
+    kernels get addresses too."""
+    device = ids.get_device()
+    _one_device(device, cu, cos_sin, *(t for n, t in w.items() if n != "layers"))
+    for L in w["layers"]:
+        _one_device(device, *L.values())
+
+
+def layers_ok(layers: list, names: tuple, d: int, I: int, gelu: bool, device: int = -1) -> list | None:
     """Addresses of the layers' weights, ``names`` of them a layer (None: the model has none
     there), if all are bf16 tensors of the configuration's shapes as they are stored, on 16
-    bytes.  Else None: the models' own loop takes or refuses them."""
+    bytes.  Else None: the models' own loop takes or refuses them.  ``device``: _one_device's."""
     want, bf16, out = list(zip(names, _shapes(d, I, gelu))), torch.bfloat16, []
     for L in layers:
         for n, shape in want:
@@ -83,6 +99,8 @@ def layers_ok(layers: list, names: tuple, d: int, I: int, gelu: bool) -> list | 
             t = L.get(n)
             if t is None or t.dtype is not bf16 or t.shape != shape or not t.is_contiguous():
                 return None
+            if t.get_device() != device:
+                _one_device(device, t)
             out.append(t.data_ptr())
     return None if functools.reduce(operator.or_, out, 0) & 15 else out
 
@@ -113,6 +131,7 @@ def embed_norm(ids: torch.Tensor, word: torch.Tensor, type_row: torch.Tensor, w,
     """LayerNorm(word[ids] + type (+ pos[positions])), bf16 rows.  ``positions`` are the caller's
     to keep below pos's rows."""
     from . import _chk
+    _one_device(ids.get_device(), word, type_row, w, b, pos, positions)
     _chk(embed_ok(ids, word, type_row, w, b, pos, positions)
          and (pos is None or positions is not None), "embed_norm operands")
     return _embed_norm(ids, word, type_row, w, b, eps, pos, positions)
@@ -135,6 +154,8 @@ def encode(ids: torch.Tensor, cu: torch.Tensor, lens: list, w: dict, names: tupl
     from . import _chk
     d, I, H, D = cfg.hidden_size, cfg.intermediate_size, cfg.num_heads, cfg.head_dim
     word, pos = w["word"], None if cos_sin is not None else w["pos"]
+    device = ids.get_device()
+    _one_device(device, cu, word, w["type"], w["emb_ln_w"], w["emb_ln_b"], pos, cos_sin)
     if not (sizes_ok(d, I, H, D, gelu) and word.shape[-1] == d and sum(lens) == ids.numel() > 0
             and _index_ok(cu, len(lens) + 1, ids.device)
             and embed_ok(ids, word, w["type"], w["emb_ln_w"], w["emb_ln_b"], pos)):
@@ -145,7 +166,7 @@ def encode(ids: torch.Tensor, cu: torch.Tensor, lens: list, w: dict, names: tupl
     x = _embed_norm(ids, word, w["type"], w["emb_ln_w"], w["emb_ln_b"], cfg.ln_eps, pos,
                     b.positions if pos is not None else None)
     # here, while the upload and the first norm run (50 us for 12 layers)
-    ptrs = layers_ok(w["layers"], names, d, I, gelu)
+    ptrs = layers_ok(w["layers"], names, d, I, gelu, device)
     return (layers(x, ptrs, b, cu, I, H, D, cfg.ln_eps, scale, gelu, cos_sin), b) if ptrs else None
 
 

@@ -1,11 +1,13 @@
 """Which operands the encoders' native layers take (ops.encoder): the kernels get addresses and the
 configuration's sizes, so all others go to the models' own loop or are refused."""
+import dataclasses
 import types
 
 import pytest
 import torch
 
 from llm_mcp_amd.models import bert, nomic_bert
+from llm_mcp_amd.models import config as mc
 from llm_mcp_amd.ops import encoder
 
 D, I, V, P = 256, 512, 40, 20
@@ -28,13 +30,13 @@ def _ok(names, w, gelu):
     return encoder.layers_ok(w["layers"], names, D, I, gelu)
 
 
-def _encode(names, w, gelu, ids=None, cu=None, lens=LENS, rows=P):
+def _encode(names, w, gelu, ids=None, cu=None, lens=LENS, rows=P, cos_sin=None):
     cfg = types.SimpleNamespace(hidden_size=D, intermediate_size=I, num_heads=D // 64, head_dim=64,
                                 ln_eps=1e-12)
     ids = torch.zeros(sum(LENS), dtype=torch.int32) if ids is None else ids
     cu = torch.tensor([0, 7, 8, 20], dtype=torch.int32) if cu is None else cu
-    return encoder.encode(ids, cu, lens, w, names, cfg, 0.125, gelu,
-                          None if gelu else torch.zeros(rows, 64))
+    cos_sin = torch.zeros(rows, 64) if cos_sin is None else cos_sin
+    return encoder.encode(ids, cu, lens, w, names, cfg, 0.125, gelu, None if gelu else cos_sin)
 
 
 class _Reached(Exception):
@@ -106,6 +108,76 @@ def test_positions_within_their_table(gelu, reached):
     w["pos"] = _zeros(12, D)
     with pytest.raises(_Reached):
         _encode(names, w, gelu, rows=12)
+
+
+class _Elsewhere(torch.Tensor):
+    """A host tensor that says it is on a device."""
+    def get_device(self):
+        return 0
+
+
+@pytest.mark.parametrize("gelu", [True, False])
+def test_operands_of_several_devices(gelu, reached):
+    """Refused, and not left to the models' own loop, whose kernels get addresses too."""
+    names, w = _model(gelu)
+    for n in ["word", "type", "emb_ln_w", "emb_ln_b"] + ["pos"] * gelu:
+        with pytest.raises(ValueError):
+            _encode(names, {**w, n: w[n].as_subclass(_Elsewhere)}, gelu)
+    cu, ids = torch.tensor([0, 7, 8, 20], dtype=torch.int32), torch.zeros(5, dtype=torch.int32)
+    for kw in ([dict(cu=cu.as_subclass(_Elsewhere))]
+               + [dict(cos_sin=torch.zeros(P, 64).as_subclass(_Elsewhere))] * (not gelu)):
+        with pytest.raises(ValueError):
+            _encode(names, w, gelu, **kw)
+    with pytest.raises(ValueError):
+        encoder.embed_norm(ids, w["word"], w["type"].as_subclass(_Elsewhere), w["emb_ln_w"], w["emb_ln_b"], 1e-12)
+    for n in filter(None, names):
+        t = w["layers"][1][n]
+        w["layers"][1][n] = t.as_subclass(_Elsewhere)
+        with pytest.raises(ValueError):
+            _encode(names, w, gelu)
+        w["layers"][1][n] = t
+    with pytest.raises(ValueError):
+        encoder.layers_ok(w["layers"], names, D, I, gelu, 0)       # all of them on the host, the rows not
+
+
+@pytest.mark.parametrize("gelu", [True, False])
+def test_weights_on(gelu):
+    """The check before the models' own loop: every tensor of the model."""
+    names, w = _model(gelu)
+    ids, cu, cos_sin = torch.zeros(20, dtype=torch.int32), torch.tensor([0, 20], dtype=torch.int32), _zeros(P, 64)
+    encoder.weights_on(ids, cu, w, cos_sin)
+    away = lambda t: t.as_subclass(_Elsewhere)
+    for args in ([(ids, away(cu), w, cos_sin), (ids, cu, w, away(cos_sin)), (away(ids), cu, w)]
+                 + [(ids, cu, {**w, n: away(w[n])}) for n in w if n != "layers"]
+                 + [(ids, cu, {**w, "layers": [w["layers"][0], {**w["layers"][1], n: away(t)}]})
+                    for n, t in w["layers"][1].items()]):
+        with pytest.raises(ValueError):
+            encoder.weights_on(*args)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads", [4, 2])
+@pytest.mark.parametrize("model", ["tiny-bert", "tiny-nomic"])
+def test_models_refuse_operands_of_several_devices(model, heads):
+    """A weight left on the host, anywhere in the model: no kernel gets its address, on the native
+    layers (heads of 64) and in the models' own loop."""
+    cfg = dataclasses.replace(mc.resolve(model), num_heads=heads)
+    gelu = cfg.family == "bert"
+    m = (bert.BertModel if gelu else nomic_bert.NomicBertModel)(cfg, "cuda", seed=1)
+    ids, cu = (torch.tensor(a, dtype=torch.int32) for a in (list(range(20)), [0, 7, 8, 20]))
+    run = lambda c, i=ids.cuda(): m.forward(i, c, LENS)
+    names = bert.NATIVE if gelu else nomic_bert.NATIVE
+    for where, n in ([(m.w, n) for n in ("word", "type", "emb_ln_w", "emb_ln_b")] + [(m.w, "pos")] * gelu
+                     + [(m.w["layers"][-1], n) for n in names if n]):
+        keep = where[n]
+        where[n] = keep.cpu()
+        with pytest.raises(ValueError):
+            run(cu.cuda())
+        where[n] = keep
+    for args in ((cu,), (cu.cuda(), ids), (cu, ids)):
+        with pytest.raises(ValueError):
+            run(*args)
+    assert bool(run(cu.cuda()).isfinite().all())
 
 
 def test_embed_norm_refuses():
