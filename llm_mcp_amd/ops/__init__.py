@@ -198,7 +198,8 @@ def rope_and_cache(qkv: torch.Tensor, positions: torch.Tensor, cos_sin: torch.Te
     T = qkv.shape[0]
     _chk(qkv.stride(1) == 1 and qkv.shape[1] >= (Hq + 2 * Hkv) * D, "qkv shape")
     _chk(positions.dtype == torch.int32 and positions.numel() >= T, "positions int32[T]")
-    _chk(cos_sin.dtype == torch.float32 and cos_sin.shape[1] == D, "cos_sin [P, D] fp32")
+    _chk(cos_sin.dtype == torch.float32 and cos_sin.shape[1] == D and cos_sin.is_contiguous(),
+         "cos_sin [P, D] fp32")
     BS = 0
     if k_cache is not None:
         _chk(slots is not None and slots.dtype == torch.int32, "slots int32")

@@ -110,6 +110,11 @@ def _rows_ok(t: torch.Tensor, cols: int, dims: int = 2) -> bool:
             and t.data_ptr() % 16 == 0)
 
 
+def _rotary_ok(t: torch.Tensor, D: int) -> bool:
+    return (t.dtype is torch.float32 and t.dim() == 2 and t.shape[1] == D and t.is_contiguous()
+            and t.data_ptr() % 16 == 0)
+
+
 def _index_ok(t: torch.Tensor, n: int, device: torch.device) -> bool:
     return (t.dtype is torch.int32 and t.dim() == 1 and t.numel() == n and t.is_contiguous()
             and t.device == device)
@@ -158,7 +163,8 @@ def encode(ids: torch.Tensor, cu: torch.Tensor, lens: list, w: dict, names: tupl
     _one_device(device, cu, word, w["type"], w["emb_ln_w"], w["emb_ln_b"], pos, cos_sin)
     if not (sizes_ok(d, I, H, D, gelu) and word.shape[-1] == d and sum(lens) == ids.numel() > 0
             and _index_ok(cu, len(lens) + 1, ids.device)
-            and embed_ok(ids, word, w["type"], w["emb_ln_w"], w["emb_ln_b"], pos)):
+            and embed_ok(ids, word, w["type"], w["emb_ln_w"], w["emb_ln_b"], pos)
+            and (cos_sin is None or _rotary_ok(cos_sin, D))):
         return None
     b = batch(lens, ids.device)
     _chk(b.longest <= (pos if cos_sin is None else cos_sin).shape[0],
@@ -196,8 +202,7 @@ def attention(qkv: torch.Tensor, cu: torch.Tensor, b: Batch, H: int, scale: floa
     from . import _chk, _ptr, _stream, native
     T, D = qkv.shape[0], qkv.shape[1] // (3 * H)
     _chk(qkv.dtype is torch.bfloat16 and qkv.stride(1) == 1, "qkv rows")
-    _chk(cos_sin is None or (cos_sin.dtype is torch.float32 and cos_sin.is_contiguous()
-                             and cos_sin.shape[0] >= b.longest), "cos_sin")
+    _chk(cos_sin is None or (_rotary_ok(cos_sin, D) and cos_sin.shape[0] >= b.longest), "cos_sin")
     out = torch.empty((T, H * D), dtype=qkv.dtype, device=qkv.device)
     native().enc_attention(_ptr(qkv), qkv.stride(0), H, D, _ptr(cu), _ptr(b.tiles), b.tiles.numel() // 2,
                            _ptr(cos_sin), _ptr(out), H * D, float(scale), float(rescale_thr), _stream())

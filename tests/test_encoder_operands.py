@@ -110,6 +110,19 @@ def test_positions_within_their_table(gelu, reached):
         _encode(names, w, gelu, rows=12)
 
 
+def test_rotary_table(reached):
+    """fp32 rows of a head on 16 bytes: others go to the models' own loop, which takes an address
+    off 16 bytes and whose rotation refuses the rest."""
+    names, w = _model(False)
+    t = torch.zeros(P, 64)
+    off = torch.zeros(P * 64 + 4)
+    off = off[-off.data_ptr() // 4 % 4 + 1:][:P * 64].view(P, 64)
+    for bad in (t.bfloat16(), t[:, :32].contiguous(), torch.zeros(P, 128)[:, :64], t.flatten(), off):
+        assert _encode(names, w, False, cos_sin=bad) is None
+    with pytest.raises(_Reached):
+        _encode(names, w, False, cos_sin=t)
+
+
 class _Elsewhere(torch.Tensor):
     """A host tensor that says it is on a device."""
     def get_device(self):
@@ -178,6 +191,19 @@ def test_models_refuse_operands_of_several_devices(model, heads):
         with pytest.raises(ValueError):
             run(*args)
     assert bool(run(cu.cuda()).isfinite().all())
+
+
+@pytest.mark.gpu
+def test_models_refuse_other_rotary_tables():
+    for heads in (4, 2):
+        cfg = dataclasses.replace(mc.resolve("tiny-nomic"), num_heads=heads)
+        m = nomic_bert.NomicBertModel(cfg, "cuda", seed=1)
+        ids, cu = (torch.tensor(a, dtype=torch.int32).cuda() for a in (list(range(20)), [0, 7, 8, 20]))
+        t = m.cos_sin
+        for bad in (t.bfloat16(), t[:, :32].contiguous(), torch.cat([t, t], 1)[:, :t.shape[1]]):
+            m.cos_sin = bad
+            with pytest.raises(ValueError):
+                m.forward(ids, cu, LENS)
 
 
 def test_embed_norm_refuses():
