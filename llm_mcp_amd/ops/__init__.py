@@ -154,12 +154,24 @@ def rms_norm(x, w: torch.Tensor, eps: float,
     return out
 
 
+def layer_norm_ok(x, w, b, residual=None) -> bool:
+    """What the kernel reads by address: contiguous bf16 rows and vectors of their width, on one
+    device; a residual may be a longer buffer of such rows."""
+    vec = lambda t: (t.dtype == x.dtype and t.numel() == x.shape[1] and t.is_contiguous()
+                     and t.get_device() == x.get_device())
+    return (x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous() and x.shape[1] % 8 == 0
+            and vec(w) and vec(b)
+            and (residual is None or (residual.dtype == x.dtype and residual.is_contiguous()
+                                      and residual.shape[-1:] == x.shape[-1:]
+                                      and residual.numel() >= x.numel()
+                                      and residual.get_device() == x.get_device())))
+
+
 def layer_norm(x, w, b, eps, residual=None):
     if not x.is_cuda:
         return ref.layer_norm(x, w, b, eps, residual)
-    _bf16(x, "x")
+    _chk(layer_norm_ok(x, w, b, residual), "layer_norm operands")
     rows, cols = x.shape
-    _chk(x.is_contiguous() and cols % 8 == 0, "layer_norm shape")
     out = torch.empty_like(x)
     native().layernorm(_ptr(out), _ptr(x), _ptr(residual), _ptr(w), _ptr(b), rows, cols,
                        float(eps), _stream())

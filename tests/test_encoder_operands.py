@@ -6,6 +6,7 @@ import types
 import pytest
 import torch
 
+from llm_mcp_amd import ops
 from llm_mcp_amd.models import bert, nomic_bert
 from llm_mcp_amd.models import config as mc
 from llm_mcp_amd.ops import encoder
@@ -191,6 +192,34 @@ def test_models_refuse_operands_of_several_devices(model, heads):
         with pytest.raises(ValueError):
             run(*args)
     assert bool(run(cu.cuda()).isfinite().all())
+
+
+def test_layer_norm_operands():
+    """What the models' own loop passes to its LayerNorm by address."""
+    x, v, r = _zeros(5, D), _zeros(D), _zeros(7, D)
+    assert ops.layer_norm_ok(x, v, v) and ops.layer_norm_ok(x, v[None], v, r) and ops.layer_norm_ok(x, v, v, r[:5])
+    for args in ((x.float(), v, v), (x, v.float(), v), (x, v, v.float()), (x, v[:-8], v), (x, v, _zeros(D + 8)),
+                 (x, _zeros(2 * D)[::2], v), (x, v, v, x.float()), (x, v, v, x[:4]), (x, v, v, _zeros(D, 5).t()),
+                 (x, v, v, _zeros(5, 2 * D)[:, :D]), (x, v, v, _zeros(10, D // 2)), (_zeros(D, 5).t(), v, v),
+                 (x, v.as_subclass(_Elsewhere), v), (x, v, v.as_subclass(_Elsewhere)),
+                 (x, v, v, r.as_subclass(_Elsewhere))):
+        assert not ops.layer_norm_ok(*args)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads", [4, 2])
+@pytest.mark.parametrize("model", ["tiny-bert", "tiny-nomic"])
+def test_models_refuse_other_norm_weights(model, heads):
+    cfg = dataclasses.replace(mc.resolve(model), num_heads=heads)
+    m = (bert.BertModel if cfg.family == "bert" else nomic_bert.NomicBertModel)(cfg, "cuda", seed=1)
+    ids, cu = (torch.tensor(a, dtype=torch.int32).cuda() for a in (list(range(20)), [0, 7, 8, 20]))
+    for where, n in ((m.w, "emb_ln_w"), (m.w["layers"][0], "ln1_b"), (m.w["layers"][-1], "ln2_w")):
+        keep = where[n]
+        for bad in (keep.float(), keep[:-8].clone()):
+            where[n] = bad
+            with pytest.raises(ValueError):
+                m.forward(ids, cu, LENS)
+        where[n] = keep
 
 
 @pytest.mark.gpu
