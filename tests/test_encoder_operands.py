@@ -175,7 +175,7 @@ def test_weights_on(gelu):
 def test_models_refuse_operands_of_several_devices(model, heads):
     """A weight left on the host, anywhere in the model: no kernel gets its address, on the native
     layers (heads of 64) and in the models' own loop."""
-    cfg = dataclasses.replace(mc.resolve(model), num_heads=heads)
+    cfg = dataclasses.replace(mc.resolve(model), num_heads=heads, head_dim=D // heads)
     gelu = cfg.family == "bert"
     m = (bert.BertModel if gelu else nomic_bert.NomicBertModel)(cfg, "cuda", seed=1)
     ids, cu = (torch.tensor(a, dtype=torch.int32) for a in (list(range(20)), [0, 7, 8, 20]))
@@ -210,7 +210,7 @@ def test_layer_norm_operands():
 @pytest.mark.parametrize("heads", [4, 2])
 @pytest.mark.parametrize("model", ["tiny-bert", "tiny-nomic"])
 def test_models_refuse_other_norm_weights(model, heads):
-    cfg = dataclasses.replace(mc.resolve(model), num_heads=heads)
+    cfg = dataclasses.replace(mc.resolve(model), num_heads=heads, head_dim=D // heads)
     m = (bert.BertModel if cfg.family == "bert" else nomic_bert.NomicBertModel)(cfg, "cuda", seed=1)
     ids, cu = (torch.tensor(a, dtype=torch.int32).cuda() for a in (list(range(20)), [0, 7, 8, 20]))
     for where, n in ((m.w, "emb_ln_w"), (m.w["layers"][0], "ln1_b"), (m.w["layers"][-1], "ln2_w")):
@@ -225,7 +225,7 @@ def test_models_refuse_other_norm_weights(model, heads):
 @pytest.mark.gpu
 def test_models_refuse_other_rotary_tables():
     for heads in (4, 2):
-        cfg = dataclasses.replace(mc.resolve("tiny-nomic"), num_heads=heads)
+        cfg = dataclasses.replace(mc.resolve("tiny-nomic"), num_heads=heads, head_dim=D // heads)
         m = nomic_bert.NomicBertModel(cfg, "cuda", seed=1)
         ids, cu = (torch.tensor(a, dtype=torch.int32).cuda() for a in (list(range(20)), [0, 7, 8, 20]))
         t = m.cos_sin
