@@ -110,6 +110,7 @@ class BertModel:
             return ops.mean_pool_l2(x, cu, dims or cfg.embed_dim, normalize)
         if dev.type == "cuda":
             encoder.weights_on(ids, cu, w)
+        ids, cu = ids.contiguous(), cu.contiguous()
         pages = np.maximum(1, -(-ln // PAGE))
         page_off = np.concatenate([[0], np.cumsum(pages)])
         NB = int(page_off[-1])

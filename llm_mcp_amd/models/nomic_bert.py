@@ -117,6 +117,7 @@ class NomicBertModel:
             return ops.mean_pool_l2(x, cu, dims or cfg.embed_dim, normalize)
         if dev.type == "cuda":
             encoder.weights_on(ids, cu, w, self.cos_sin)
+        ids, cu = ids.contiguous(), cu.contiguous()
         # per-sequence page-aligned slots in a scratch paged K/V cache, built
         # with array ops (no per-token Python work on the host critical path)
         ln = np.asarray(lens, dtype=np.int64)

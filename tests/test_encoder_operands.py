@@ -223,6 +223,24 @@ def test_models_refuse_other_norm_weights(model, heads):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads", [4, 2])
+@pytest.mark.parametrize("model", ["tiny-bert", "tiny-nomic"])
+def test_strided_indices(model, heads):
+    """Every second element of an index array: the vectors of the loop on a contiguous copy."""
+    cfg = dataclasses.replace(mc.resolve(model), num_heads=heads, head_dim=D // heads)
+    m = (bert.BertModel if cfg.family == "bert" else nomic_bert.NomicBertModel)(cfg, "cuda", seed=1)
+    ids, cu = (torch.tensor(a, dtype=torch.int32).cuda() for a in (list(range(20)), [0, 7, 8, 20]))
+    every2 = lambda t: torch.stack([t, t.flip(0)], 1).flatten()[::2]
+    y = m.forward(every2(ids), every2(cu), LENS)       # the loop, with heads of 64 too
+    assert torch.equal(y, m.forward(every2(ids), cu, LENS)) and torch.equal(y, m.forward(ids, every2(cu), LENS))
+    if heads == 2:
+        assert torch.equal(y, m.forward(ids, cu, LENS))
+    else:
+        # other kernels: 2^-8 of a row's length at each of some twenty roundings, at random, on both sides
+        assert float((y - m.forward(ids, cu, LENS)).norm(dim=1).max()) < 20 ** 0.5 * 2 ** 0.5 * 2.0 ** -8
+
+
+@pytest.mark.gpu
 def test_models_refuse_other_rotary_tables():
     for heads in (4, 2):
         cfg = dataclasses.replace(mc.resolve("tiny-nomic"), num_heads=heads, head_dim=D // heads)
