@@ -810,8 +810,8 @@ __global__ void __launch_bounds__(PG_THREADS, 1) pgemm_pp2_kernel(
 // At decode batch sizes (M <= 256) one 256-row tile covers the batch, and every
 // column tile re-reads the whole 256 x K activation panel from L2: at the
 // 128-column tiles of K11 / hipBLASLt each CU moves 2 bytes of activations
-// through its vector L1 per byte of weights, and the L1's outstanding-miss
-// capacity bounds those kernels (profiles/r3_decode_gemm_study.md).  A
+// through its vector L1 per byte of weights, and what a CU takes in is the L1's
+// outstanding misses over their latency (profiles/rows_128_256.md).  A
 // 256-column tile halves that ratio; split-K over S slices gives the N / 256
 // tiles enough workgroups to fill the CUs (Llama-3-8B gate/up: 112 tiles x 2).
 // One workgroup per (slice, tile), slice-major (the workgroups of one XCD read

@@ -1,5 +1,5 @@
 """Can decode attention (HBM-bound) run under the decode GEMMs (bound by the
-per-CU vector-L1 fill rate)?  Times, at a half batch (--rows, default 128):
+vector L1's misses in flight and their latency)?  Times, at a half batch (--rows, default 128):
 
   * K14 gate/up + SwiGLU (Llama-3-8B 28672 x 4096, packed, cold: copies rotate)
   * paged decode attention (32 q / 8 kv heads, contexts 535-791, random pages)
