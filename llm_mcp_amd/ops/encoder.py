@@ -55,6 +55,7 @@ def batch(lens, device) -> Batch:
     return Batch(*(dev[a:a + n] for a, n in zip(at, sizes)), int(ln.max(initial=0)))
 
 
+@functools.lru_cache(maxsize=64)
 def _shapes(d: int, I: int, gelu: bool) -> tuple:
     """Shapes of a layer's tensors in the order of encoder.h."""
     v, w1 = (d,), I if gelu else 2 * I
@@ -115,20 +116,19 @@ def _rotary_ok(t: torch.Tensor, D: int) -> bool:
             and t.data_ptr() % 16 == 0)
 
 
-def _index_ok(t: torch.Tensor, n: int, device: torch.device) -> bool:
-    return (t.dtype is torch.int32 and t.dim() == 1 and t.numel() == n and t.is_contiguous()
-            and t.device == device)
+def _index_ok(t: torch.Tensor, n: int) -> bool:
+    return t.dtype is torch.int32 and t.dim() == 1 and t.numel() == n and t.is_contiguous()
 
 
 def embed_ok(ids: torch.Tensor, word: torch.Tensor, type_row: torch.Tensor, w, b,
              pos: torch.Tensor | None = None, positions: torch.Tensor | None = None) -> bool:
-    """Whether ``embed_norm`` reads these: int32 indices, contiguous bf16 tables and vectors of
-    one width on 16 bytes."""
+    """Whether ``embed_norm`` reads these, all on one device (``_one_device``): int32 indices,
+    contiguous bf16 tables and vectors of one width on 16 bytes."""
     d = word.shape[-1]
-    return (_index_ok(ids, ids.numel(), word.device) and _rows_ok(word, d) and d % 8 == 0 and d <= 2048
+    return (_index_ok(ids, ids.numel()) and _rows_ok(word, d) and d % 8 == 0 and d <= 2048
             and _rows_ok(type_row, d) and type_row.shape[0] > 0 and _rows_ok(w, d, 1) and _rows_ok(b, d, 1)
             and (pos is None or _rows_ok(pos, d))
-            and (positions is None or _index_ok(positions, ids.numel(), word.device)))
+            and (positions is None or _index_ok(positions, ids.numel())))
 
 
 def embed_norm(ids: torch.Tensor, word: torch.Tensor, type_row: torch.Tensor, w, b, eps: float,
@@ -162,7 +162,7 @@ def encode(ids: torch.Tensor, cu: torch.Tensor, lens: list, w: dict, names: tupl
     device = ids.get_device()
     _one_device(device, cu, word, w["type"], w["emb_ln_w"], w["emb_ln_b"], pos, cos_sin)
     if not (sizes_ok(d, I, H, D, gelu) and word.shape[-1] == d and sum(lens) == ids.numel() > 0
-            and _index_ok(cu, len(lens) + 1, ids.device)
+            and _index_ok(cu, len(lens) + 1)
             and embed_ok(ids, word, w["type"], w["emb_ln_w"], w["emb_ln_b"], pos)
             and (cos_sin is None or _rotary_ok(cos_sin, D))):
         return None
