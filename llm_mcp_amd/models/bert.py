@@ -109,7 +109,7 @@ class BertModel:
                 x, cu = ops.embed_gather(x, b.first), b.count
             return ops.mean_pool_l2(x, cu, dims or cfg.embed_dim, normalize)
         if dev.type == "cuda":
-            encoder.weights_on(ids, cu, w)
+            encoder.weights_on(ids, cu, w, NATIVE)
         ids, cu = ids.contiguous(), cu.contiguous()
         pages = np.maximum(1, -(-ln // PAGE))
         page_off = np.concatenate([[0], np.cumsum(pages)])

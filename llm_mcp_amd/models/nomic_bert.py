@@ -116,7 +116,9 @@ class NomicBertModel:
             x, _ = r
             return ops.mean_pool_l2(x, cu, dims or cfg.embed_dim, normalize)
         if dev.type == "cuda":
-            encoder.weights_on(ids, cu, w, self.cos_sin)
+            # w_gate_up is read where no interleaved copy was made of it
+            names = NATIVE if all("w_gu_il" in L for L in w["layers"]) else NATIVE + ("w_gate_up",)
+            encoder.weights_on(ids, cu, w, names, self.cos_sin)
         ids, cu = ids.contiguous(), cu.contiguous()
         # per-sequence page-aligned slots in a scratch paged K/V cache, built
         # with array ops (no per-token Python work on the host critical path)

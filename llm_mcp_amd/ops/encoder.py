@@ -78,13 +78,15 @@ def _one_device(device: int, *tensors) -> None:
             raise ValueError(f"an encoder operand on {t.device}, its rows on device {device}")
 
 
-def weights_on(ids: torch.Tensor, cu: torch.Tensor, w: dict, cos_sin: torch.Tensor | None = None) -> None:
-    """Everything that a forward reads is on the rows' device.  Before the models' own loop, whose
-    kernels get addresses too."""
+def weights_on(ids: torch.Tensor, cu: torch.Tensor, w: dict, names: tuple,
+               cos_sin: torch.Tensor | None = None) -> None:
+    """Everything that a forward reads (``names`` of a layer) is on the rows' device.  Before the
+    models' own loop, whose kernels get addresses too."""
     device = ids.get_device()
-    _one_device(device, cu, cos_sin, *(t for n, t in w.items() if n != "layers"))
+    _one_device(device, cu, cos_sin, *(w.get(n) for n in ("word", "type", "emb_ln_w", "emb_ln_b")),
+                w.get("pos") if cos_sin is None else None)
     for L in w["layers"]:
-        _one_device(device, *L.values())
+        _one_device(device, *(L.get(n) for n in names))
 
 
 def layers_ok(layers: list, names: tuple, d: int, I: int, gelu: bool, device: int = -1) -> list | None:

@@ -156,15 +156,16 @@ def test_operands_of_several_devices(gelu, reached):
 
 @pytest.mark.parametrize("gelu", [True, False])
 def test_weights_on(gelu):
-    """The check before the models' own loop: every tensor of the model."""
+    """The check before the models' own loop: every tensor that it reads, and no other."""
     names, w = _model(gelu)
     ids, cu, cos_sin = torch.zeros(20, dtype=torch.int32), torch.tensor([0, 20], dtype=torch.int32), _zeros(P, 64)
-    encoder.weights_on(ids, cu, w, cos_sin)
+    encoder.weights_on(ids, cu, w, names)
     away = lambda t: t.as_subclass(_Elsewhere)
-    for args in ([(ids, away(cu), w, cos_sin), (ids, cu, w, away(cos_sin)), (away(ids), cu, w)]
-                 + [(ids, cu, {**w, n: away(w[n])}) for n in w if n != "layers"]
-                 + [(ids, cu, {**w, "layers": [w["layers"][0], {**w["layers"][1], n: away(t)}]})
-                    for n, t in w["layers"][1].items()]):
+    layer = lambda n, t: {**w, "layers": [w["layers"][0], {**w["layers"][1], n: t}]}
+    encoder.weights_on(ids, cu, {**layer("other", away(cu)), "pos": away(cu), "note": "text"}, names, cos_sin)
+    for args in ([(ids, away(cu), w, names, cos_sin), (ids, cu, w, names, away(cos_sin)), (away(ids), cu, w, names)]
+                 + [(ids, cu, {**w, n: away(w[n])}, names) for n in w if n != "layers"]
+                 + [(ids, cu, layer(n, away(t)), names) for n, t in w["layers"][1].items()]):
         with pytest.raises(ValueError):
             encoder.weights_on(*args)
 
